@@ -285,6 +285,25 @@ int32_t tp_append_stage(const void* k, const void* v, int32_t in_dtype, int64_t 
                         int64_t copy_begin, int64_t n_copy, void* tail_k, void* tail_v, int64_t tail_tokens,
                         int64_t tail_pos, int32_t check, uint32_t* flag, uint32_t epoch, void* stream);
 
+/* One buffer of tp_grow_rows: rows of src_row bytes (src; NULL when keep is 0)
+ * move into rows of dst_row bytes (dst). */
+typedef struct tp_grow {
+  const void* src;
+  void* dst;
+  int64_t src_row;
+  int64_t dst_row;
+  int64_t keep;       /* bytes of each row copied from src, 0 <= keep <= src_row */
+  int64_t clear_from; /* bytes [clear_from, dst_row) of each row are zeroed, keep <= clear_from */
+} tp_grow;
+
+/* Growth of a page store (replaces the fill and the copy per buffer of
+ * PolarKBlockStorage._grow / QuantVBlockStorage._grow, storage.py:57-73,
+ * 138-147): for each of the n_bufs (1..8) buffers and each of `rows` (batch,
+ * head) rows, bytes [0, keep) are copied, [keep, clear_from) left as they are
+ * and [clear_from, dst_row) zeroed.  One launch; a kernel, not a memset node.
+ * src and dst must not overlap. */
+int32_t tp_grow_rows(const tp_grow* bufs, int32_t n_bufs, int64_t rows, void* stream);
+
 /* ---- QJL (rejected by TurboPolarConfig, turbo_polar_config.py:46-47, as in
  * the reference; these serve the bridge-level QJL calls the reference's own
  * tests make). ---- */

@@ -63,6 +63,19 @@ class TPQjl(ctypes.Structure):
     ]
 
 
+class TPGrow(ctypes.Structure):
+    """tp_grow: one buffer of tp_grow_rows."""
+
+    _fields_ = [
+        ("src", c_vp),
+        ("dst", c_vp),
+        ("src_row", c_i64),
+        ("dst_row", c_i64),
+        ("keep", c_i64),
+        ("clear_from", c_i64),
+    ]
+
+
 class TPBoundsCase(ctypes.Structure):
     """tp_bounds_case: one launch shape for tp_selftest_decode_bounds."""
 
@@ -128,6 +141,7 @@ _SIGNATURES = {
         c_i32,
         [c_vp, c_vp, c_i32, c_i64, c_i64, c_i64, c_i64, c_vp, c_vp, c_i64, c_i64, c_i32, c_vp, ctypes.c_uint32, c_vp],
     ),
+    "tp_grow_rows": (c_i32, [ctypes.POINTER(TPGrow), c_i32, c_i64, c_vp]),
     "tp_fused_qk_qjl": (c_i32, [c_vp, c_i64, c_i32, c_i32, _P_LAYOUT, _P_PAGES, c_i32, _P_QJL, c_float, c_vp, c_vp]),
     "tp_decode_attention_qjl": (
         c_i32,

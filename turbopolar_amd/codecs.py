@@ -48,18 +48,21 @@ class PolarQuantEncoder:
             packed_row_bytes(self.head_dim // 2 - split_half, self.k_angle_bits_deep),
         )
 
-    def alloc_pages(self, B: int, H: int, n_pages: int, device) -> dict:
-        """Zeroed page buffers ``[B, H, n_pages, 64, .]`` for this layout."""
+    def page_shapes(self, B: int, H: int) -> dict:
+        """((B, H), page shape, dtype) of each page buffer of this layout (None: it has none)."""
         l1_row, deep_row = self.row_bytes()
         rdt = torch.int8 if self.use_int8_radii else torch.float16
         return {
-            "radii": torch.zeros((B, H, n_pages, PAGE, self.head_dim // 2), dtype=rdt, device=device),
-            "angle_codes_l1": torch.zeros((B, H, n_pages, PAGE, l1_row), dtype=torch.uint8, device=device),
-            "angle_codes_deep": torch.zeros((B, H, n_pages, PAGE, deep_row), dtype=torch.uint8, device=device),
-            "radii_scales": (
-                torch.zeros((B, H, n_pages, 1, 1), dtype=torch.float16, device=device) if self.use_int8_radii else None
-            ),
+            "radii": ((B, H), (PAGE, self.head_dim // 2), rdt),
+            "angle_codes_l1": ((B, H), (PAGE, l1_row), torch.uint8),
+            "angle_codes_deep": ((B, H), (PAGE, deep_row), torch.uint8),
+            "radii_scales": ((B, H), (1, 1), torch.float16) if self.use_int8_radii else None,
         }
+
+    def alloc_pages(self, B: int, H: int, n_pages: int, device) -> dict:
+        """Zeroed page buffers ``[B, H, n_pages, 64, .]`` for this layout."""
+        return {name: None if spec is None else torch.zeros(spec[0] + (n_pages,) + spec[1], dtype=spec[2], device=device)
+                for name, spec in self.page_shapes(B, H).items()}
 
     def encode_block(self, k_block: torch.Tensor) -> PolarKeyBlock:
         """Encode ``[B, H, L, D]`` keys into a single (4-D) block."""

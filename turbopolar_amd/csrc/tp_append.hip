@@ -79,11 +79,83 @@ __global__ __launch_bounds__(256) void append_stage_kernel(AppendArgs a) {
   }
 }
 
+// ---- growth of a page store -------------------------------------------------------
+//
+// Bound by launches, not by bytes: a store of 512 pages x 8 heads was filled and
+// copied buffer by buffer in 12 torch launches, most of them 2-4 us of kernel
+// behind 10-20 us of host; here every buffer's kept and cleared bytes go out
+// in one.  blockIdx.z is the buffer, y the (batch, head) row, x strides over the
+// row's chunks; a buffer whose pointers, rows and bounds are all multiples of 16
+// bytes moves 16 bytes a thread, any other (the fp16 page scales) 2, or 1.
+constexpr int kGrowMax = 8;
+struct GrowArgs {
+  tp_grow b[kGrowMax];
+  int64_t rows;
+};
+
+template <class T>
+__device__ __forceinline__ void grow_row(const tp_grow& g, int64_t row) {
+  const int64_t keep = g.keep / (int64_t)sizeof(T);
+  const int64_t clear = g.clear_from / (int64_t)sizeof(T);
+  const int64_t total = keep + g.dst_row / (int64_t)sizeof(T) - clear;
+  const T* src = reinterpret_cast<const T*>(static_cast<const char*>(g.src) + row * g.src_row);
+  T* dst = reinterpret_cast<T*>(static_cast<char*>(g.dst) + row * g.dst_row);
+  for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < total; i += (int64_t)gridDim.x * 256) {
+    if (i < keep)
+      dst[i] = src[i];
+    else
+      dst[clear + i - keep] = T{};
+  }
+}
+
+__global__ __launch_bounds__(256) void grow_rows_kernel(GrowArgs a) {
+  const tp_grow& g = a.b[blockIdx.z];
+  const uint64_t u = (uint64_t)(uintptr_t)g.src | (uint64_t)(uintptr_t)g.dst | (uint64_t)g.src_row |
+                     (uint64_t)g.dst_row | (uint64_t)g.keep | (uint64_t)g.clear_from;
+  for (int64_t row = blockIdx.y; row < a.rows; row += gridDim.y) {
+    if ((u & 15u) == 0)
+      grow_row<uint4>(g, row);
+    else if ((u & 1u) == 0)
+      grow_row<uint16_t>(g, row);
+    else
+      grow_row<uint8_t>(g, row);
+  }
+}
+
 }  // namespace tp
 
 using namespace tp;
 
 extern "C" {
+
+int32_t tp_grow_rows(const tp_grow* bufs, int32_t n_bufs, int64_t rows, void* stream) {
+  clear_error();
+  if (!bufs || n_bufs < 1 || n_bufs > kGrowMax || rows < 1) {
+    set_error("tp_grow_rows takes 1 to %d buffers and at least one row, got %d and %lld", kGrowMax, n_bufs,
+              (long long)rows);
+    return TP_ERR_INVALID;
+  }
+  GrowArgs a{};
+  a.rows = rows;
+  int64_t most = 0;
+  for (int i = 0; i < n_bufs; ++i) {
+    const tp_grow& g = bufs[i];
+    if (!g.dst || g.keep < 0 || g.keep > g.src_row || g.keep > g.clear_from || g.clear_from > g.dst_row ||
+        (g.keep > 0 && !g.src)) {
+      set_error("tp_grow_rows: buffer %d keeps %lld of %lld bytes and clears from %lld of %lld", i, (long long)g.keep,
+                (long long)g.src_row, (long long)g.clear_from, (long long)g.dst_row);
+      return TP_ERR_INVALID;
+    }
+    a.b[i] = g;
+    most = std::max(most, g.keep + g.dst_row - g.clear_from);
+  }
+  if (most == 0) return TP_OK;
+  // Four chunks of 16 bytes a thread, at most 64 workgroups a row.
+  const unsigned x = (unsigned)std::min<int64_t>((most + 16383) / 16384, 64);
+  const dim3 grid(x, (unsigned)std::min<int64_t>(rows, 65535), (unsigned)n_bufs);
+  hipLaunchKernelGGL(grow_rows_kernel, grid, dim3(256), 0, static_cast<hipStream_t>(stream), a);
+  return launch_status("tp_grow_rows");
+}
 
 int32_t tp_append_stage(const void* k, const void* v, int32_t in_dtype, int64_t bh, int64_t in_tokens,
                         int64_t copy_begin, int64_t n_copy, void* tail_k, void* tail_v, int64_t tail_tokens,

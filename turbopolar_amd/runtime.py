@@ -27,7 +27,7 @@ from .codecs import GroupedVQuantizer, PolarQuantDecoder, PolarQuantEncoder
 from .config import TurboPolarConfig
 from .kernels import PAGE, decode_pages_gather, encode_pages
 from .payload import PolarKeyBlock, QuantizedVBlock
-from .storage import PolarKBlockStorage, QuantVBlockStorage, pages_of
+from .storage import Growth, PolarKBlockStorage, QuantVBlockStorage, pages_of
 
 
 def _nbytes(x: torch.Tensor) -> int:
@@ -165,11 +165,24 @@ class TurboPolarKVCacheRuntime:
         v = B * H * PAGE * self._head_dim + B * H * PAGE * (self._head_dim // 32) * 2
         return k + v
 
-    def _encode_into_storage(self, k: torch.Tensor, v: torch.Tensor, token_begin: int, n_pages: int) -> None:
+    def _reserve(self, needed: int, fresh: int, device) -> None:
+        """Room for ``needed`` pages in both storages, the last ``fresh`` of
+        which the caller encodes next."""
         B, H = self._batch_size, self._num_kv_heads
+        ks, vs = self.k_storage, self.v_storage
+        if needed <= ks.capacity and needed <= vs.capacity:
+            return
+        if ks.radii is None:
+            ks.metadata = self.polar_encoder.metadata
+        growth = Growth(fresh)
+        ks.plan(growth, needed, self.polar_encoder, B, H, device)
+        vs.plan(growth, needed, B, H, device)
+        growth.fill()
+        growth.commit()
+
+    def _encode_into_storage(self, k: torch.Tensor, v: torch.Tensor, token_begin: int, n_pages: int) -> None:
         start = self.k_storage.block_count
-        self.k_storage.reserve(start + n_pages, self.polar_encoder, B, H, k.device)
-        self.v_storage.reserve(start + n_pages, B, H, k.device)
+        self._reserve(start + n_pages, n_pages, k.device)
         encode_pages(
             k, v, token_begin, n_pages * PAGE, self.polar_encoder.layout,
             pages_of(self.k_storage, self.v_storage), start,
