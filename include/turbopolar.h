@@ -266,7 +266,7 @@ int32_t tp_decode_pages_gather(const tp_page_layout* layout, const tp_pages* pag
  * k, v: [bh][in_tokens][128] of in_dtype (0 fp16, 1 fp32), 16-byte aligned.
  * Copies tokens [copy_begin, copy_begin + n_copy) of every (b, h) row into
  * tail_k / tail_v ([bh][tail_tokens][128], same dtype) at token tail_pos.
- * With check != 0 it also scans every element of k and v; the kernel stores
+ * Without a check it reads those tokens alone.  With check != 0 it also scans every element of k and v; the kernel stores
  * `epoch` into *flag if any is NaN or inf, and this call then synchronises
  * `stream`, reads the flag and returns TP_ERR_NONFINITE, or TP_OK.  check == 1:
  * flag is caller-owned device memory, read back with a 4-byte copy.  check == 2:
@@ -284,6 +284,23 @@ int32_t tp_decode_pages_gather(const tp_page_layout* layout, const tp_pages* pag
 int32_t tp_append_stage(const void* k, const void* v, int32_t in_dtype, int64_t bh, int64_t in_tokens,
                         int64_t copy_begin, int64_t n_copy, void* tail_k, void* tail_v, int64_t tail_tokens,
                         int64_t tail_pos, int32_t check, uint32_t* flag, uint32_t epoch, void* stream);
+
+/* An append of at least one whole page in one launch: the non-finite check, the
+ * page encode and the copies to the dense tail of
+ * TurboPolarKVCacheRuntime.append (turbo_polar_cache.py:69,106-161), which read
+ * the input once.  k, v: [bh][in_tokens][128] as for tp_encode_pages.  Tokens
+ * [0, n_head) (n_head < 64) go to tail rows tail_pos .. of the tail buffers
+ * ([bh][tail_tokens][128], same dtype); the whole pages after them are encoded
+ * into page slots page_begin ..; the tokens past the last whole page go to tail
+ * row 0 .. if copy_rem is set (n_head must then be 0), and are only checked
+ * otherwise.  Every value is checked: the call synchronises `stream` and
+ * returns TP_ERR_NONFINITE if one is NaN or inf, its page slots and tail rows
+ * then holding whatever was written.  flag: pinned host memory as for
+ * tp_append_stage with check == 2; epoch: even, a fresh one each call. */
+int32_t tp_append_pages(const void* k, const void* v, int32_t in_dtype, int64_t bh, int64_t in_tokens,
+                        int64_t n_head, void* tail_k, void* tail_v, int64_t tail_tokens, int64_t tail_pos,
+                        int32_t copy_rem, const tp_page_layout* layout, const tp_pages* pages, int64_t page_begin,
+                        uint32_t* flag, uint32_t epoch, void* stream);
 
 /* One buffer of tp_grow_rows: rows of src_row bytes (src; NULL when keep is 0)
  * move into rows of dst_row bytes (dst). */

@@ -402,3 +402,45 @@ def test_deferred_check_resolved_by_next_plain_append(device):
     assert rt.actual_seq_len == 5 and rt._tail_len == 5
     rt.append(x[:, :, :2], x[:, :, :2])
     assert rt.actual_seq_len == 7
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.float32])
+@pytest.mark.parametrize("layout_name", ["default", "fast", "odd_split"])
+@pytest.mark.parametrize("before,T", [(0, 64), (0, 65), (0, 191), (1, 127), (1, 128), (63, 65), (63, 128), (37, 300), (64, 130)])
+def test_append_of_whole_pages(device, dtype, layout_name, before, T):
+    """One tp_append_pages launch (check, encode, tail copies) equals the same
+    tokens appended one by one, from an empty, a partial and a just flushed
+    tail; a non-finite value anywhere in it is refused and leaves pages, tail,
+    capacity and counters as they were, so the append can be repeated."""
+    print(f"[append-pages] {dtype} {layout_name} before={before} T={T}", flush=True)
+    int8, l1, deep, split = LAYOUTS[layout_name]
+    cfg = TurboPolarConfig(num_q_heads=4, num_kv_heads=2, use_int8_radii=int8, k_angle_bits_level1=l1,
+                           k_angle_bits_deep=deep, split_dim=split)
+    g = torch.Generator(device=device).manual_seed(before + T)
+    k, v = (torch.randn((2, 2, before + T, 128), generator=g, device=device).to(dtype) for _ in range(2))
+    rt, ref = TurboPolarKVCacheRuntime(cfg), TurboPolarKVCacheRuntime(cfg)
+    for t in range(before + T):
+        ref.append(k[:, :, t:t + 1].contiguous(), v[:, :, t:t + 1].contiguous())
+    if before:
+        rt.append(k[:, :, :before].contiguous(), v[:, :, :before].contiguous())
+    state, tail = rt.get_io_telemetry(), (rt.partial_k, rt.partial_v)
+    kn, vn = k[:, :, before:].contiguous(), v[:, :, before:].contiguous()
+    for which, t in ((0, 0), (1, T - 1), (0, T - 1), (1, min(T - 1, 70))):
+        bad = [kn.clone(), vn.clone()]
+        bad[which][1, 1, t, 77] = float("nan") if t else float("-inf")
+        with pytest.raises(ValueError, match="finite"):
+            rt.append(*bad)
+        assert rt.get_io_telemetry() == state
+        for was, now in zip(tail, (rt.partial_k, rt.partial_v)):
+            assert (was is None and now is None) or torch.equal(was, now)
+    rt.append(kn, vn)
+    assert rt.get_io_telemetry() == ref.get_io_telemetry()
+    n = rt.k_storage.block_count
+    assert n == (before + T) // 64
+    for name in ("radii", "angle_codes_l1", "angle_codes_deep", "radii_scales"):
+        x, y = getattr(rt.k_storage, name), getattr(ref.k_storage, name)
+        assert x is None or torch.equal(x[:, :, :n], y[:, :, :n]), name
+    assert torch.equal(rt.v_storage.codes[:, :, :n], ref.v_storage.codes[:, :, :n])
+    assert torch.equal(rt.v_storage.scales[:, :, :n], ref.v_storage.scales[:, :, :n])
+    if rt._tail_len:
+        assert torch.equal(rt.partial_k, ref.partial_k) and torch.equal(rt.partial_v, ref.partial_v)

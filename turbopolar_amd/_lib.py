@@ -116,6 +116,13 @@ _SIGNATURES = {
         c_i32,
         [c_vp, c_vp, c_i32, c_i64, c_i64, c_i64, c_i64, _P_LAYOUT, _P_PAGES, c_i64, c_vp],
     ),
+    "tp_append_pages": (
+        c_i32,
+        [
+            c_vp, c_vp, c_i32, c_i64, c_i64, c_i64, c_vp, c_vp, c_i64, c_i64, c_i32, _P_LAYOUT, _P_PAGES, c_i64,
+            c_vp, ctypes.c_uint32, c_vp,
+        ],
+    ),
     "tp_fused_qk": (c_i32, [c_vp, c_i64, c_i32, c_i32, _P_LAYOUT, _P_PAGES, c_i32, c_float, c_vp, c_vp]),
     "tp_decode_attention": (
         c_i32,

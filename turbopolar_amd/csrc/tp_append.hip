@@ -21,6 +21,8 @@ struct AppendArgs {
   int64_t in_tokens;
   int64_t copy_begin;
   int64_t n_copy;
+  int64_t scan_begin;   // tokens of each row that the launch reads: all of them
+  int64_t scan_tokens;  // with a check, the copied ones without
   int64_t tail_tokens;  // token capacity of one (b, h) row of the tail
   int64_t tail_pos;
   uint32_t* flag;
@@ -47,15 +49,16 @@ template <bool kF32>
 __global__ __launch_bounds__(256) void append_stage_kernel(AppendArgs a) {
   constexpr int kElems = kF32 ? 4 : 8;           // elements per 16-byte chunk
   constexpr int kChunks = kHeadDim / kElems;     // chunks per token row
-  const int64_t n = a.bh * a.in_tokens * kChunks;
+  const int64_t n = a.bh * a.scan_tokens * kChunks;
   bool bad = false;
   for (int64_t c = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; c < n; c += (int64_t)gridDim.x * blockDim.x) {
-    const int64_t row = c / kChunks;             // (bh, token)
+    const int64_t row = c / kChunks;             // (bh, scanned token)
     const int part = (int)(c - row * kChunks);
-    const int64_t bh = row / a.in_tokens;
-    const int64_t tok = row - bh * a.in_tokens;
-    const uint4 kw = reinterpret_cast<const uint4*>(a.k)[c];
-    const uint4 vw = reinterpret_cast<const uint4*>(a.v)[c];
+    const int64_t bh = row / a.scan_tokens;
+    const int64_t tok = a.scan_begin + (row - bh * a.scan_tokens);
+    const int64_t src = (bh * a.in_tokens + tok) * kChunks + part;
+    const uint4 kw = reinterpret_cast<const uint4*>(a.k)[src];
+    const uint4 vw = reinterpret_cast<const uint4*>(a.v)[src];
     if (a.check) bad = bad || !all_finite(kw, kF32) || !all_finite(vw, kF32);
     const int64_t rel = tok - a.copy_begin;
     if (rel >= 0 && rel < a.n_copy) {
@@ -189,6 +192,9 @@ int32_t tp_append_stage(const void* k, const void* v, int32_t in_dtype, int64_t 
   AppendArgs a;
   a.k = k;
   a.v = v;
+  if (!check && n_copy == 0) return TP_OK;
+  a.scan_begin = check ? 0 : copy_begin;
+  a.scan_tokens = check ? in_tokens : n_copy;
   a.tail_k = tail_k;
   a.tail_v = tail_v;
   a.bh = bh;
@@ -200,7 +206,7 @@ int32_t tp_append_stage(const void* k, const void* v, int32_t in_dtype, int64_t 
   a.flag = flag;
   a.epoch = epoch;
   a.check = check;
-  const int64_t chunks = bh * in_tokens * (in_dtype ? kHeadDim / 4 : kHeadDim / 8);
+  const int64_t chunks = bh * a.scan_tokens * (in_dtype ? kHeadDim / 4 : kHeadDim / 8);
   const unsigned blocks = (unsigned)std::min<int64_t>((chunks + 255) / 256, 1024);
   hipStream_t s = static_cast<hipStream_t>(stream);
   if (in_dtype)

@@ -34,7 +34,67 @@ struct EncodeArgs {
   uint16_t* v_scales;
   int64_t capacity;
   int64_t page_begin;
+  // Append launches (tp_append_pages; flag NULL otherwise): a non-finite value
+  // anywhere in the input stores epoch + 1 into the pinned host word `flag`.
+  // The workgroups past the n_pages pages take each row's tokens outside them,
+  // [0, n_head) and [rem_begin, in_tokens): checked, and copied to the dense
+  // tail (head rows at tail_pos, the others at row 0 if copy_rem).
+  uint32_t* flag;
+  uint32_t epoch;
+  int32_t n_pages;
+  int64_t n_head;
+  int64_t rem_begin;
+  void* tail_k;
+  void* tail_v;
+  int64_t tail_tokens;
+  int64_t tail_pos;
+  int32_t copy_rem;
 };
+
+__device__ __forceinline__ void report_nonfinite(const EncodeArgs& a) {  // every writer stores the same value
+  __hip_atomic_store(a.flag, a.epoch + 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
+// True if any element of a 16-byte chunk is NaN or inf.
+template <bool kF32>
+__device__ __forceinline__ bool any_nonfinite(uint4 w) {
+  const uint32_t ws[4] = {w.x, w.y, w.z, w.w};
+  bool bad = false;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    if constexpr (kF32)
+      bad = bad || (ws[i] & 0x7f800000u) == 0x7f800000u;
+    else
+      bad = bad || (ws[i] & 0x7c00u) == 0x7c00u || (ws[i] & 0x7c000000u) == 0x7c000000u;
+  }
+  return bad;
+}
+
+// The tokens of row blockIdx.y outside the launch's whole pages, by one
+// 256-thread workgroup: at most 126 rows, one 16-byte chunk of k and of v at a time.
+template <bool kF32>
+__device__ __forceinline__ void edge_tokens(const EncodeArgs& a) {
+  constexpr int kChunks = kHeadDim * (kF32 ? 4 : 2) / 16;  // per token row
+  const int64_t bh = blockIdx.y;
+  const int n_head = (int)a.n_head;
+  const int n_rows = n_head + (int)(a.in_tokens - a.rem_begin);
+  bool bad = false;
+  for (int c = threadIdx.x; c < n_rows * kChunks; c += blockDim.x) {
+    const int r = c / kChunks;
+    const int part = c - r * kChunks;
+    const bool head = r < n_head;
+    const int64_t src = (bh * a.in_tokens + (head ? r : a.rem_begin + (r - n_head))) * kChunks + part;
+    const uint4 kw = static_cast<const uint4*>(a.k)[src];
+    const uint4 vw = static_cast<const uint4*>(a.v)[src];
+    bad = bad || any_nonfinite<kF32>(kw) || any_nonfinite<kF32>(vw);
+    if (head || a.copy_rem) {
+      const int64_t dst = (bh * a.tail_tokens + (head ? a.tail_pos + r : r - n_head)) * kChunks + part;
+      static_cast<uint4*>(a.tail_k)[dst] = kw;
+      static_cast<uint4*>(a.tail_v)[dst] = vw;
+    }
+  }
+  if (bad) report_nonfinite(a);
+}
 
 // 32 consecutive input values of one token row: issue the loads (raw) first,
 // convert to floats later, so K and V rows are in flight together.  Tokens past
@@ -120,6 +180,11 @@ __global__ __launch_bounds__(256) void encode_pages_kernel(EncodeArgs a) {
   __shared__ uint8_t s_codes[kPageTokens * kPairs];
   __shared__ uint32_t s_max[4];
 
+  if (a.flag && (int)blockIdx.x == a.n_pages) {
+    edge_tokens<kF32>(a);
+    return;
+  }
+  bool bad = false;
   const int page = blockIdx.x;
   const int64_t bh = blockIdx.y;
   const int tid = threadIdx.x;
@@ -135,6 +200,10 @@ __global__ __launch_bounds__(256) void encode_pages_kernel(EncodeArgs a) {
   if (a.k) load_row32<kF32>(a.k, in_off, valid, kraw);
 
   if (a.k) {
+    if (a.flag) {
+#pragma unroll
+      for (int i = 0; i < (kF32 ? 8 : 4); ++i) bad = bad || any_nonfinite<kF32>(kraw.w[i]);
+    }
     uint16_t r16[16];
     // Angles whose fast fp32 atan2 lands too close to an fp16 rounding
     // boundary are flagged here and recomputed in float64 after the loop, so
@@ -228,6 +297,10 @@ __global__ __launch_bounds__(256) void encode_pages_kernel(EncodeArgs a) {
 
   if (a.v) {
     load_row32<kF32>(a.v, in_off, valid, vraw);
+    if (a.flag) {
+#pragma unroll
+      for (int i = 0; i < (kF32 ? 8 : 4); ++i) bad = bad || any_nonfinite<kF32>(vraw.w[i]);
+    }
     // v_quant/encoder.py:21-25: s = f16(max|v| / 127) (1e-4 if zero),
     // code = int8(clip(rint(v / s))) with an fp16 quotient for fp16 inputs.
     float m = 0.0f;
@@ -253,6 +326,7 @@ __global__ __launch_bounds__(256) void encode_pages_kernel(EncodeArgs a) {
     dst[1] = make_uint4(packed[4], packed[5], packed[6], packed[7]);
     a.v_scales[row * kVGroups + qq] = s16;
   }
+  if (bad) report_nonfinite(a);
 }
 
 // ---- fp16 fast path for the runtime's two layouts ----------------------------
@@ -396,12 +470,20 @@ __device__ __forceinline__ uint32_t lcode_exact_byte(uint16_t lr16, float ls) {
 // of n sits in bit n - 1 - j.
 __device__ __forceinline__ uint32_t push_flag(uint32_t m, bool f) { return (m << 1) | (f ? 1u : 0u); }
 
+// The non-finite check of an append (a.flag) rides on the values in registers:
+// a packed maximum of the key words, and the value groups' maxima that the
+// scales need anyway.  A check kernel of its own read the whole input a second
+// time (24 us for 32,773 tokens of 8 heads beside 39 of encoding).
 template <int L>
 __global__ __launch_bounds__(256) void encode_f16_kernel(EncodeArgs a) {
   constexpr bool kFastLayout = L == kEncFast;
   constexpr int kBits = kFastLayout ? 8 : 4;
   __shared__ uint32_t s_max[4];
 
+  if (a.flag && (int)blockIdx.x == a.n_pages) {
+    edge_tokens<false>(a);
+    return;
+  }
   const int page = blockIdx.x;
   const int64_t bh = blockIdx.y;
   const int tid = threadIdx.x;
@@ -415,6 +497,11 @@ __global__ __launch_bounds__(256) void encode_f16_kernel(EncodeArgs a) {
 
   RawRow32<false> kraw;
   load_row32<false>(a.k, in_off, valid, kraw);
+  u16x2 k2 = {0, 0};  // maxima of |k|'s bit patterns: 0x7c00 and above is inf or NaN
+#pragma unroll
+  for (int i = 0; i < 16; ++i)
+    k2 = __builtin_elementwise_max(k2, __builtin_bit_cast(u16x2, raw_word(kraw, i) & 0x7fff7fffu));
+  const bool k_bad = max((uint32_t)k2[0], (uint32_t)k2[1]) >= 0x7c00u;
   uint16_t r16[16];
   uint32_t cw[kFastLayout ? 4 : 2];
 #pragma unroll
@@ -559,6 +646,7 @@ __global__ __launch_bounds__(256) void encode_f16_kernel(EncodeArgs a) {
     vw[i >> 2] = vcode_fast_byte(raw_val(vraw, i), rs, one, (uint32_t)(i & 3), vw[i >> 2], &near);
     vfix = push_flag(vfix, near);
   }
+  if (a.flag && (k_bad || nonfinite)) report_nonfinite(a);
   if (nonfinite) vfix = 0xffffffffu;  // inf or NaN in the group: every value on the exact path
   const uint16_t* vin = static_cast<const uint16_t*>(a.v) + in_off;
   while (vfix) {  // exact quotients of the flagged values, reloaded (never padding)
@@ -739,13 +827,10 @@ __global__ __launch_bounds__(256) void lcode_exhaustive_kernel(unsigned long lon
 
 using namespace tp;
 
-extern "C" {
-
-int32_t tp_encode_pages(const void* k, const void* v, int32_t in_dtype, int64_t bh,
-                        int64_t in_tokens, int64_t token_begin, int64_t n_tokens,
-                        const tp_page_layout* layout, const tp_pages* pages, int64_t page_begin,
-                        void* stream) {
-  clear_error();
+// Checks one encode launch's arguments and fills `a` (no launch).
+static int32_t fill_encode(EncodeArgs& a, const void* k, const void* v, int32_t in_dtype, int64_t bh,
+                           int64_t in_tokens, int64_t token_begin, int64_t n_tokens,
+                           const tp_page_layout* layout, const tp_pages* pages, int64_t page_begin) {
   int l1_row = 0, deep_row = 0;
   if (!check_layout(layout, &l1_row, &deep_row)) return TP_ERR_UNSUPPORTED;
   if (!pages) {
@@ -760,7 +845,7 @@ int32_t tp_encode_pages(const void* k, const void* v, int32_t in_dtype, int64_t 
     set_error("k and v are both NULL");
     return TP_ERR_INVALID;
   }
-  if (n_tokens == 0) return TP_OK;
+  if (n_tokens == 0) return TP_OK;  // nothing to launch
   if (bh < 1 || bh > 65535 || n_tokens < 0 || token_begin < 0 || in_tokens < 0 ||
       token_begin + n_tokens > in_tokens) {
     set_error("bad token range: bh=%lld in_tokens=%lld token_begin=%lld n_tokens=%lld",
@@ -796,7 +881,7 @@ int32_t tp_encode_pages(const void* k, const void* v, int32_t in_dtype, int64_t 
       return TP_ERR_INVALID;
     }
   }
-  EncodeArgs a;
+  a = EncodeArgs{};
   a.k = k;
   a.v = v;
   a.in_tokens = in_tokens;
@@ -816,22 +901,93 @@ int32_t tp_encode_pages(const void* k, const void* v, int32_t in_dtype, int64_t 
   a.v_scales = static_cast<uint16_t*>(pages->v_scales);
   a.capacity = pages->capacity;
   a.page_begin = page_begin;
-  const dim3 grid((unsigned)n_pages, (unsigned)bh);
-  hipStream_t s = static_cast<hipStream_t>(stream);
+  a.n_pages = (int32_t)n_pages;
+  return TP_OK;
+}
+
+// Launches the page encoder over a filled `a`; `edge` adds each row's workgroup
+// for the tokens outside the pages.
+static void launch_encode(const EncodeArgs& a, int32_t in_dtype, int64_t bh, bool edge, hipStream_t s) {
+  const dim3 grid((unsigned)(a.n_pages + (edge ? 1 : 0)), (unsigned)bh);
   // fp16 K and V in the runtime's two layouts take the specialised kernel.
-  const bool is_default = !layout->int8_radii && layout->l1_bits == 4 && layout->deep_bits == 4 &&
-                          layout->split_dim == 64 && !(((uintptr_t)pages->angle_l1 | (uintptr_t)pages->angle_deep) & 7u);
-  const bool is_fast = layout->int8_radii && layout->deep_bits == 8 && layout->split_dim == 0 &&
-                       !((uintptr_t)pages->angle_deep & 15u);
-  if (in_dtype == 0 && k && v && is_default)
+  const bool is_default = !a.int8_radii && a.l1_bits == 4 && a.deep_bits == 4 && a.split_half == 32 &&
+                          !(((uintptr_t)a.angle_l1 | (uintptr_t)a.angle_deep) & 7u);
+  const bool is_fast = a.int8_radii && a.deep_bits == 8 && a.split_half == 0 && !((uintptr_t)a.angle_deep & 15u);
+  if (in_dtype == 0 && a.k && a.v && is_default)
     hipLaunchKernelGGL(encode_f16_kernel<kEncDefault>, grid, dim3(256), 0, s, a);
-  else if (in_dtype == 0 && k && v && is_fast)
+  else if (in_dtype == 0 && a.k && a.v && is_fast)
     hipLaunchKernelGGL(encode_f16_kernel<kEncFast>, grid, dim3(256), 0, s, a);
   else if (in_dtype == 1)
     hipLaunchKernelGGL(encode_pages_kernel<true>, grid, dim3(256), 0, s, a);
   else
     hipLaunchKernelGGL(encode_pages_kernel<false>, grid, dim3(256), 0, s, a);
+}
+
+extern "C" {
+
+int32_t tp_encode_pages(const void* k, const void* v, int32_t in_dtype, int64_t bh,
+                        int64_t in_tokens, int64_t token_begin, int64_t n_tokens,
+                        const tp_page_layout* layout, const tp_pages* pages, int64_t page_begin,
+                        void* stream) {
+  clear_error();
+  EncodeArgs a{};
+  const int32_t st = fill_encode(a, k, v, in_dtype, bh, in_tokens, token_begin, n_tokens, layout, pages, page_begin);
+  if (st != TP_OK || a.n_pages == 0) return st;
+  launch_encode(a, in_dtype, bh, false, static_cast<hipStream_t>(stream));
   return launch_status("tp_encode_pages");
+}
+
+int32_t tp_append_pages(const void* k, const void* v, int32_t in_dtype, int64_t bh, int64_t in_tokens,
+                        int64_t n_head, void* tail_k, void* tail_v, int64_t tail_tokens, int64_t tail_pos,
+                        int32_t copy_rem, const tp_page_layout* layout, const tp_pages* pages, int64_t page_begin,
+                        uint32_t* flag, uint32_t epoch, void* stream) {
+  clear_error();
+  if (!k || !v || n_head < 0 || n_head >= kPageTokens || in_tokens - n_head < kPageTokens) {
+    set_error("bad input: k=%p v=%p, %lld tokens with %lld before the first whole page", k, v, (long long)in_tokens,
+              (long long)n_head);
+    return TP_ERR_INVALID;
+  }
+  if (!flag || (epoch & 1u)) {
+    set_error("a pinned host flag and an even epoch are needed");
+    return TP_ERR_INVALID;
+  }
+  const int64_t n_full = (in_tokens - n_head) / kPageTokens;
+  EncodeArgs a{};
+  const int32_t st =
+      fill_encode(a, k, v, in_dtype, bh, in_tokens, n_head, n_full * kPageTokens, layout, pages, page_begin);
+  if (st != TP_OK) return st;
+  a.flag = flag;
+  a.epoch = epoch;
+  a.n_head = n_head;
+  a.rem_begin = n_head + n_full * kPageTokens;
+  const int64_t rem = in_tokens - a.rem_begin;
+  if (n_head + rem > 0) {
+    const bool copies = n_head > 0 || (copy_rem && rem > 0);
+    if (copies && (!tail_k || !tail_v || (((uintptr_t)tail_k | (uintptr_t)tail_v) & 15u) || tail_pos < 0 ||
+                   tail_pos + n_head > tail_tokens || (copy_rem && rem > tail_tokens) || (copy_rem && n_head > 0))) {
+      set_error("tail buffers missing, misaligned or too small: %lld tokens at %lld and %lld at 0 of %lld",
+                (long long)n_head, (long long)tail_pos, (long long)(copy_rem ? rem : 0), (long long)tail_tokens);
+      return TP_ERR_INVALID;
+    }
+    a.tail_k = tail_k;
+    a.tail_v = tail_v;
+    a.tail_tokens = tail_tokens;
+    a.tail_pos = tail_pos;
+    a.copy_rem = copy_rem != 0;
+  }
+  hipStream_t s = static_cast<hipStream_t>(stream);
+  launch_encode(a, in_dtype, bh, n_head + rem > 0, s);
+  const int32_t ls = launch_status("tp_append_pages");
+  if (ls != TP_OK) return ls;
+  if (hipStreamSynchronize(s) != hipSuccess) {
+    set_error("tp_append_pages: synchronising the stream failed");
+    return TP_ERR_HIP;
+  }
+  if (*reinterpret_cast<volatile uint32_t*>(flag) == epoch + 1u) {
+    set_error("append() inputs must contain finite values");
+    return TP_ERR_NONFINITE;
+  }
+  return TP_OK;
 }
 
 int32_t tp_selftest_f16_tables(uint16_t* sqrt_out, uint16_t* log_out, uint8_t* codes_out,

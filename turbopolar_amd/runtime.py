@@ -10,14 +10,16 @@ rfsn_v11/generation/turbo_polar_cache.py:18-395.  Differences of mechanism
   them, like the reference's immutable arrays); ``get_fused_attention_inputs``
   returns views of it, valid until the next append, so a decode step copies
   nothing;
-* full pages are encoded by one ``tp_encode_pages`` launch per append, written
-  straight into the storage slots (no per-page Python loop, no intermediate
-  block copies);
+* an append of whole pages is one ``tp_append_pages`` launch, which checks,
+  encodes and copies to the tail in one read of the input and writes straight
+  into the storage slots (no per-page Python loop, no intermediate block
+  copies);
 * a bulk append reserves capacity once (the doubling telemetry is unchanged).
 """
 
 from __future__ import annotations
 
+import ctypes
 from typing import Any, Dict, Optional, Tuple
 
 import torch
@@ -165,40 +167,47 @@ class TurboPolarKVCacheRuntime:
         v = B * H * PAGE * self._head_dim + B * H * PAGE * (self._head_dim // 32) * 2
         return k + v
 
-    def _reserve(self, needed: int, fresh: int, device) -> None:
-        """Room for ``needed`` pages in both storages, the last ``fresh`` of
-        which the caller encodes next."""
-        B, H = self._batch_size, self._num_kv_heads
+    def _growth(self, needed: int, fresh: int, B: int, H: int, device) -> Optional[Growth]:
+        """Buffers with room for ``needed`` pages in both storages, the last
+        ``fresh`` of which the caller encodes next; None if they have it."""
         ks, vs = self.k_storage, self.v_storage
         if needed <= ks.capacity and needed <= vs.capacity:
-            return
-        if ks.radii is None:
-            ks.metadata = self.polar_encoder.metadata
+            return None
         growth = Growth(fresh)
         ks.plan(growth, needed, self.polar_encoder, B, H, device)
         vs.plan(growth, needed, B, H, device)
         growth.fill()
-        growth.commit()
+        return growth
 
-    def _encode_into_storage(self, k: torch.Tensor, v: torch.Tensor, token_begin: int, n_pages: int) -> None:
-        start = self.k_storage.block_count
-        self._reserve(start + n_pages, n_pages, k.device)
-        encode_pages(
-            k, v, token_begin, n_pages * PAGE, self.polar_encoder.layout,
-            pages_of(self.k_storage, self.v_storage), start,
-        )
+    def _grown(self, growth: Optional[Growth]) -> None:
+        if growth is not None:
+            if self.k_storage.radii is None:
+                self.k_storage.metadata = self.polar_encoder.metadata
+            growth.commit()
+
+    def _pages_added(self, n_pages: int) -> None:
         self.k_storage.block_count += n_pages
         self.v_storage.block_count += n_pages
         self.total_blocks += n_pages
         self.bytes_written += n_pages * self._page_bytes()
 
+    def _encode_into_storage(self, k: torch.Tensor, v: torch.Tensor, token_begin: int, n_pages: int) -> None:
+        start = self.k_storage.block_count
+        self._grown(self._growth(start + n_pages, n_pages, self._batch_size, self._num_kv_heads, k.device))
+        encode_pages(
+            k, v, token_begin, n_pages * PAGE, self.polar_encoder.layout,
+            pages_of(self.k_storage, self.v_storage), start,
+        )
+        self._pages_added(n_pages)
+
     def append(self, k_new: torch.Tensor, v_new: torch.Tensor, defer_check: bool = False) -> None:
         """turbo_polar_cache.py:106-126: extend the tail, flush every full page.
 
-        On a HIP device one tp_append_stage launch checks the whole input for
-        non-finite values and copies the tokens bound for the dense tail, with
-        a single 4-byte read back (the reference synchronises once per input
-        in mx.isfinite(...).all()).  Errors come in the reference's order and
+        On a HIP device one launch checks the whole input for non-finite values
+        and copies the tokens bound for the dense tail (tp_append_stage; with
+        whole pages tp_append_pages, which encodes them too), with a single
+        4-byte read back (the reference synchronises once per input in
+        mx.isfinite(...).all()).  Errors come in the reference's order and
         leave the cache unchanged.
 
         ``defer_check`` (no counterpart in the reference; single-token appends
@@ -222,8 +231,9 @@ class TurboPolarKVCacheRuntime:
         if self._tail_k is not None and self._tail_k.device != k_new.device:
             raise ValueError(f"append() inputs moved from {self._tail_k.device} to {k_new.device}")
         if self._tail_k is None:
-            self._tail_k = torch.zeros((B, H, PAGE, D), dtype=k_new.dtype, device=k_new.device)
-            self._tail_v = torch.zeros((B, H, PAGE, D), dtype=k_new.dtype, device=k_new.device)
+            # Rows past the tail's length are never read, so they are not cleared.
+            self._tail_k = torch.empty((B, H, PAGE, D), dtype=k_new.dtype, device=k_new.device)
+            self._tail_v = torch.empty((B, H, PAGE, D), dtype=k_new.dtype, device=k_new.device)
         if self._flag is None:
             # Written by the staging kernel and read after one synchronisation,
             # with no device-to-host copy.
@@ -234,6 +244,9 @@ class TurboPolarKVCacheRuntime:
             n_head, head_dst = T, 0
         else:
             n_head, head_dst = 0, 0
+        if T - n_head >= PAGE:
+            self._append_pages(k_new, v_new, n_head)
+            return
         # A deferred single token lands at tail position tail_len (< 64) and
         # overwrites nothing valid (a pending append never lets a later one
         # restart the tail at row 0), so restoring the counters undoes it.
@@ -245,18 +258,47 @@ class TurboPolarKVCacheRuntime:
         self._commit_invariants(k_new)
         self.actual_seq_len += T
         self._tail_len += n_head
-        pos = n_head
         if self._tail_len == PAGE:
             self._encode_into_storage(self._tail_k, self._tail_v, 0, 1)
             self._tail_len = 0
-        n_full = (T - pos) // PAGE
-        if n_full:
-            self._encode_into_storage(k_new, v_new, pos, n_full)
-            pos += n_full * PAGE
-        rem = T - pos
-        if rem:
-            self._stage(k_new, v_new, pos, rem, 0, check=0)
-            self._tail_len = rem
+        if n_head < T:
+            self._stage(k_new, v_new, n_head, T - n_head, 0, check=0)
+            self._tail_len = T - n_head
+
+    def _append_pages(self, k_new, v_new, n_head: int) -> None:
+        """An append of at least one whole page past the ``n_head`` tokens that
+        complete the dense tail: one tp_append_pages launch checks every value,
+        encodes the whole pages and copies the tokens bound for the tail, with
+        one synchronisation.  Pages are encoded into slots past the stored ones
+        (of larger buffers, if the store has to grow), which only become part of
+        the cache once the verdict is in."""
+        B, H, T, _ = k_new.shape
+        ks = self.k_storage
+        rest, flush = (T - n_head) % PAGE, 1 if self._tail_len else 0
+        n_full = (T - n_head) // PAGE
+        start = ks.block_count
+        growth = self._growth(start + flush + n_full, flush + n_full, B, H, k_new.device)
+        self._epoch = ((self._epoch + 2) & 0xFFFFFFFE) or 2
+        # Rows of a tail that holds tokens are only overwritten after the verdict.
+        with _lib.on_device(k_new.device):
+            st = _lib.lib().tp_append_pages(
+                k_new.data_ptr(), v_new.data_ptr(), 1 if k_new.dtype == torch.float32 else 0, B * H, T, n_head,
+                self._tail_k.data_ptr(), self._tail_v.data_ptr(), PAGE, self._tail_len, 0 if flush else 1,
+                ctypes.byref(self.polar_encoder.layout), ctypes.byref(pages_of(ks, self.v_storage, growth)),
+                start + flush, self._flag.data_ptr(), self._epoch, _lib.raw_stream(k_new.device.index),
+            )
+        if st == _lib.TP_ERR_NONFINITE:
+            raise ValueError("append() inputs must contain finite values")
+        _lib.check(st, "tp_append_pages")
+        self._grown(growth)
+        self._commit_invariants(k_new)
+        self.actual_seq_len += T
+        if flush:
+            self._encode_into_storage(self._tail_k, self._tail_v, 0, 1)
+        self._pages_added(n_full)
+        if rest and flush:
+            self._stage(k_new, v_new, T - rest, rest, 0, check=0)
+        self._tail_len = rest
 
     def _state(self) -> tuple:
         return (self.actual_seq_len, self._tail_len, self.k_storage.block_count, self.v_storage.block_count,

@@ -108,6 +108,13 @@ class Growth:
             st = _lib.lib().tp_grow_rows(descs, len(rows), new.shape[0] * new.shape[1], _lib.stream_handle(new.device))
         _lib.check(st, "tp_grow_rows")
 
+    def buffer(self, storage, name: str):
+        """``storage``'s buffer as it will be after ``commit``."""
+        for s, made, _, _, _ in self._sets:
+            if s is storage:
+                return made[name]
+        return getattr(storage, name)
+
     def commit(self) -> None:
         for storage, made, cap, reallocs, grown in self._sets:
             for name, new in made.items():
@@ -242,14 +249,19 @@ class QuantVBlockStorage:
         )
 
 
-def pages_of(k_storage: PolarKBlockStorage, v_storage: QuantVBlockStorage) -> _lib.TPPages:
-    """``tp_pages`` over the whole capacity of a pair of storages."""
+def pages_of(k_storage: PolarKBlockStorage, v_storage: QuantVBlockStorage, growth: Optional[Growth] = None) -> _lib.TPPages:
+    """``tp_pages`` over the whole capacity of a pair of storages (as they will
+    be after ``growth`` is committed, if given)."""
+    if growth is None:
+        get, capacity = getattr, k_storage.capacity
+    else:
+        get, capacity = growth.buffer, growth.buffer(k_storage, "radii").shape[2]
     return _lib.TPPages(
-        _lib.ptr(k_storage.radii),
-        _lib.ptr(k_storage.radii_scales),
-        _lib.ptr(k_storage.angle_codes_l1),
-        _lib.ptr(k_storage.angle_codes_deep),
-        _lib.ptr(v_storage.codes),
-        _lib.ptr(v_storage.scales),
-        int(k_storage.capacity),
+        _lib.ptr(get(k_storage, "radii")),
+        _lib.ptr(get(k_storage, "radii_scales")),
+        _lib.ptr(get(k_storage, "angle_codes_l1")),
+        _lib.ptr(get(k_storage, "angle_codes_deep")),
+        _lib.ptr(get(v_storage, "codes")),
+        _lib.ptr(get(v_storage, "scales")),
+        int(capacity),
     )
