@@ -80,6 +80,50 @@ def _qjl_case(device, layout_name, hq, hkv, S, tail, seed, B=1, P=64):
     return block, qv, host, tk, tv, q, qd, pay, qs, tup
 
 
+@pytest.mark.parametrize("dtype", [torch.float16, torch.float32])
+@pytest.mark.parametrize("rows,P", [(1, 64), (15, 8), (16, 16), (17, 24), (33, 56), (100, 72), (31, 128), (47, 200),
+                                    (64, 256), (16 * 1024 + 5, 64)])
+def test_sketch_row_tiles(device, dtype, rows, P):
+    """The matrix-core sketch kernel at partial row tiles, every packing width
+    (whole and half column tiles) and a launch whose workgroups walk several
+    tiles: bits against the float64 projection away from zero (fp32 sums of 128
+    products err by less than 128 * 2^-24 |e|), norms within one fp16 ulp."""
+    print(f"[sketch] {dtype} rows={rows} P={P}", flush=True)
+    enc = QJLResidualEncoder(_cfg(P=P))
+    g = torch.Generator(device=device).manual_seed(rows + P)
+    e = torch.randn((1, 1, 1, rows, 128), generator=g, device=device).to(dtype)
+    pay = enc.compute_residual_sketch(e)
+    assert torch.equal(enc.query_signs(e[:, 0, 0]), pay.packed_signs[:, 0, 0])
+    x = e[0, 0, 0].double().cpu().numpy()
+    proj = x @ enc.W_host.astype(np.float64)
+    norm = np.linalg.norm(x, axis=-1)
+    bits = np.unpackbits(pay.packed_signs[0, 0, 0].cpu().numpy(), axis=-1, bitorder="little")
+    wrong = (bits == 1) != (proj >= 0)
+    assert not np.any(wrong & (np.abs(proj) > 128 * 2.0 ** -24 * norm[:, None]))
+    gn = pay.norms[0, 0, 0].float().cpu().numpy()
+    assert np.all(np.abs(gn - norm) <= _fp16_ulp(norm))
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.float32])
+def test_sketch_unaligned_and_nonfinite_rows(device, dtype):
+    """Rows that are not 16-byte aligned keep the scalar kernel, and both kernels
+    agree on rows of zeros, infinities, NaN, the largest and subnormal values."""
+    enc = QJLResidualEncoder(_cfg())
+    g = torch.Generator(device=device).manual_seed(9)
+    flat = torch.randn(128 * 40 + 1, generator=g, device=device).to(dtype)
+    e = flat[1:].reshape(40, 128)
+    e[0] = 0.0
+    e[1, 5], e[2, 7], e[3, 100] = float("inf"), float("-inf"), float("nan")
+    e[4, 3], e[4, 90] = float("inf"), float("inf")
+    e[5] *= 60000.0 / float(e[5].abs().max())
+    e[6] *= 6e-8
+    assert e.data_ptr() % 16
+    a, an = enc._sketch(e, True)
+    b, bn = enc._sketch(e.clone(), True)
+    assert torch.equal(a, b)
+    assert torch.allclose(an.float(), bn.float(), rtol=2e-3, equal_nan=True)
+
+
 def test_dot_estimate_matches_oracle(device):
     block, qv, host, tk, tv, q, qd, pay, qs, tup = _qjl_case(device, "default", 8, 2, 3, 0, 11)
     got = qjl_dot_estimate(qd, pay, qs).cpu().numpy()
