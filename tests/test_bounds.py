@@ -20,7 +20,9 @@ import pytest
 
 from turbopolar_amd import _lib
 
-LAYOUTS = {"default": (0, 4, 4, 64), "fast": (1, 4, 8, 0), "deep2": (0, 4, 2, 64), "l1_8bit": (0, 8, 4, 32)}
+LAYOUTS = {"default": (0, 4, 4, 64), "fast": (1, 4, 8, 0), "deep2": (0, 4, 2, 64), "l1_8bit": (0, 8, 4, 32), "odd_split": (1, 4, 2, 46),
+           "deep2_only": (0, 4, 2, 0), "l1_only": (1, 8, 2, 128), "wide": (0, 8, 8, 30), "one_deep": (0, 4, 2, 126),
+           "one_l1": (1, 4, 8, 2)}
 
 
 def run(layout="default", batch=1, hq=32, hkv=8, n_pages=64, capacity=None, tail=0, tail_stride=None, seq=None,
@@ -68,6 +70,9 @@ CASES = [
     dict(n_pages=21, kernel=1),                        # fused QK: the last page reloaded past n_pages
     dict(n_pages=5, kernel=1, layout="fast"),
     dict(n_pages=5, kernel=1, layout="deep2", hq=20, hkv=1),
+    *[dict(layout=lay, **kw) for lay in ("odd_split", "deep2_only", "l1_only", "wide", "one_deep", "one_l1")
+      for kw in (dict(n_pages=7, pps=4, tail=3, tail_stride=3), dict(n_pages=21, pps=9, hq=24, hkv=2),
+                 dict(n_pages=5, kernel=1, batch=2))],
     dict(n_pages=100, capacity=128, batch=2, hq=16, hkv=4),
     dict(hq=24, hkv=2, n_pages=20, qjl=True),          # GQA 12: the row token order of default pages
     dict(hq=40, hkv=2, n_pages=9, pps=2, dense_v=True),

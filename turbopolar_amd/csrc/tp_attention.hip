@@ -73,8 +73,10 @@ __device__ unsigned long long g_timeline[kTimelineGroups][kTimelineStamps];
 
 // kKindDefaultHR: default-layout pages in the half-row token order (below),
 // the decode kernel's form of the default layout for head blocks of at most 8
-// query heads.
-enum LayoutKind { kKindDefault = 0, kKindFast = 1, kKindGeneric = 2, kKindDefaultHR = 3 };
+// query heads.  kKindAnyF16 / kKindAnyI8: any other layout, by its radii.
+// kKindNone: a launch without pages (the dense tail alone).
+enum LayoutKind { kKindDefault = 0, kKindFast = 1, kKindAnyF16 = 2, kKindDefaultHR = 3, kKindAnyI8 = 4, kKindNone = 5 };
+constexpr bool any_kind(int kind) { return kind == kKindAnyF16 || kind == kKindAnyI8; }
 
 // Division by a launch constant d as a multiply and a shift: for n < 2^31,
 // l = ceil(log2 d) and m = floor(2^(31+l) / d) + 1 (< 2^32), floor(n / d) =
@@ -167,6 +169,12 @@ __device__ __forceinline__ uint4 ldnt4(const void* p) {
   const u32x4 v = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(p));
   return make_uint4(v.x, v.y, v.z, v.w);
 }
+// 16 bytes at an 8-byte boundary (level-1 rows).
+typedef u32x4 u32x4_8 __attribute__((aligned(8)));
+__device__ __forceinline__ uint4 ldnt4_8(const void* p) {
+  const u32x4 v = __builtin_nontemporal_load(reinterpret_cast<const u32x4_8*>(p));
+  return make_uint4(v.x, v.y, v.z, v.w);
+}
 __device__ __forceinline__ uint2 ldnt2(const void* p) {
   const u32x2 v = __builtin_nontemporal_load(reinterpret_cast<const u32x2*>(p));
   return make_uint2(v.x, v.y);
@@ -242,9 +250,9 @@ __device__ __forceinline__ void i8x4_to_f16(uint32_t w, half2v& lo, half2v& hi) 
   hi = __builtin_bit_cast(half2v, b) - bias;
 }
 
+constexpr int kLutDeep = 256;  // first deep entry of Lut::code
 struct Lut {
-  uint32_t l1[256];
-  uint32_t deep[256];
+  uint32_t code[512];  // (cos, sin) of the level-1 codes, then of the deep codes
   uint2 pair[256];  // 4-bit layouts: (cos, sin) of both nibbles of a code byte
 };
 
@@ -254,10 +262,10 @@ __device__ __forceinline__ void build_lut(Lut& lut, const AttnArgs& a, int tid) 
   if constexpr (KIND == kKindDefault || KIND == kKindDefaultHR) {
     lut.pair[c] = make_uint2(make_cs(c & 15u, 4), make_cs(c >> 4, 4));
   } else if constexpr (KIND == kKindFast) {
-    lut.deep[c] = make_cs(c, 8);
-  } else {
-    if (c < (1u << a.l1_bits)) lut.l1[c] = make_cs(c, a.l1_bits);
-    if (c < (1u << a.deep_bits)) lut.deep[c] = make_cs(c, a.deep_bits);
+    lut.code[kLutDeep + c] = make_cs(c, 8);
+  } else if constexpr (any_kind(KIND)) {
+    if (c < (1u << a.l1_bits)) lut.code[c] = make_cs(c, a.l1_bits);
+    if (c < (1u << a.deep_bits)) lut.code[kLutDeep + c] = make_cs(c, a.deep_bits);
   }
 }
 
@@ -345,6 +353,20 @@ __host__ __device__ inline int k_code_row(int t) { return t * 16; }
 __host__ __device__ inline int64_t fast_base(int64_t slot, int l4) { return slot * (kPageTokens * kPairs) + 16 * l4; }
 __host__ __device__ inline int fast_row(int t) { return t * kPairs; }
 __host__ __device__ inline int64_t fast_scale(int64_t slot) { return slot * 2; }
+// Any other layout: radii as above (fp16: k_radii_*, int8: fast_*); the page's
+// code rows, 64 of l1_row and 64 of deep_row bytes, as 16-byte chunks: lane
+// `lane` takes chunks lane + 64 j, j < kAnyChunks, those past the last one
+// rereading it (at most 64 code bytes a token, so 256 chunks).
+constexpr int kAnyChunks = 4;
+__host__ __device__ inline int any_chunk(int lane, int j, int l1_row, int deep_row) {
+  const int c = lane + 64 * j, last = 4 * (l1_row + deep_row) - 1;
+  return c < last ? c : last;
+}
+__host__ __device__ inline bool any_chunk_from_l1(int chunk, int l1_row) { return chunk < 4 * l1_row; }
+__host__ __device__ inline int64_t any_chunk_off(int64_t slot, int chunk, int l1_row, int deep_row) {
+  return any_chunk_from_l1(chunk, l1_row) ? slot * (kPageTokens * l1_row) + 16 * chunk
+                                          : slot * (kPageTokens * deep_row) + 16 * (chunk - 4 * l1_row);
+}
 // Value codes: 8 bytes of token v_token(ks, l4, e), dims 8*l16 .. +7, at
 // v_code_base + v_code_row(ks, l4, e); the page's 512 bytes of scales as the
 // dwords `lane` and `lane + 64` at v_scale_base + 4*lane (+256).
@@ -562,9 +584,20 @@ struct KRegs<kKindFast> {  // int8 log radii + fp16 page scale, 8-bit deep codes
 };
 
 template <>
-struct KRegs<kKindGeneric> {  // any layout: codes are gathered during the math
-  int64_t slot;
+struct KRegs<kKindAnyF16> {  // any layout with fp16 radii; the page's code rows by chunks
+  uint4 r[4][2];
+  uint4 c[kAnyChunks];
 };
+
+template <>
+struct KRegs<kKindAnyI8> {  // any layout with int8 log radii
+  uint4 r[4];
+  uint4 c[kAnyChunks];
+  uint32_t ls_bits;
+};
+
+template <>
+struct KRegs<kKindNone> {};
 
 template <int KIND>
 __device__ __forceinline__ void load_k(const AttnArgs& a, int64_t slot, int l16, int l4, KRegs<KIND>& k) {
@@ -599,8 +632,26 @@ __device__ __forceinline__ void load_k(const AttnArgs& a, int64_t slot, int l16,
       k.c[mt] = ldnt4(cbase + fast_row(t));
     }
     k.ls_bits = *reinterpret_cast<const uint16_t*>(reinterpret_cast<const char*>(a.radii_scales) + fast_scale(slot));
-  } else {
-    k.slot = slot;
+  } else if constexpr (any_kind(KIND)) {
+#pragma unroll
+    for (int mt = 0; mt < 4; ++mt) {
+      const int t = 16 * mt + l16;
+      if constexpr (KIND == kKindAnyF16) {
+        const char* rp = static_cast<const char*>(a.radii) + k_radii_base(slot, l4) + k_radii_row(t);
+        k.r[mt][0] = ldnt4(rp);
+        k.r[mt][1] = ldnt4(rp + 16);
+      } else {
+        k.r[mt] = ldnt4(static_cast<const char*>(a.radii) + fast_base(slot, l4) + fast_row(t));
+      }
+    }
+#pragma unroll
+    for (int j = 0; j < kAnyChunks; ++j) {
+      const int c = any_chunk(16 * l4 + l16, j, a.l1_row, a.deep_row);
+      const uint8_t* base = any_chunk_from_l1(c, a.l1_row) ? a.angle_l1 : a.angle_deep;
+      k.c[j] = ldnt4_8(base + any_chunk_off(slot, c, a.l1_row, a.deep_row));
+    }
+    if constexpr (KIND == kKindAnyI8)
+      k.ls_bits = *reinterpret_cast<const uint16_t*>(reinterpret_cast<const char*>(a.radii_scales) + fast_scale(slot));
   }
 }
 
@@ -637,11 +688,43 @@ __device__ __forceinline__ void fold_halves(const float4v& acc, float4v& s, int 
   s[j + 1] = acc[2] + from_lane_xor8(acc[3]);
 }
 
+// ---- codes of any layout ----------------------------------------------------------
+//
+// A lane needs the codes of pairs 16 l4 .. +15 of four tokens.  Gathered byte by
+// byte from memory (64 loads a lane and page, none of them ahead of its use) the
+// codes took the decode step of a 2-bit deep layout at 16,400 tokens x 8 heads
+// to 54 us (16.5 now).  Instead a page's rows travel with the other page loads as whole
+// chunks, go through the wave's own LDS (its merge area, free until the pages
+// are done), and come back as a bit stream per token: 16 codes of 2, 4 or 8 bits
+// from the bit where the lane's run starts, five dwords funnelled to that bit.
+// A run that holds the split (split_dim not a multiple of 32) takes both rows'
+// streams and picks per pair.
+constexpr int kAnyCodeBytes = 16 * (64 * kAnyChunks + 2);  // the chunks, and what a stream reads past them
+
+__device__ __forceinline__ void code_stream(const uint32_t* words, int bit, uint32_t (&s)[4]) {
+  const uint32_t* d = words + (bit >> 5);
+  const uint32_t sh = (uint32_t)bit & 31u;
+  const uint32_t w[5] = {d[0], d[1], d[2], d[3], d[4]};
+#pragma unroll
+  for (int i = 0; i < 4; ++i) s[i] = __builtin_amdgcn_alignbit(w[i + 1], w[i], sh);
+}
+
+// Codes 4 kk .. 4 kk + 3 of a stream as bytes.
+__device__ __forceinline__ uint32_t stream_codes(const uint32_t (&s)[4], int kk, int bits) {
+  uint32_t x4 = (s[kk >> 1] >> (16 * (kk & 1))) & 0xffffu;
+  x4 = (x4 | (x4 << 8)) & 0x00ff00ffu;
+  x4 = (x4 | (x4 << 4)) & 0x0f0f0f0fu;
+  uint32_t x2 = (s[0] >> (8 * kk)) & 0xffu;
+  x2 = (x2 | (x2 << 12)) & 0x000f000fu;
+  x2 = (x2 | (x2 << 6)) & 0x03030303u;
+  return bits == 8 ? s[kk] : bits == 4 ? x4 : x2;
+}
+
 // QK over one compressed page: s[mt][i] = score(token score_token(mt, i, l4,
 // KIND == kKindDefaultHR), head l16).
 template <int KIND>
 __device__ __forceinline__ void qk_regs(const AttnArgs& a, const Lut& lut, const KRegs<KIND>& k,
-                                        const half8v* qb, int l16, int l4, float4v* s) {
+                                        const half8v* qb, int l16, int l4, float4v* s, void* wave_lds) {
   if constexpr (KIND == kKindDefaultHR) {
     // Load g: 8 pairs of one token half (A operand row l16 = (8g + l16/2,
     // half l16&1)); k-step kk takes its pairs 4kk .. 4kk+3, code bytes 2kk
@@ -705,7 +788,7 @@ __device__ __forceinline__ void qk_regs(const AttnArgs& a, const Lut& lut, const
           const int rc = (int)(int8_t)((rw[kk] >> (8 * i)) & 0xffu);
           const uint32_t code = (cw[kk] >> (8 * i)) & 0xffu;
           const f16 r = (f16)__builtin_amdgcn_exp2f((float)rc * ls2);
-          const half2v cs = __builtin_bit_cast(half2v, lut.deep[code]);
+          const half2v cs = __builtin_bit_cast(half2v, lut.code[kLutDeep + code]);
           e[i] = pack_h2(half2v{r, r} * cs);
         }
         acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(as_half8(e[0], e[1], e[2], e[3]), qb[kk], acc, 0, 0, 0);
@@ -713,31 +796,58 @@ __device__ __forceinline__ void qk_regs(const AttnArgs& a, const Lut& lut, const
       s[mt] = acc;
     }
   } else {
-    const int64_t row0 = k.slot * kPageTokens;
-    const float ls = a.radii_scales ? h2f(a.radii_scales[k.slot]) : 1.0f;
+    uint4* chunks = static_cast<uint4*>(wave_lds);
+    const uint32_t* words = static_cast<const uint32_t*>(wave_lds);
+    wave_lds_sync();  // the previous page's streams are read
+#pragma unroll
+    for (int j = 0; j < kAnyChunks; ++j) chunks[64 * j + 16 * l4 + l16] = k.c[j];
+    wave_lds_sync();
+    // The lane's stream: the row that its run starts in.
+    const int p0 = 16 * l4;
+    const bool in_l1 = p0 < a.split_half;
+    const int bits = in_l1 ? a.l1_bits : a.deep_bits;
+    const int row = 8 * (in_l1 ? a.l1_row : a.deep_row);
+    const int deep0 = 8 * kPageTokens * a.l1_row;  // first deep bit of the page
+    const int start = in_l1 ? p0 * bits : deep0 + (p0 - a.split_half) * bits;
+    const int table = in_l1 ? 0 : kLutDeep;
+    const bool holds_split = (a.split_half & 15) != 0;  // some lane's run does
+    const int n_l1 = min(max(a.split_half - p0, 0), 16);
+    float ls2 = 0.0f;
+    if constexpr (KIND == kKindAnyI8) ls2 = h2f((uint16_t)k.ls_bits) * 1.44269504088896341f;
+#pragma unroll
     for (int mt = 0; mt < 4; ++mt) {
-      const int64_t row = row0 + 16 * mt + l16;
-      const uint8_t* l1row = a.angle_l1 + row * a.l1_row;
-      const uint8_t* deeprow = a.angle_deep + row * a.deep_row;
+      const int t = 16 * mt + l16;
+      uint32_t st[4], sd[4] = {0u, 0u, 0u, 0u};
+      code_stream(words, start + t * row, st);
+      if (holds_split) code_stream(words, deep0 + (p0 - a.split_half) * a.deep_bits + 8 * t * a.deep_row, sd);
       float4v acc = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
       for (int kk = 0; kk < 4; ++kk) {
+        uint32_t codes = stream_codes(st, kk, bits);
+        int tab[4] = {table, table, table, table};
+        if (holds_split) {
+          const int n = min(max(n_l1 - 4 * kk, 0), 4);  // of these four pairs, the level-1 ones
+          const uint32_t mask = n == 4 ? 0xffffffffu : (1u << (8 * n)) - 1u;
+          codes = (codes & mask) | (stream_codes(sd, kk, a.deep_bits) & ~mask);
+#pragma unroll
+          for (int i = 0; i < 4; ++i) tab[i] = i < n ? 0 : kLutDeep;
+        }
         uint32_t e[4];
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
-          const int p = 16 * l4 + 4 * kk + i;
-          f16 r;
-          if (a.radii_scales) {
-            const int rc = static_cast<const int8_t*>(a.radii)[row * kPairs + p];
-            r = (f16)expf((float)rc * ls);
+          half2v r;
+          if constexpr (KIND == kKindAnyI8) {
+            const uint4 q = k.r[mt];
+            const uint32_t w = kk == 0 ? q.x : kk == 1 ? q.y : kk == 2 ? q.z : q.w;
+            const f16 x = (f16)__builtin_amdgcn_exp2f((float)(int8_t)((w >> (8 * i)) & 0xffu) * ls2);
+            r = half2v{x, x};
           } else {
-            r = __builtin_bit_cast(f16, static_cast<const uint16_t*>(a.radii)[row * kPairs + p]);
+            const uint4 q = k.r[mt][kk >> 1];
+            const uint32_t w = (kk & 1) ? ((i & 2) ? q.w : q.z) : ((i & 2) ? q.y : q.x);
+            r = (i & 1) ? hi_hi(w) : lo_lo(w);
           }
-          uint32_t csw;
-          if (p < a.split_half)
-            csw = lut.l1[packed_code(l1row, p, a.l1_bits)];
-          else
-            csw = lut.deep[packed_code(deeprow, p - a.split_half, a.deep_bits)];
-          e[i] = pack_h2(half2v{r, r} * __builtin_bit_cast(half2v, csw));
+          const uint32_t cs = lut.code[tab[i] + (int)((codes >> (8 * i)) & 0xffu)];
+          e[i] = pack_h2(r * __builtin_bit_cast(half2v, cs));
         }
         acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(as_half8(e[0], e[1], e[2], e[3]), qb[kk], acc, 0, 0, 0);
       }
@@ -1664,16 +1774,10 @@ __global__ __launch_bounds__(WAVES * 64) void decode_attention_kernel(AttnArgs a
   KRegs<KIND> kr;
   // V: the page store's codes, or the dense V planes' rows (DV).
   typename std::conditional<DV, DenseVRegs, VRegs>::type vr;
-  if constexpr (KIND == kKindGeneric) {  // also the launch for a call without pages
-    if (page < p_end) {
-      load_k<KIND>(a, bkv * a.capacity + page, l16, l4, kr);
-      if constexpr (DV)
-        load_v<HR>(a, bkv * a.v_capacity + page, l16, l4, lane, vr);
-      else
-        load_v<HR>(a, bkv * a.capacity + page, l16, l4, lane, vr);
-    }
-  } else {
-    // The specialised layouts always have pages (p_begin < n_pages).  A wave
+  void* wave_lds = &sh.acc[wave][0];  // this wave's merge area, free until finish_unit
+  static_assert(sizeof(sh.acc[0]) >= kAnyCodeBytes, "a page's code rows fit the merge area");
+  if constexpr (KIND != kKindNone) {
+    // A launch with pages has one in every split (p_begin < n_pages).  A wave
     // without a page of its own issues the same loads with every lane on the
     // first bytes of the split's first page (one cache line per load) instead
     // of branching around them: a load under a branch would make the
@@ -1688,7 +1792,9 @@ __global__ __launch_bounds__(WAVES * 64) void decode_attention_kernel(AttnArgs a
       load_v<HR>(a, bkv * a.capacity + p_load, lane_e & 15, lane_e >> 4, lane_e, vr);
   }
   TP_STAMP(1);
-  if (tid < 256) build_lut<KIND>(sh.lut, a, tid);
+  if constexpr (KIND != kKindNone) {
+    if (tid < 256) build_lut<KIND>(sh.lut, a, tid);
+  }
   TP_STAMP(3);
   __shared__ float qjl_sin[QJL != kQjlOff ? kQjlMaxBits + 1 : 1];
   __shared__ uint32_t qjl_qw[QJL == kQjlAny ? 16 * kQjlMaxWords : 1];
@@ -1699,7 +1805,7 @@ __global__ __launch_bounds__(WAVES * 64) void decode_attention_kernel(AttnArgs a
     qjl_query<HR, QJL>(a, b, kv, h0, nh, l16, qb, qsig, qnorm);
     if constexpr (QJL == kQjlAny) qjl_query_words(a, b, kv, h0, nh, tid, qjl_qw);
   }
-  lds_barrier();
+  if constexpr (KIND != kKindNone) lds_barrier();
   TP_STAMP(2);
 
   const int sbase4 = 4 * (2 * v_token(0, l4, 0, HR) + (l16 >> 3));
@@ -1716,48 +1822,50 @@ __global__ __launch_bounds__(WAVES * 64) void decode_attention_kernel(AttnArgs a
   // unconditional and every wait covers only the loads it needs: QK waits for
   // the page's K codes while its V codes may still be in flight.  A page with
   // a successor is fully valid (only the last live page can be partial).
-  for (int it = 0; page + WAVES < p_end; page += WAVES, ++it) {
-    float4v s[4];
-    qk_regs<KIND>(a, sh.lut, kr, qb, l16, l4, s);
-    if constexpr (QJL == kQjl64) qjl_correct<HR>(a, bkv * a.qjl_capacity + page, l4, qsig, qnorm, qjl_sin, s);
-    if constexpr (QJL == kQjlAny)
-      qjl_correct_any<HR>(a, bkv * a.qjl_capacity + page, l4, qjl_qw, HR ? (l16 & 7) : l16, qnorm, qjl_sin, s);
-    if (it < 12) TP_STAMP(4 + 4 * it);
-    load_k<KIND>(a, bkv * a.capacity + page + WAVES, l16, l4, kr);
-    half8v pb[2];
-    softmax_page<HR>(s, kPageTokens, a.scale_log2, l4, m_run, l_run, acc, pb);
-    pv_regs<HR>(vr, sbase4, ssel, pb, acc);
-    if constexpr (DV)
-      load_v<HR>(a, bkv * a.v_capacity + page + WAVES, l16, l4, lane, vr);
-    else
-      load_v<HR>(a, bkv * a.capacity + page + WAVES, l16, l4, lane, vr);
-    if (it < 12) TP_STAMP(5 + 4 * it);
-  }
-  if (page < p_end) {
-    float4v s[4];
-    qk_regs<KIND>(a, sh.lut, kr, qb, l16, l4, s);
-    if constexpr (QJL == kQjl64) qjl_correct<HR>(a, bkv * a.qjl_capacity + page, l4, qsig, qnorm, qjl_sin, s);
-    if constexpr (QJL == kQjlAny)
-      qjl_correct_any<HR>(a, bkv * a.qjl_capacity + page, l4, qjl_qw, HR ? (l16 & 7) : l16, qnorm, qjl_sin, s);
-    const int valid = (int)min((int64_t)kPageTokens, a.seq_len - (int64_t)page * kPageTokens);
-    half8v pb[2];
-    softmax_page<HR>(s, valid, a.scale_log2, l4, m_run, l_run, acc, pb);
-    if constexpr (DV) {
-      // Dense V rows of masked tokens get P = 0, but 0 * NaN is NaN in the
-      // MFMA: rows at or past `valid` are zeroed, so whatever a caller's
-      // buffer holds there adds nothing (the reference skips those tokens in
-      // its V sum, tqpolar_online_attention.metal:10-196).
-      if (valid < kPageTokens) {
+  if constexpr (KIND != kKindNone) {
+    for (int it = 0; page + WAVES < p_end; page += WAVES, ++it) {
+      float4v s[4];
+      qk_regs<KIND>(a, sh.lut, kr, qb, l16, l4, s, wave_lds);
+      if constexpr (QJL == kQjl64) qjl_correct<HR>(a, bkv * a.qjl_capacity + page, l4, qsig, qnorm, qjl_sin, s);
+      if constexpr (QJL == kQjlAny)
+        qjl_correct_any<HR>(a, bkv * a.qjl_capacity + page, l4, qjl_qw, HR ? (l16 & 7) : l16, qnorm, qjl_sin, s);
+      if (it < 12) TP_STAMP(4 + 4 * it);
+      load_k<KIND>(a, bkv * a.capacity + page + WAVES, l16, l4, kr);
+      half8v pb[2];
+      softmax_page<HR>(s, kPageTokens, a.scale_log2, l4, m_run, l_run, acc, pb);
+      pv_regs<HR>(vr, sbase4, ssel, pb, acc);
+      if constexpr (DV)
+        load_v<HR>(a, bkv * a.v_capacity + page + WAVES, l16, l4, lane, vr);
+      else
+        load_v<HR>(a, bkv * a.capacity + page + WAVES, l16, l4, lane, vr);
+      if (it < 12) TP_STAMP(5 + 4 * it);
+    }
+    if (page < p_end) {
+      float4v s[4];
+      qk_regs<KIND>(a, sh.lut, kr, qb, l16, l4, s, wave_lds);
+      if constexpr (QJL == kQjl64) qjl_correct<HR>(a, bkv * a.qjl_capacity + page, l4, qsig, qnorm, qjl_sin, s);
+      if constexpr (QJL == kQjlAny)
+        qjl_correct_any<HR>(a, bkv * a.qjl_capacity + page, l4, qjl_qw, HR ? (l16 & 7) : l16, qnorm, qjl_sin, s);
+      const int valid = (int)min((int64_t)kPageTokens, a.seq_len - (int64_t)page * kPageTokens);
+      half8v pb[2];
+      softmax_page<HR>(s, valid, a.scale_log2, l4, m_run, l_run, acc, pb);
+      if constexpr (DV) {
+        // Dense V rows of masked tokens get P = 0, but 0 * NaN is NaN in the
+        // MFMA: rows at or past `valid` are zeroed, so whatever a caller's
+        // buffer holds there adds nothing (the reference skips those tokens in
+        // its V sum, tqpolar_online_attention.metal:10-196).
+        if (valid < kPageTokens) {
 #pragma unroll
-        for (int ks = 0; ks < 2; ++ks) {
+          for (int ks = 0; ks < 2; ++ks) {
 #pragma unroll
-          for (int e = 0; e < 8; ++e) {
-            if (v_token(ks, l4, e, HR) >= valid) vr.w[8 * ks + e] = u32x4{0u, 0u, 0u, 0u};
+            for (int e = 0; e < 8; ++e) {
+              if (v_token(ks, l4, e, HR) >= valid) vr.w[8 * ks + e] = u32x4{0u, 0u, 0u, 0u};
+            }
           }
         }
       }
+      pv_regs<HR>(vr, sbase4, ssel, pb, acc);
     }
-    pv_regs<HR>(vr, sbase4, ssel, pb, acc);
   }
 
   // The dense tail follows the last page; the last split's least loaded wave
@@ -1803,6 +1911,7 @@ __global__ __launch_bounds__(kQkWaves * 64) void fused_qk_kernel(AttnArgs a) {
   __shared__ float qjl_sin[QJL != kQjlOff ? kQjlMaxBits + 1 : 1];
   __shared__ uint32_t qjl_qw[QJL == kQjlAny ? 16 * kQjlMaxWords : 1];
   __shared__ uint4 stage[kQkWaves][16 * kQkRow / 8];
+  __shared__ uint4 code_rows[any_kind(KIND) ? kQkWaves : 1][any_kind(KIND) ? kAnyCodeBytes / 16 : 1];
   const int tid = threadIdx.x;
   const int lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);  // wave-uniform: scalar branches
@@ -1832,7 +1941,7 @@ __global__ __launch_bounds__(kQkWaves * 64) void fused_qk_kernel(AttnArgs a) {
   __syncthreads();
   if (page >= a.n_pages) return;
   float4v s[4];
-  qk_regs<KIND>(a, lut, kr, qb, l16, l4, s);
+  qk_regs<KIND>(a, lut, kr, qb, l16, l4, s, &code_rows[any_kind(KIND) ? wave : 0][0]);
   if constexpr (QJL == kQjl64) qjl_correct<false>(a, bkv * a.qjl_capacity + page, l4, qsig, qnorm, qjl_sin, s);
   if constexpr (QJL == kQjlAny) qjl_correct_any<false>(a, bkv * a.qjl_capacity + page, l4, qjl_qw, l16, qnorm, qjl_sin, s);
   uint16_t* st = reinterpret_cast<uint16_t*>(&stage[wave][0]);
@@ -1862,7 +1971,7 @@ __global__ __launch_bounds__(kQkWaves * 64) void fused_qk_kernel(AttnArgs a) {
 static int layout_kind(const tp_page_layout* L) {
   if (!L->int8_radii && L->l1_bits == 4 && L->deep_bits == 4 && L->split_dim == 64) return kKindDefault;
   if (L->int8_radii && L->deep_bits == 8 && L->split_dim == 0) return kKindFast;
-  return kKindGeneric;
+  return L->int8_radii ? kKindAnyI8 : kKindAnyF16;
 }
 
 constexpr int kDecodeWaves = 8;  // wave64s per decode workgroup
@@ -1968,7 +2077,8 @@ static void launch_fused_qk(const AttnArgs& a, int kind, dim3 grid, hipStream_t 
   switch (kind) {
     case kKindDefault: hipLaunchKernelGGL((fused_qk_kernel<kKindDefault, QJL>), grid, dim3(kQkWaves * 64), 0, s, a); break;
     case kKindFast: hipLaunchKernelGGL((fused_qk_kernel<kKindFast, QJL>), grid, dim3(kQkWaves * 64), 0, s, a); break;
-    default: hipLaunchKernelGGL((fused_qk_kernel<kKindGeneric, QJL>), grid, dim3(kQkWaves * 64), 0, s, a); break;
+    case kKindAnyI8: hipLaunchKernelGGL((fused_qk_kernel<kKindAnyI8, QJL>), grid, dim3(kQkWaves * 64), 0, s, a); break;
+    default: hipLaunchKernelGGL((fused_qk_kernel<kKindAnyF16, QJL>), grid, dim3(kQkWaves * 64), 0, s, a); break;
   }
 }
 
@@ -2149,8 +2259,18 @@ static void launch_decode_kind(const AttnArgs& a, int kind, dim3 grid, hipStream
     case kKindDefaultHR: launch_decode<kKindDefaultHR, QJL>(a, grid, s); break;
     case kKindDefault: launch_decode<kKindDefault, QJL>(a, grid, s); break;
     case kKindFast: launch_decode<kKindFast, QJL>(a, grid, s); break;
-    default: launch_decode<kKindGeneric, QJL>(a, grid, s); break;
+    case kKindAnyI8: launch_decode<kKindAnyI8, QJL>(a, grid, s); break;
+    default: launch_decode<kKindAnyF16, QJL>(a, grid, s); break;
   }
+}
+
+// A call without pages: one split over the dense tail, no table, no page loads
+// and no sketches (the tail takes no correction).
+static void launch_decode_tail(const AttnArgs& a, dim3 grid, hipStream_t s) {
+  if (a.g <= 8)
+    hipLaunchKernelGGL((decode_attention_kernel<kKindNone, 4>), grid, dim3(256), 0, s, a);
+  else
+    hipLaunchKernelGGL((decode_attention_kernel<kKindNone, kDecodeWaves>), grid, dim3(kDecodeWaves * 64), 0, s, a);
 }
 
 // Dense V (the reference's dense_v_debug storage) takes the same workgroup
@@ -2177,11 +2297,17 @@ static void launch_decode_dense_v(const AttnArgs& a, int kind, dim3 grid, hipStr
       else
         launch_decode_w<kKindFast, kDecodeWaves, QJL, true>(a, grid, s);
       break;
+    case kKindAnyI8:
+      if (w4)
+        launch_decode_w<kKindAnyI8, 4, QJL, true>(a, grid, s);
+      else
+        launch_decode_w<kKindAnyI8, kDecodeWaves, QJL, true>(a, grid, s);
+      break;
     default:
       if (w4)
-        launch_decode_w<kKindGeneric, 4, QJL, true>(a, grid, s);
+        launch_decode_w<kKindAnyF16, 4, QJL, true>(a, grid, s);
       else
-        launch_decode_w<kKindGeneric, kDecodeWaves, QJL, true>(a, grid, s);
+        launch_decode_w<kKindAnyF16, kDecodeWaves, QJL, true>(a, grid, s);
       break;
   }
 }
@@ -2291,8 +2417,12 @@ static int32_t decode_attention_impl(const void* q, int64_t batch, int32_t hq, i
       launch_decode_dense_v<kQjlAny>(a, kind, grid, s);
     return launch_status("tp_decode_attention_dense_v");
   }
+  if (n_pages == 0) {
+    launch_decode_tail(a, grid, s);
+    return launch_status(use_qjl ? "tp_decode_attention_qjl" : "tp_decode_attention");
+  }
   if (use_qjl) {
-    const int kind = n_pages > 0 ? decode_kind(layout_kind(layout), a) : (int)kKindGeneric;
+    const int kind = decode_kind(layout_kind(layout), a);
     if (a.qjl_bits == kQjlBits)
       launch_decode_kind<kQjl64>(a, kind, grid, s);
     else
@@ -2304,10 +2434,10 @@ static int32_t decode_attention_impl(const void* q, int64_t batch, int32_t hq, i
     // The measurement variants combine in one tier (any split count).
     a.tier_splits = 0;
     a.tier_groups = 0;
-    return launch_measure_variant(a, grid, n_pages > 0 ? layout_kind(layout) : -1, s);
+    return launch_measure_variant(a, grid, layout_kind(layout), s);
   }
 #endif
-  launch_decode_kind<kQjlOff>(a, n_pages > 0 ? decode_kind(layout_kind(layout), a) : (int)kKindGeneric, grid, s);
+  launch_decode_kind<kQjlOff>(a, decode_kind(layout_kind(layout), a), grid, s);
   return launch_status("tp_decode_attention");
 }
 
@@ -2426,6 +2556,37 @@ extern "C" unsigned long long tp_selftest_decode_bounds(const tp_bounds_case* c,
   const int64_t sz_nrm = BH * c->qjl_capacity * kPageTokens * 2;
   const int64_t sz_qs = c->batch * c->hq * qjl_nb;
 
+  // The key loads of any layout but the default and the fast one.
+  auto any_loads = [&](int lin, int wave, int lane, int64_t slot, int lane_e) {
+    const int l16 = lane_e & 15, l4 = lane_e >> 4;
+    for (int mt = 0; mt < 4; ++mt) {
+      const int t = 16 * mt + l16;
+      if (int8r)
+        log.check("radii", fast_base(slot, l4) + fast_row(t), 16, sz_radii, lin, wave, lane);
+      else
+        log.check("radii", k_radii_base(slot, l4) + k_radii_row(t), 32, sz_radii, lin, wave, lane);
+    }
+    for (int j = 0; j < kAnyChunks; ++j) {
+      const int ch = any_chunk(lane_e, j, l1_row, deep_row);
+      const bool from_l1 = any_chunk_from_l1(ch, l1_row);
+      log.check(from_l1 ? "angle_l1" : "angle_deep", any_chunk_off(slot, ch, l1_row, deep_row), 16,
+                from_l1 ? sz_l1 : sz_deep, lin, wave, lane);
+    }
+    if (int8r) log.check("radii_scales", fast_scale(slot), 2, sz_rs, lin, wave, lane);
+    // The lane's code streams stay in the wave's LDS area: five dwords from the
+    // bit where its run starts, for the first and last token.
+    const int split_half = c->layout.split_dim / 2, p0 = 16 * l4;
+    const int deep0 = 8 * kPageTokens * l1_row;
+    for (int t = 0; t < kPageTokens; t += kPageTokens - 1) {
+      const bool in_l1 = p0 < split_half;
+      const int bit = in_l1 ? p0 * c->layout.l1_bits + 8 * t * l1_row
+                            : deep0 + (p0 - split_half) * c->layout.deep_bits + 8 * t * deep_row;
+      log.check("code rows in LDS", (bit >> 5) * 4, 20, kAnyCodeBytes, lin, wave, lane);
+      if (split_half & 15)
+        log.check("code rows in LDS", ((deep0 + (p0 - split_half) * c->layout.deep_bits + 8 * t * deep_row) >> 5) * 4, 20,
+                  kAnyCodeBytes, lin, wave, lane);
+    }
+  };
   // One lane's loads of page `page` (lane addresses of lane_e), as the kernels issue them.
   auto page_loads = [&](int lin, int wave, int lane, int64_t bkv, int page, int lane_e) {
     const int64_t slot = bkv * cap + page;
@@ -2450,6 +2611,8 @@ extern "C" unsigned long long tp_selftest_decode_bounds(const tp_bounds_case* c,
         log.check("angle_deep", fast_base(slot, l4) + fast_row(t), 16, sz_deep, lin, wave, lane);
       }
       log.check("radii_scales", fast_scale(slot), 2, sz_rs, lin, wave, lane);
+    } else {
+      any_loads(lin, wave, lane, slot, lane_e);
     }
     if (c->dense_v) {
       for (int ks = 0; ks < 2; ++ks)
@@ -2465,27 +2628,6 @@ extern "C" unsigned long long tp_selftest_decode_bounds(const tp_bounds_case* c,
       log.check("v_scales", sb + 4 * (lane_e + 64) + (c->mutate == 1 ? 512 : 0), 4, sz_vs, lin, wave, lane);
     }
   };
-  // The generic layout's codes, gathered during the math of a page it owns.
-  auto generic_loads = [&](int lin, int wave, int lane, int64_t bkv, int page) {
-    const int64_t slot = bkv * cap + page;
-    const int l16 = lane & 15, l4 = lane >> 4;
-    const int split_half = c->layout.split_dim / 2;
-    if (int8r) log.check("radii_scales", slot * 2, 2, sz_rs, lin, wave, lane);
-    for (int mt = 0; mt < 4; ++mt) {
-      const int64_t row = slot * kPageTokens + 16 * mt + l16;
-      for (int kk = 0; kk < 4; ++kk)
-        for (int i = 0; i < 4; ++i) {
-          const int p = 16 * l4 + 4 * kk + i;
-          log.check("radii", (row * kPairs + p) * (int8r ? 1 : 2), int8r ? 1 : 2, sz_radii, lin, wave, lane);
-          if (p < split_half)
-            log.check("angle_l1", row * l1_row + (p * c->layout.l1_bits) / 8, 1, sz_l1, lin, wave, lane);
-          else
-            log.check("angle_deep", row * deep_row + ((p - split_half) * c->layout.deep_bits) / 8, 1, sz_deep, lin, wave,
-                      lane);
-        }
-    }
-  };
-
   if (c->kernel == 1) {  // fused_qk_kernel: one page per wave, the last page reloaded past n_pages
     const int gx = (n_pages + kQkWaves - 1) / kQkWaves;
     for (int64_t bkv = 0; bkv < BH; ++bkv)
@@ -2498,11 +2640,12 @@ extern "C" unsigned long long tp_selftest_decode_bounds(const tp_bounds_case* c,
               const int lin = (int)((bkv * head_blocks + hb) * gx + bx);
               log.check("q (buffer range)", ((int64_t)b * c->hq + (int64_t)kv * g + h0) * kHeadDim * 2,
                         (int64_t)nh * kHeadDim * 2, sz_q, lin, wave, lane);
-              if (kind != kKindGeneric) {
+              {
                 const int64_t slot_page = std::min(page, n_pages - 1);
                 const int l16 = lane & 15, l4 = lane >> 4;
                 const int64_t slot = bkv * cap + slot_page;
-                for (int mt = 0; mt < 4; ++mt) {
+                if (any_kind(kind)) any_loads(lin, wave, lane, slot, lane);
+                for (int mt = 0; mt < 4 && !any_kind(kind); ++mt) {
                   const int t = 16 * mt + l16;
                   if (kind == kKindDefault) {
                     log.check("radii", k_radii_base(slot, l4) + k_radii_row(t), 32, sz_radii, lin, wave, lane);
@@ -2513,8 +2656,6 @@ extern "C" unsigned long long tp_selftest_decode_bounds(const tp_bounds_case* c,
                     log.check("angle_deep", fast_base(slot, l4) + fast_row(t), 16, sz_deep, lin, wave, lane);
                   }
                 }
-              } else if (page < n_pages) {
-                generic_loads(lin, wave, lane, bkv, page);
               }
               if (page < n_pages) {
                 const int64_t sz_scores = c->batch * c->hq * (int64_t)n_pages * kPageTokens * 2;
@@ -2583,12 +2724,7 @@ extern "C" unsigned long long tp_selftest_decode_bounds(const tp_bounds_case* c,
           log.check("q (buffer range)", ((int64_t)b * c->hq + (int64_t)kv * g + h0) * kHeadDim * 2,
                     (int64_t)nh * kHeadDim * 2, sz_q, L, wave, lane);
           int page = p_begin + wave;
-          if (kind == kKindGeneric) {
-            for (; page < p_end; page += waves) {
-              generic_loads(L, wave, lane, bkv, page);
-              page_loads(L, wave, lane, bkv, page, lane);
-            }
-          } else {
+          {
             int p_load, lane_e;
             first_page_load(page, p_begin, p_end, lane, p_load, lane_e);
             if (c->mutate == 2 && page >= p_end) p_load = p_begin + pps;  // the no-page load moved one split on
