@@ -155,6 +155,52 @@ def test_encode_inf_inputs(device, layout_name, dtype):
     check_against_oracle(k.astype(dtype), v.astype(dtype), LAYOUTS[layout_name], device)
 
 
+@pytest.mark.parametrize("layout_name", sorted(LAYOUTS))
+@pytest.mark.parametrize("dtype", [np.float16, np.float32])
+@pytest.mark.parametrize("H,T", [(8, 64 * 32), (8, 64 * 33), (8, 64 * 64), (8, 64 * 64 + 17), (3, 64 * 260 + 63)])
+def test_encode_instances_agree(device, layout_name, dtype, H, T):
+    """Launches on both sides of the pairs-per-thread lines (256 and 512 pages),
+    of whole and partial last pages, against the same pages encoded one at a time
+    (the instance the oracle tests above run on), with zeros, infinities and NaN."""
+    print(f"[encode-np] {layout_name} {np.dtype(dtype).name} H={H} T={T}", flush=True)
+    k, v = gen_kv(T, 1, H, T, "loguniform", dtype)
+    rng = np.random.default_rng(T)
+    for x in (k, v):
+        flat = x.reshape(-1)
+        for value in (0.0, -0.0, np.inf, -np.inf, np.nan, 3e4, 1e-7):
+            flat[rng.integers(0, flat.size, 40)] = value
+    whole = encode_gpu(k, v, LAYOUTS[layout_name], device)
+    parts = [encode_gpu(np.ascontiguousarray(k[:, :, t:t + 640]), np.ascontiguousarray(v[:, :, t:t + 640]),
+                        LAYOUTS[layout_name], device) for t in range(0, T, 640)]
+    for name, got in whole.items():
+        if got is not None:
+            assert_bits_equal(got, np.concatenate([p[name] for p in parts], axis=2), name)
+
+
+@pytest.mark.parametrize("bits", [2, 4, 8])
+def test_f32_angle_codes_at_the_boundaries(device, bits):
+    """fp32 pairs within a few ulps of every code boundary, of the wrap at a turn
+    of 1 - 1e-6 and of the axes, over radii from fp32's subnormals to its largest
+    values: codes, radii and the values beside them are the oracle's."""
+    print(f"[encode-f32] bits={bits}", flush=True)
+    rng = np.random.default_rng(bits)
+    lv = 2 ** bits - 1
+    edges = np.concatenate([(np.arange(lv) + 0.5) / lv, [1 - 1e-6, 0.0, 0.25, 0.5, 0.75, 1.0]])
+    n = 16 * PAGE * 64
+    turn = rng.choice(edges, n) + rng.integers(-12, 13, n) * 2.0 ** -25
+    r = np.where(rng.random(n) < 0.5, 1.0 + rng.random(n), 2.0 ** rng.uniform(-150, 126, n))
+    theta = turn * 2 * np.pi - np.pi
+    k = np.stack([r * np.cos(theta), r * np.sin(theta)], -1).astype(np.float32).reshape(1, 1, 16 * PAGE, 128)
+    # Values at and beside the half-way points of their codes.
+    s = np.float32(np.float16(0.37))
+    v = ((rng.integers(-127, 128, k.size) + 0.5) * s).astype(np.float32).reshape(k.shape)
+    v.reshape(-1, 32)[:, 0] = 127 * s
+    v = np.nextafter(v, rng.choice([-np.inf, np.inf, 0.0], v.shape).astype(np.float32)).astype(np.float32)
+    layout = (False, 4, bits, 0) if bits != 8 else (False, 8, 8, 64)
+    with np.errstate(over="ignore"):
+        check_against_oracle(k, v, layout, device)
+
+
 def test_encode_into_capacity_slot(device):
     """Pages land in slots [page_begin, page_begin + S) of a larger store."""
     k, v = gen_kv(8, 2, 2, 2 * PAGE, "normal", np.float16)

@@ -200,20 +200,6 @@ __device__ __forceinline__ float div_f16(float v, float s, float rs) {
   return h2f(f2h(q));
 }
 
-// encoder.py:33 for fp16 inputs: f16(sqrt(f16(f16(x*x) + f16(y*y)))).
-__device__ __forceinline__ uint16_t radius_f16_in(float x, float y) {
-  const float xx = h2f(f2h(x * x));
-  const float yy = h2f(f2h(y * y));
-  return sqrt_f16(h2f(f2h(xx + yy)));
-}
-
-// encoder.py:33 for fp32 inputs: f16(sqrt(x*x + y*y)) with fp32 ops.
-__device__ __forceinline__ uint16_t radius_f32_in(float x, float y) {
-  const float xx = x * x;
-  const float yy = y * y;
-  return f2h(sqrtf(xx + yy));
-}
-
 // encoder.py:47-55 for an fp16 angle: fp16 shift and divide, clip, then the
 // float32 product with (2^bits - 1) rounded half-even.
 __device__ __forceinline__ uint32_t angle_code_f16(uint16_t a16, int bits) {
