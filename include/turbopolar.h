@@ -160,6 +160,27 @@ int32_t tp_decode_attention(const void* q, int64_t batch, int32_t hq, int32_t hk
                             size_t workspace_bytes, void* out, void* stream);
 
 /*
+ * A decode step on a cache whose new token does not complete a page, in one
+ * launch: TurboPolarFastCache.decode_attention of the reference
+ * (turbopolar_fast_attention.py:106-188), which appends the token and then
+ * attends.  new_k, new_v: fp16 [batch][hkv][128], the token's rows, 16-byte
+ * aligned; tail_k, tail_v hold the tail_len (0..62) tokens before it and get
+ * its rows at row tail_len.  Attends every stored token and the new one.  check 2:
+ * the call returns once the launch has reported whether every value of new_k and
+ * new_v is finite, TP_ERR_NONFINITE if not (`out` and the tail's row tail_len
+ * then hold no result; the tokens before it are as they were); check 3 (deferred)
+ * returns after the launch, which writes epoch + 1 to flag on a non-finite value.
+ * flag and epoch as for tp_append_stage with check 2 and 3, everything else as for
+ * tp_decode_attention (at most 65534 splits).
+ */
+int32_t tp_decode_step(const void* q, int64_t batch, int32_t hq, int32_t hkv,
+                       const tp_page_layout* layout, const tp_pages* pages, int32_t n_pages,
+                       const void* new_k, const void* new_v, void* tail_k, void* tail_v,
+                       int32_t tail_len, int64_t tail_stride, float scale, int32_t pages_per_split,
+                       void* workspace, size_t workspace_bytes, void* out, int32_t check,
+                       uint32_t* flag, uint32_t epoch, void* stream);
+
+/*
  * tp_decode_attention without a workspace argument: allocates nothing (no
  * hipMalloc, hipFree or allocating library call).  No counterpart in the
  * reference; it is for callers that cannot allocate device memory: code under
@@ -222,6 +243,7 @@ typedef struct tp_bounds_case {
   int32_t kernel;
   int32_t mutate;
   int32_t qjl_bits; /* QJL sketch bits (0 reads as 64) */
+  int32_t step;     /* tp_decode_step: tail_len counts the new token */
 } tp_bounds_case;
 unsigned long long tp_selftest_decode_bounds(const tp_bounds_case* c, char* msg, int32_t msg_len);
 

@@ -26,7 +26,7 @@ LAYOUTS = {"default": (0, 4, 4, 64), "fast": (1, 4, 8, 0), "deep2": (0, 4, 2, 64
 
 
 def run(layout="default", batch=1, hq=32, hkv=8, n_pages=64, capacity=None, tail=0, tail_stride=None, seq=None,
-        pps=0, qjl=False, dense_v=False, kernel=0, mutate=0, qjl_bits=0):
+        pps=0, qjl=False, dense_v=False, kernel=0, mutate=0, qjl_bits=0, step=0):
     c = _lib.TPBoundsCase()
     c.batch, c.hq, c.hkv = batch, hq, hkv
     c.layout = _lib.make_layout(*LAYOUTS[layout])
@@ -39,6 +39,7 @@ def run(layout="default", batch=1, hq=32, hkv=8, n_pages=64, capacity=None, tail
     c.qjl, c.qjl_capacity = int(qjl), n_pages
     c.dense_v, c.v_capacity = int(dense_v), n_pages
     c.kernel, c.mutate, c.qjl_bits = kernel, mutate, qjl_bits
+    c.step = step
     msg = ctypes.create_string_buffer(512)
     bad = _lib.lib().tp_selftest_decode_bounds(ctypes.byref(c), msg, 512)
     return bad, msg.value.decode()
@@ -73,6 +74,9 @@ CASES = [
     *[dict(layout=lay, **kw) for lay in ("odd_split", "deep2_only", "l1_only", "wide", "one_deep", "one_l1")
       for kw in (dict(n_pages=7, pps=4, tail=3, tail_stride=3), dict(n_pages=21, pps=9, hq=24, hkv=2),
                  dict(n_pages=5, kernel=1, batch=2))],
+    dict(n_pages=16, tail=1, tail_stride=1, step=1),   # one-launch step: the token alone in the tail
+    dict(n_pages=9, tail=63, tail_stride=64, step=1, hq=24, hkv=2),
+    dict(n_pages=520, tail=20, tail_stride=64, step=1, batch=2, layout="fast", hq=4, hkv=1),
     dict(n_pages=100, capacity=128, batch=2, hq=16, hkv=4),
     dict(hq=24, hkv=2, n_pages=20, qjl=True),          # GQA 12: the row token order of default pages
     dict(hq=40, hkv=2, n_pages=9, pps=2, dense_v=True),

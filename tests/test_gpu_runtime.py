@@ -12,7 +12,9 @@ import torch
 import oracle
 from common import ATOL, LAYOUTS, PAGE, RTOL_L2, cosine, max_abs, oracle_pages, rel_l2
 from turbopolar_amd import TurboPolarConfig, TurboPolarFastCache, TurboPolarKVCacheRuntime, make_turbo_caches
+from turbopolar_amd import kernels
 from turbopolar_amd.kernels import fp16_scale
+from turbopolar_amd.storage import pages_of
 
 pytestmark = pytest.mark.gpu
 
@@ -444,3 +446,47 @@ def test_append_of_whole_pages(device, dtype, layout_name, before, T):
     assert torch.equal(rt.v_storage.scales[:, :, :n], ref.v_storage.scales[:, :, :n])
     if rt._tail_len:
         assert torch.equal(rt.partial_k, ref.partial_k) and torch.equal(rt.partial_v, ref.partial_v)
+
+
+STEP_LAYOUTS = {"default": (False, 4, 4, 64), "fast": (True, 4, 8, 0), "deep2": (False, 4, 2, 64),
+                "odd_split": (True, 4, 2, 46)}
+
+
+@pytest.mark.parametrize("layout_name", sorted(STEP_LAYOUTS))
+@pytest.mark.parametrize("hq,hkv,start", [(8, 2, 1), (32, 8, 61), (8, 8, 64), (24, 2, 125), (4, 1, 64 * 16 + 5),
+                                          (8, 1, 64 * 270 + 40), (16, 1, 64 * 40), (40, 2, 64 * 33 + 60)])
+def test_decode_step_equals_append_then_attend(device, layout_name, hq, hkv, start):
+    """The one-launch step against an append followed by an attention launch, over
+    a page flush, from tail lengths 0 to 62, without pages, with one split, 16,
+    and two tiers of splits, 4- and 8-wave workgroups and two head blocks: the
+    same outputs, tail and telemetry."""
+    print(f"[step] {layout_name} hq={hq} hkv={hkv} start={start}", flush=True)
+    int8, l1, deep, split = STEP_LAYOUTS[layout_name]
+    cfg = TurboPolarConfig(num_q_heads=hq, num_kv_heads=hkv, use_int8_radii=int8, k_angle_bits_level1=l1,
+                           k_angle_bits_deep=deep, split_dim=split)
+    g = torch.Generator(device=device).manual_seed(start)
+    k, v = (torch.randn((1, hkv, start + 8, 128), generator=g, device=device).half() for _ in range(2))
+    fast, ref = TurboPolarFastCache(cfg), TurboPolarKVCacheRuntime(cfg)
+    for rt in (fast.runtime, ref):
+        rt.append(k[:, :, :start].contiguous(), v[:, :, :start].contiguous())
+    scale = fp16_scale(cfg.attention_scale)
+    for t in range(start, start + 8):
+        q = torch.randn((1, hq, 1, 128), generator=g, device=device).half()
+        kn, vn = k[:, :, t:t + 1], v[:, :, t:t + 1]  # strided views
+        if t == start + 2:  # a refused token changes nothing
+            bad = kn.clone()
+            bad[0, hkv - 1, 0, 127] = float("nan")
+            before = fast.runtime.get_io_telemetry()
+            with pytest.raises(ValueError, match="^append"):
+                fast.decode_attention(q, kn, bad, cfg.attention_scale)
+            assert fast.runtime.get_io_telemetry() == before
+        out = fast.decode_attention(q, kn, vn, cfg.attention_scale)
+        ref.append(kn.contiguous(), vn.contiguous())
+        n = ref.k_storage.block_count
+        want = kernels.decode_attention_store(q[:, :, 0], ref.polar_encoder.layout,
+                                              pages_of(ref.k_storage, ref.v_storage) if n else None, n, hkv,
+                                              *ref._tail_views(), ref.actual_seq_len, scale)
+        assert torch.equal(out, want), (t, float((out.float() - want.float()).abs().max()))
+        assert fast.runtime.get_io_telemetry() == ref.get_io_telemetry()
+        assert ref.partial_k is None and fast.runtime.partial_k is None or torch.equal(fast.runtime.partial_k, ref.partial_k)
+        assert ref.partial_v is None and fast.runtime.partial_v is None or torch.equal(fast.runtime.partial_v, ref.partial_v)

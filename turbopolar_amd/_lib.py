@@ -97,6 +97,7 @@ class TPBoundsCase(ctypes.Structure):
         ("kernel", c_i32),
         ("mutate", c_i32),
         ("qjl_bits", c_i32),
+        ("step", c_i32),
     ]
 
 
@@ -129,6 +130,13 @@ _SIGNATURES = {
         [
             c_vp, c_i64, c_i32, c_i32, _P_LAYOUT, _P_PAGES, c_i32,
             c_vp, c_vp, c_i32, c_i64, c_i64, c_float, c_i32, c_vp, c_size, c_vp, c_vp,
+        ],
+    ),
+    "tp_decode_step": (
+        c_i32,
+        [
+            c_vp, c_i64, c_i32, c_i32, _P_LAYOUT, _P_PAGES, c_i32, c_vp, c_vp,
+            c_vp, c_vp, c_i32, c_i64, c_float, c_i32, c_vp, c_size, c_vp, c_i32, c_vp, ctypes.c_uint32, c_vp,
         ],
     ),
     "tp_decode_attention_noalloc": (

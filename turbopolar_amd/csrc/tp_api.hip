@@ -56,6 +56,28 @@ int32_t launch_status(const char* what) {
   return TP_OK;
 }
 
+int32_t wait_verdict(const uint32_t* flag, uint32_t epoch, hipStream_t s, bool reports, const char* what) {
+  const volatile uint32_t* vf = flag;
+  uint32_t verdict = 0;
+  bool done = false;
+  for (int spin = 0; reports && spin < (1 << 22) && !done; ++spin) {
+    verdict = *vf;
+    done = verdict == epoch || verdict == epoch + 1u;
+  }
+  if (!done) {
+    if (hipStreamSynchronize(s) != hipSuccess) {
+      set_error("%s: synchronising the stream failed", what);
+      return TP_ERR_HIP;
+    }
+    verdict = *vf;
+  }
+  if (verdict == epoch + 1u) {
+    set_error("append() inputs must contain finite values");
+    return TP_ERR_NONFINITE;
+  }
+  return TP_OK;
+}
+
 }  // namespace tp
 
 extern "C" {

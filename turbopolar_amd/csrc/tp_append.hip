@@ -215,31 +215,9 @@ int32_t tp_append_stage(const void* k, const void* v, int32_t in_dtype, int64_t 
     hipLaunchKernelGGL(append_stage_kernel<false>, dim3(blocks), dim3(256), 0, s, a);
   int32_t st = launch_status("tp_append_stage");
   if (st != TP_OK || !check || check == 3) return st;
-  if (check == 2) {  // the kernel writes the pinned host flag directly, no copy
-    volatile uint32_t* vf = reinterpret_cast<volatile uint32_t*>(flag);
-    uint32_t verdict = 0;
-    bool done = false;
-    if (blocks == 1) {
-      // Poll for the workgroup's completion word (bounded; a launch that has
-      // not reported by then is waited for the ordinary way).
-      for (int spin = 0; spin < (1 << 22) && !done; ++spin) {
-        verdict = *vf;
-        done = verdict == epoch || verdict == epoch + 1u;
-      }
-    }
-    if (!done) {
-      if (hipStreamSynchronize(s) != hipSuccess) {
-        set_error("tp_append_stage: synchronising the stream failed");
-        return TP_ERR_HIP;
-      }
-      verdict = *vf;
-    }
-    if (verdict == epoch + 1u) {
-      set_error("append() inputs must contain finite values");
-      return TP_ERR_NONFINITE;
-    }
-    return TP_OK;
-  }
+  // The kernel writes the pinned host flag directly, no copy; one workgroup also
+  // reports a finite input, so the host polls for it.
+  if (check == 2) return wait_verdict(flag, epoch, s, blocks == 1, "tp_append_stage");
   uint32_t verdict = 0;
   if (hipMemcpyAsync(&verdict, flag, sizeof(verdict), hipMemcpyDeviceToHost, s) != hipSuccess ||
       hipStreamSynchronize(s) != hipSuccess) {

@@ -157,6 +157,14 @@ struct AttnArgs {
   // argument offsets.
   const uint16_t* v_dense;
   int64_t v_capacity;
+  // A decode step's own token (tp_decode_step): one row of 128 per (batch, kv
+  // head), the tail's last; checked, copied to the tail and attended in one launch.
+  const uint16_t* new_k;
+  const uint16_t* new_v;
+  int32_t new_rows;  // batch * hkv
+  int32_t check;     // as tp_append_stage: 2 reports the verdict, 3 only a non-finite value
+  uint32_t* flag;
+  uint32_t epoch;
 };
 
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
@@ -948,10 +956,12 @@ struct TailRegs {
   u32x4 v[16];
 };
 
-template <bool HR>
+// STEP: the last row is not in the tail yet (stage_new_rows copies it there in
+// this launch); it comes from new_k / new_v, and the tail's range ends before it.
+template <bool HR, bool STEP>
 __device__ __forceinline__ void load_tail(const AttnArgs& a, int64_t bkv, int l16, int l4, TailRegs& r) {
   const int64_t plane = bkv * a.tail_stride * kHeadDim;
-  const int bytes = a.tail_len * kHeadDim * (int)sizeof(uint16_t);
+  const int bytes = (a.tail_len - (STEP ? 1 : 0)) * kHeadDim * (int)sizeof(uint16_t);
   const __amdgpu_buffer_rsrc_t rk = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(a.tail_k + plane),
                                                                       (short)0, bytes, kRawBufferWord3);
   const __amdgpu_buffer_rsrc_t rv = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(a.tail_v + plane),
@@ -969,6 +979,53 @@ __device__ __forceinline__ void load_tail(const AttnArgs& a, int64_t bkv, int l1
       const int off = (v_token(ks, l4, e, HR) * kHeadDim + 8 * l16) * (int)sizeof(uint16_t);
       r.v[8 * ks + e] = __builtin_amdgcn_raw_buffer_load_b128(rv, off, 0, 0);
     }
+  }
+  if constexpr (STEP) {
+    const uint16_t* nk = a.new_k + bkv * kHeadDim;
+    const int row = a.tail_len - 1;
+    u32x4 w[HR ? 2 : 4];
+#pragma unroll
+    for (int kk = 0; kk < (HR ? 2 : 4); ++kk)
+      w[kk] = *reinterpret_cast<const u32x4*>(nk + (HR ? 64 * (l16 & 1) + 16 * l4 : 32 * l4) + 8 * kk);
+    const u32x4 wv = *reinterpret_cast<const u32x4*>(a.new_v + bkv * kHeadDim + 8 * l16);
+    __builtin_amdgcn_sched_barrier(0);  // every load out before the first selection waits
+#pragma unroll
+    for (int j = 0; j < 16; ++j) {
+      const bool mine = (HR ? 8 * (j >> 1) + (l16 >> 1) : 16 * (j >> 2) + l16) == row;
+      r.k[j] = mine ? w[HR ? j & 1 : j & 3] : r.k[j];
+    }
+#pragma unroll
+    for (int e = 0; e < 16; ++e) r.v[e] = v_token(e >> 3, l4, e & 7, HR) == row ? wv : r.v[e];
+  }
+}
+
+// A step's staging, by the one working workgroup of the launch's first z layer:
+// what append_stage_kernel does for a single token (check every value, copy the
+// rows to the tail, report), so the host has its verdict while the other
+// workgroups attend.  A launch of its own in front held the step up twice: the
+// attention launch waited for the verdict on the host, the next step's staging
+// for the attention on the GPU.
+__device__ __forceinline__ void stage_new_rows(const AttnArgs& a) {
+  if (blockIdx.x != 0 || blockIdx.y != 0) return;
+  constexpr int kChunks = kHeadDim * 2 / 16;
+  auto finite = [](uint32_t w) { return (w & 0x7c00u) != 0x7c00u && (w & 0x7c000000u) != 0x7c000000u; };
+  bool bad = false;
+  for (int c = threadIdx.x; c < a.new_rows * kChunks; c += blockDim.x) {
+    const int64_t row = c / kChunks;
+    const uint4 k = reinterpret_cast<const uint4*>(a.new_k)[c];
+    const uint4 v = reinterpret_cast<const uint4*>(a.new_v)[c];
+    bad = bad || !(finite(k.x) && finite(k.y) && finite(k.z) && finite(k.w) && finite(v.x) && finite(v.y) &&
+                   finite(v.z) && finite(v.w));
+    const int64_t dst = (row * a.tail_stride + a.tail_len - 1) * kChunks + c % kChunks;
+    reinterpret_cast<uint4*>(const_cast<uint16_t*>(a.tail_k))[dst] = k;
+    reinterpret_cast<uint4*>(const_cast<uint16_t*>(a.tail_v))[dst] = v;
+  }
+  if (a.check == 2) {
+    const bool any_bad = __syncthreads_or(bad);
+    if (threadIdx.x == 0)
+      __hip_atomic_store(a.flag, any_bad ? a.epoch + 1u : a.epoch, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+  } else if (bad) {
+    __hip_atomic_store(a.flag, a.epoch + 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
   }
 }
 
@@ -1295,10 +1352,11 @@ struct DecodeSlot {
   int64_t bkv;
 };
 
+template <bool STEP>
 __device__ __forceinline__ DecodeSlot decode_slot(const AttnArgs& a) {
   DecodeSlot d;
   d.kv = (int)blockIdx.x;
-  d.split = (int)blockIdx.z;
+  d.split = (int)blockIdx.z - (STEP ? 1 : 0);  // a step's first z layer is stage_new_rows'
   d.b = (int)fast_div(blockIdx.y, a.div_head_blocks);
   d.hb = (int)blockIdx.y - d.b * a.head_blocks;
   d.bkv = (int64_t)d.b * a.hkv + d.kv;
@@ -1332,6 +1390,7 @@ constexpr int kFlRelease = 1;    // agent-scope release fence before the ticket
 constexpr int kFlNoAcquire = 2;  // no acquire fence in the combining workgroup
 constexpr int kFlTiers = 4;      // two-tier combine (launched only when tier_splits > 0)
 constexpr int kFlBatch16 = 8;    // one-tier combine of exactly 16 splits (4-wave launches)
+constexpr int kFlStep = 16;      // tp_decode_step: the tail's last row is the launch's own token
 
 // One thread draws a ticket of a counter that `count` workgroups increment:
 // relaxed agent-scope add; the workgroup that draws the last ticket issues an
@@ -1739,7 +1798,14 @@ __global__ __launch_bounds__(WAVES * 64) void decode_attention_kernel(AttnArgs a
   // Half-row token order (kKindDefaultHR): the host launches it only for head
   // blocks of at most 8 query heads.
   constexpr bool HR = KIND == kKindDefaultHR;
+  constexpr bool STEP = (FL & kFlStep) != 0;
   __shared__ AttnShared<WAVES> sh;
+  if constexpr (STEP) {
+    if (blockIdx.z == 0) {
+      stage_new_rows(a);
+      return;
+    }
+  }
   TP_STAMP(0);
   // Every argument the prologue reads arrives in one round of scalar loads:
   // left to itself the compiler loaded the page pointers only after waiting
@@ -1755,7 +1821,7 @@ __global__ __launch_bounds__(WAVES * 64) void decode_attention_kernel(AttnArgs a
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);  // wave-uniform: scalar branches
   const int l16 = lane & 15;
   const int l4 = lane >> 4;
-  const DecodeSlot ds = decode_slot(a);
+  const DecodeSlot ds = decode_slot<STEP>(a);
   const int split = ds.split, b = ds.b, kv = ds.kv, hb = ds.hb;
   const int64_t bkv = ds.bkv;
   const int h0 = hb * 16;
@@ -1877,7 +1943,7 @@ __global__ __launch_bounds__(WAVES * 64) void decode_attention_kernel(AttnArgs a
       const int valid = (int)min((int64_t)a.tail_len, a.seq_len - tok0);
       if (valid > 0) {
         TailRegs tr;
-        load_tail<HR>(a, bkv, l16, l4, tr);
+        load_tail<HR, STEP>(a, bkv, l16, l4, tr);
         __builtin_amdgcn_sched_barrier(0);  // all 32 loads out before the first MFMA waits
         float4v s[4];
         qk_tail<HR>(tr, qb, s);
@@ -2210,6 +2276,18 @@ static int32_t launch_measure_variant(const AttnArgs& a, dim3 grid, int kind, hi
 template <int KIND, int W, int QJL, bool DV = false>
 static void launch_decode_w(const AttnArgs& a, dim3 grid, hipStream_t s) {
   const dim3 block(W * 64);
+  if constexpr (QJL == kQjlOff && !DV) {
+    if (a.new_k) {  // a step: one z layer more, for stage_new_rows
+      const dim3 g(grid.x, grid.y, grid.z + 1);
+      if (a.tier_splits > 0)
+        hipLaunchKernelGGL((decode_attention_kernel<KIND, W, kFlStep | kFlTiers>), g, block, 0, s, a);
+      else if (W == 4 && a.n_splits == 16)
+        hipLaunchKernelGGL((decode_attention_kernel<KIND, 4, kFlStep | kFlBatch16>), g, dim3(256), 0, s, a);
+      else
+        hipLaunchKernelGGL((decode_attention_kernel<KIND, W, kFlStep>), g, block, 0, s, a);
+      return;
+    }
+  }
   if (a.tier_splits > 0) {
     hipLaunchKernelGGL((decode_attention_kernel<KIND, W, kFlTiers, QJL, DV>), grid, block, 0, s, a);
     return;
@@ -2267,6 +2345,14 @@ static void launch_decode_kind(const AttnArgs& a, int kind, dim3 grid, hipStream
 // A call without pages: one split over the dense tail, no table, no page loads
 // and no sketches (the tail takes no correction).
 static void launch_decode_tail(const AttnArgs& a, dim3 grid, hipStream_t s) {
+  if (a.new_k) {
+    grid.z += 1;
+    if (a.g <= 8)
+      hipLaunchKernelGGL((decode_attention_kernel<kKindNone, 4, kFlStep>), grid, dim3(256), 0, s, a);
+    else
+      hipLaunchKernelGGL((decode_attention_kernel<kKindNone, kDecodeWaves, kFlStep>), grid, dim3(kDecodeWaves * 64), 0, s, a);
+    return;
+  }
   if (a.g <= 8)
     hipLaunchKernelGGL((decode_attention_kernel<kKindNone, 4>), grid, dim3(256), 0, s, a);
   else
@@ -2318,7 +2404,7 @@ static int32_t decode_attention_impl(const void* q, int64_t batch, int32_t hq, i
                                      int64_t tail_stride, int64_t actual_seq_len, float scale,
                                      int32_t pages_per_split, void* workspace, size_t workspace_bytes, void* out,
                                      void* stream, bool use_qjl, const void* v_dense = nullptr,
-                                     int64_t v_capacity = 0) {
+                                     int64_t v_capacity = 0, const AttnArgs* step = nullptr) {
   clear_error();
   AttnArgs a{};
   if (!fill_common(a, q, batch, hq, hkv, layout, pages, n_pages, v_dense == nullptr)) return TP_ERR_INVALID;
@@ -2365,7 +2451,7 @@ static int32_t decode_attention_impl(const void* q, int64_t batch, int32_t hq, i
   const int32_t n_splits = n_splits_of(n_pages, pages_per_split);
   // The grid is (hkv, batch * head_blocks, n_splits); y and z are at most 65535.
   const int64_t n_rows = (int64_t)batch * a.head_blocks;
-  if (n_splits > 65535 || n_rows > 65535) {
+  if (n_splits > (step ? 65534 : 65535) || n_rows > 65535) {
     set_error("grid (%d, %lld, %d) exceeds the grid limit of 65535 in y and z%s", hkv, (long long)n_rows,
               n_splits, n_splits > 65535 ? "; raise pages_per_split" : "");
     return TP_ERR_INVALID;
@@ -2382,6 +2468,14 @@ static int32_t decode_attention_impl(const void* q, int64_t batch, int32_t hq, i
   a.n_splits = n_splits;
   a.live_end = (int32_t)std::min<int64_t>(n_pages, (actual_seq_len + kPageTokens - 1) / kPageTokens);
   a.div_head_blocks = make_fastdiv((uint32_t)a.head_blocks);
+  if (step) {
+    a.new_k = step->new_k;
+    a.new_v = step->new_v;
+    a.new_rows = (int32_t)(batch * hkv);
+    a.check = step->check;
+    a.flag = step->flag;
+    a.epoch = step->epoch;
+  }
   if (n_splits > 1) {
     const size_t need = tp_decode_workspace_bytes(batch, hq, hkv, n_pages, tail_len, pages_per_split);
     if (!workspace || workspace_bytes < need || ((uintptr_t)workspace & 255u)) {
@@ -2430,7 +2524,7 @@ static int32_t decode_attention_impl(const void* q, int64_t batch, int32_t hq, i
     return launch_status("tp_decode_attention_qjl");
   }
 #ifdef TP_TIMELINE
-  if (g_measure_variant != 0) {
+  if (g_measure_variant != 0 && !step) {
     // The measurement variants combine in one tier (any split count).
     a.tier_splits = 0;
     a.tier_groups = 0;
@@ -2452,6 +2546,35 @@ int32_t tp_decode_attention(const void* q, int64_t batch, int32_t hq, int32_t hk
   return decode_attention_impl(q, batch, hq, hkv, layout, pages, n_pages, nullptr, tail_k, tail_v, tail_len,
                                tail_stride, actual_seq_len, scale, pages_per_split, workspace, workspace_bytes, out,
                                stream, false);
+}
+
+int32_t tp_decode_step(const void* q, int64_t batch, int32_t hq, int32_t hkv, const tp_page_layout* layout,
+                       const tp_pages* pages, int32_t n_pages, const void* new_k, const void* new_v, void* tail_k,
+                       void* tail_v, int32_t tail_len, int64_t tail_stride, float scale, int32_t pages_per_split,
+                       void* workspace, size_t workspace_bytes, void* out, int32_t check, uint32_t* flag,
+                       uint32_t epoch, void* stream) {
+  clear_error();
+  if (!new_k || !new_v || (((uintptr_t)new_k | (uintptr_t)new_v) & 15u) || tail_len < 0 || tail_len + 1 >= kPageTokens) {
+    set_error("tp_decode_step takes the 16-byte aligned rows of one token that leaves the tail below a page, got "
+              "k=%p v=%p and %d tail tokens", new_k, new_v, tail_len);
+    return TP_ERR_INVALID;
+  }
+  if ((check != 2 && check != 3) || !flag || (epoch & 1u)) {
+    set_error("check must be 2 or 3 (deferred) with a pinned host flag and an even epoch");
+    return TP_ERR_INVALID;
+  }
+  AttnArgs step{};
+  step.new_k = static_cast<const uint16_t*>(new_k);
+  step.new_v = static_cast<const uint16_t*>(new_v);
+  step.check = check;
+  step.flag = flag;
+  step.epoch = epoch;
+  const int64_t total = (int64_t)n_pages * kPageTokens + tail_len + 1;
+  const int32_t st = decode_attention_impl(q, batch, hq, hkv, layout, pages, n_pages, nullptr, tail_k, tail_v,
+                                           tail_len + 1, tail_stride, total, scale, pages_per_split, workspace,
+                                           workspace_bytes, out, stream, false, nullptr, 0, &step);
+  if (st != TP_OK || check == 3) return st;
+  return wait_verdict(flag, epoch, static_cast<hipStream_t>(stream), true, "tp_decode_step");
 }
 
 int32_t tp_decode_attention_qjl(const void* q, int64_t batch, int32_t hq, int32_t hkv,
@@ -2670,6 +2793,13 @@ extern "C" unsigned long long tp_selftest_decode_bounds(const tp_bounds_case* c,
               }
             }
   } else {  // decode_attention_kernel
+    if (c->step) {  // stage_new_rows
+      for (int64_t ch = 0; ch < BH * 16; ++ch) {
+        log.check("new rows", ch * 16, 16, BH * kHeadDim * 2, -1, 0, (int)(ch & 63));
+        log.check("tail row", ((ch / 16 * c->tail_stride + c->tail_len - 1) * 16 + ch % 16) * 16, 16, sz_tail, -1, 0,
+                  (int)(ch & 63));
+      }
+    }
     AttnArgs a{};
     a.g = g;
     a.pages_per_split = pps;
@@ -2769,9 +2899,17 @@ extern "C" unsigned long long tp_selftest_decode_bounds(const tp_bounds_case* c,
             }
           }
           if (split == S - 1 && c->tail_len > 0 && wave == std::max(p_end - p_begin, 0) % waves &&
-              std::min<int64_t>(c->tail_len, seq - (int64_t)n_pages * kPageTokens) > 0)
-            log.check("tail (buffer range)", bkv * c->tail_stride * kHeadDim * 2, (int64_t)c->tail_len * kHeadDim * 2,
-                      sz_tail, L, wave, lane);
+              std::min<int64_t>(c->tail_len, seq - (int64_t)n_pages * kPageTokens) > 0) {
+            log.check("tail (buffer range)", bkv * c->tail_stride * kHeadDim * 2,
+                      (int64_t)(c->tail_len - (c->step ? 1 : 0)) * kHeadDim * 2, sz_tail, L, wave, lane);
+            if (c->step) {  // load_tail's rows of the step's own token
+              const int l4 = lane >> 4;
+              for (int kk = 0; kk < (hr ? 2 : 4); ++kk)
+                log.check("new k", (bkv * kHeadDim + (hr ? 64 * (l16 & 1) + 16 * l4 : 32 * l4) + 8 * kk) * 2, 16,
+                          BH * kHeadDim * 2, L, wave, lane);
+              log.check("new v", (bkv * kHeadDim + 8 * l16) * 2, 16, BH * kHeadDim * 2, L, wave, lane);
+            }
+          }
         }
       // The fold's record (or, with one split, output) stores: thread t, head t/32, dims 4(t%32)..+3.
       for (int tid = 0; tid < waves * 64; ++tid) {

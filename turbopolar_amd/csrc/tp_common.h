@@ -277,4 +277,9 @@ void set_error(const char* fmt, ...);
 void clear_error();
 bool check_layout(const tp_page_layout* layout, int* l1_row, int* deep_row);
 int32_t launch_status(const char* what);
+// The verdict of a check-2 launch on `s`: TP_OK, or TP_ERR_NONFINITE when the
+// pinned word `flag` holds epoch + 1.  A launch that also reports a finite input
+// (`reports`: it writes epoch then) is polled for, bounded, before the stream is
+// synchronised.
+int32_t wait_verdict(const uint32_t* flag, uint32_t epoch, hipStream_t s, bool reports, const char* what);
 }  // namespace tp

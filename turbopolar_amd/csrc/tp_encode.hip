@@ -1003,15 +1003,7 @@ int32_t tp_append_pages(const void* k, const void* v, int32_t in_dtype, int64_t 
   launch_encode(a, in_dtype, bh, n_head + rem > 0, s);
   const int32_t ls = launch_status("tp_append_pages");
   if (ls != TP_OK) return ls;
-  if (hipStreamSynchronize(s) != hipSuccess) {
-    set_error("tp_append_pages: synchronising the stream failed");
-    return TP_ERR_HIP;
-  }
-  if (*reinterpret_cast<volatile uint32_t*>(flag) == epoch + 1u) {
-    set_error("append() inputs must contain finite values");
-    return TP_ERR_NONFINITE;
-  }
-  return TP_OK;
+  return wait_verdict(flag, epoch, s, false, "tp_append_pages");
 }
 
 int32_t tp_selftest_f16_tables(uint16_t* sqrt_out, uint16_t* log_out, uint8_t* codes_out,

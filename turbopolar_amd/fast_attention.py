@@ -7,13 +7,13 @@ method names, the meaning of every argument, the validation messages of
 ``_validate_decode_shape`` (:89-104) and the layout ``make_turbo_caches``
 builds (:207-229).  The mechanism is this library's own:
 
-* ``decode_attention`` appends the token through the runtime (one staging
-  launch; a page encode when the token completes a page) and launches the
-  split-K decode kernel straight over the runtime's page store, used in place
-  with its capacity as the page stride, and over the runtime's dense-tail
-  buffer.  The store's ``tp_pages`` descriptor is kept until the store moves
-  (growth or reset).  A cache with no completed page runs the same kernel over
-  the tail alone (the reference switches to dense MLX attention there, :150-159).
+* ``decode_attention`` is one launch, which checks the token, copies it to the
+  runtime's dense-tail buffer and attends it with the tail and the runtime's page
+  store, used in place with its capacity as the page stride; a token that
+  completes a page is appended first (staging, page encode) and then attended.
+  The store's ``tp_pages`` descriptor is kept until the store moves (growth or
+  reset).  A cache with no completed page attends the tail alone (the reference
+  switches to dense MLX attention there, :150-159).
 * ``update_and_fetch`` (prefill) appends, encodes the zero-padded tail as one
   page (the reference's ``_maybe_encode_partial``) and decodes the stored
   pages and that page side by side into one fp16 K and one fp16 V buffer
@@ -128,13 +128,18 @@ class TurboPolarFastCache:
         per step; the transformers hook resolves every layer once per forward)."""
         self._validate_decode_shape(q, k_new, v_new, self.config)
         rt = self.runtime
-        rt.append(k_new.to(torch.float16), v_new.to(torch.float16), defer_check=defer_check)
+        k_new, v_new = k_new.to(torch.float16), v_new.to(torch.float16)
         if self._scale[0] != scale:
             self._scale = (scale, fp16_scale(scale))
+        layout = rt.polar_encoder.layout
+        out = rt.append_and_attend(q[:, :, 0], k_new, v_new, self._scale[1],
+                                   self._store_pages() if rt.k_storage.block_count else None, layout, defer_check)
+        if out is not None:
+            return out
+        rt.append(k_new, v_new, defer_check=defer_check)
         n_pages = rt.k_storage.block_count
         tail_k, tail_v = rt._tail_views()
         pages = self._store_pages() if n_pages else None
-        layout = rt.polar_encoder.layout
         return decode_attention_store(q[:, :, 0], layout, pages, n_pages, rt._num_kv_heads, tail_k, tail_v,
                                       rt.actual_seq_len, self._scale[1])
 

@@ -449,6 +449,33 @@ def decode_attention_store(q: torch.Tensor, layout, pages: TPPages, n_pages: int
                           0, None)
 
 
+def decode_step(q: torch.Tensor, layout, pages: Optional[TPPages], n_pages: int, new_k: torch.Tensor,
+                new_v: torch.Tensor, tail_k: torch.Tensor, tail_v: torch.Tensor, tail_len: int, scale: float,
+                check_mode: int, flag: torch.Tensor, epoch: int) -> torch.Tensor:
+    """tp_decode_step: the token ``new_k`` / ``new_v`` ``[B, H_kv, 1, 128]``
+    (contiguous fp16) joins the ``tail_len`` tokens of the tail buffers
+    ``[B, H_kv, 64, 128]`` and ``q`` ``[B, H_q, 128]`` attends all of it in one
+    launch.  Raises the append's ValueError when the launch reports a non-finite
+    value (``check_mode`` 2)."""
+    q16 = _q16(q)
+    B, Hq, _ = q16.shape
+    Hkv = new_k.shape[1]
+    dev = q16.device
+    out = torch.empty((B, Hq, HEAD_DIM), dtype=torch.float16, device=dev)
+    L = lib()
+    ws = _Workspace.get(dev, L.tp_decode_workspace_bytes(B, Hq, Hkv, n_pages, 0, 0))
+    with on_device(dev):
+        st = L.tp_decode_step(
+            q16.data_ptr(), B, Hq, Hkv, ctypes.byref(layout), ctypes.byref(pages if pages is not None else _NO_PAGES),
+            n_pages, new_k.data_ptr(), new_v.data_ptr(), tail_k.data_ptr(), tail_v.data_ptr(), tail_len, PAGE, scale, 0,
+            ws.data_ptr(), ws.numel(), out.data_ptr(), check_mode, flag.data_ptr(), epoch, stream_handle(dev),
+        )
+    if st == _lib.TP_ERR_NONFINITE:
+        raise ValueError("append() inputs must contain finite values")
+    check(st, "tp_decode_step")
+    return out
+
+
 def _tail_view(t: torch.Tensor):
     """(tensor, token stride) such that rows are dense 128-element fp16 rows and
     (batch, head) planes are ``stride`` rows apart."""
