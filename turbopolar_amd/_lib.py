@@ -248,6 +248,20 @@ def stream_handle(device: torch.device) -> int:
     return raw_stream(device.index if device.index is not None else torch.cuda.current_device())
 
 
+def call_on(device: torch.device, fn, *args):
+    """``fn(*args)`` with ``device`` current (a launch; the per-token paths'
+    form of ``on_device``)."""
+    idx = device.index
+    prev = torch._C._cuda_getDevice()
+    if prev == idx:
+        return fn(*args)
+    torch.cuda.set_device(idx)
+    try:
+        return fn(*args)
+    finally:
+        torch.cuda.set_device(prev)
+
+
 class on_device:
     """Makes ``device`` current for a launch, switching only when another
     device is current (a cheaper torch.cuda.device for the per-token paths)."""

@@ -42,6 +42,19 @@ def _pages_of(block: PolarKeyBlock, quant_v: Optional[QuantizedVBlock], head_dim
     return pages
 
 
+def _key_pages_of(block: PolarKeyBlock, head_dim: int) -> PageSet:
+    """PageSet of a key block alone, kept on the block object while its buffers
+    are those it was built from and are used in place."""
+    bufs = (block.radii, block.angle_codes_l1, block.angle_codes_deep, block.radii_scales)
+    hit = block.__dict__.get("_tp_key_pages")
+    if hit is not None and hit[1] == head_dim and hit[2] is block.metadata and all(a is b for a, b in zip(hit[0], bufs)):
+        return hit[3]
+    pages = PageSet(block, None, head_dim)
+    if pages.in_place:
+        block.__dict__["_tp_key_pages"] = (bufs, head_dim, block.metadata, pages)
+    return pages
+
+
 class HipKernelBridge:
     """Process-wide singleton, like the reference bridge (metal.py:72-86)."""
 
@@ -75,7 +88,7 @@ class HipKernelBridge:
 
     def execute_fused_qk(self, q: torch.Tensor, block: PolarKeyBlock, config) -> torch.Tensor:
         self._supports_block(block)
-        return fused_qk(q, PageSet(block, None, config.head_dim), fp16_scale(config.attention_scale))
+        return fused_qk(q, _key_pages_of(block, config.head_dim), fp16_scale(config.attention_scale))
 
     def execute_fused_qk_qjl(self, q: torch.Tensor, block: PolarKeyBlock, qjl_payload, q_proj_signs: torch.Tensor,
                              config) -> torch.Tensor:

@@ -30,6 +30,8 @@ class PolarQuantEncoder:
         self.l1_scale = float(self.l1_levels - 1)
         self.deep_scale = float(self.deep_levels - 1)
         self.use_int8_radii = bool(getattr(config, "use_int8_radii", False))
+        self._layout = _lib.make_layout(self.use_int8_radii, self.k_angle_bits_level1, self.k_angle_bits_deep,
+                                        self.split_dim)
 
     @property
     def metadata(self):
@@ -39,7 +41,7 @@ class PolarQuantEncoder:
 
     @property
     def layout(self):
-        return _lib.make_layout(self.use_int8_radii, self.k_angle_bits_level1, self.k_angle_bits_deep, self.split_dim)
+        return self._layout
 
     def row_bytes(self):
         split_half = self.split_dim // 2

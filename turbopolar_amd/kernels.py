@@ -7,13 +7,14 @@ enqueued on the current torch stream of the tensors' device.
 from __future__ import annotations
 
 import ctypes
+from functools import lru_cache
 from typing import Optional, Tuple
 
 import numpy as np
 import torch
 
 from . import _lib
-from ._lib import TPPages, check, lib, on_device, ptr, require_hip, stream_handle
+from ._lib import TPPages, call_on, check, lib, on_device, ptr, require_hip, stream_handle
 from .payload import PolarKeyBlock, QuantizedVBlock, layout_from_metadata
 
 PAGE = 64
@@ -22,6 +23,7 @@ PAIRS = 64
 V_GROUPS = 4
 
 
+@lru_cache(maxsize=64)
 def fp16_scale(scale: float) -> float:
     """The attention scale as the reference kernels receive it: a 0-d fp16
     array (rfsn_v11/kernels/turbo_polar/metal.py:518,692,774)."""
@@ -118,6 +120,8 @@ class PageSet:
                 raise ValueError(f"K pages {(self.B, self.H, self.S)} and V pages {tuple(codes.shape[:3])} differ")
             tensors["v_codes"] = (codes, (PAGE, HEAD_DIM))
             tensors["v_scales"] = (scales, (PAGE, V_GROUPS))
+        # Whether every buffer is used in place (changes to it are seen by later launches).
+        self.in_place = True
         caps = set()
         for name, (t, inner) in tensors.items():
             require_hip(t, name)
@@ -127,12 +131,14 @@ class PageSet:
             cap = _head_stride_pages(t, elems)
             if cap == -1 or not _inner_ok(t, inner) or (cap is not None and cap < self.S):
                 t = _fresh(t)
+                self.in_place = False
                 tensors[name] = (t, inner)
                 cap = _head_stride_pages(t, elems)
             caps.add(cap)
         caps.discard(None)
         if len(caps) > 1:
             # Buffers disagree on capacity: copy everything dense.
+            self.in_place = False
             for name, (t, inner) in list(tensors.items()):
                 if int(np.prod(inner)):
                     tensors[name] = (_fresh(t), inner)
@@ -244,6 +250,8 @@ def _q16(q: torch.Tensor) -> torch.Tensor:
     require_hip(q, "q")
     if q.dim() != 3 or q.shape[-1] != HEAD_DIM:
         raise ValueError(f"q must be [B, H_q, {HEAD_DIM}], got {tuple(q.shape)}")
+    if q.dtype is torch.float16 and q.is_contiguous():
+        return q
     return q.to(torch.float16).contiguous()
 
 
@@ -254,19 +262,15 @@ def fused_qk(q: torch.Tensor, pageset: PageSet, scale: float, qjl=None) -> torch
     B, Hq, _ = q16.shape
     if B != pageset.B or Hq % pageset.H:
         raise ValueError(f"q heads {Hq} / batch {B} do not match kv pages {pageset.B}x{pageset.H}")
-    scores = torch.empty((B, Hq, pageset.S * PAGE), dtype=torch.float16, device=q16.device)
-    with on_device(q16.device):
-        if qjl is None:
-            st = lib().tp_fused_qk(
-                ptr(q16), B, Hq, pageset.H, ctypes.byref(pageset.layout), ctypes.byref(pageset.pages),
-                pageset.S, float(scale), ptr(scores), stream_handle(q16.device),
-            )
-        else:
-            qjl.check_against(pageset.B, pageset.H, pageset.S, Hq)
-            st = lib().tp_fused_qk_qjl(
-                ptr(q16), B, Hq, pageset.H, ctypes.byref(pageset.layout), ctypes.byref(pageset.pages),
-                pageset.S, ctypes.byref(qjl.desc), float(scale), ptr(scores), stream_handle(q16.device),
-            )
+    dev = q16.device
+    scores = torch.empty((B, Hq, pageset.S * PAGE), dtype=torch.float16, device=dev)
+    common = (q16.data_ptr(), B, Hq, pageset.H, ctypes.byref(pageset.layout), ctypes.byref(pageset.pages), pageset.S)
+    if qjl is None:
+        st = call_on(dev, lib().tp_fused_qk, *common, float(scale), ptr(scores), stream_handle(dev))
+    else:
+        qjl.check_against(pageset.B, pageset.H, pageset.S, Hq)
+        st = call_on(dev, lib().tp_fused_qk_qjl, *common, ctypes.byref(qjl.desc), float(scale), ptr(scores),
+                     stream_handle(dev))
     check(st, "tp_fused_qk_qjl" if qjl is not None else "tp_fused_qk")
     return scores
 
@@ -278,13 +282,19 @@ class _Workspace:
     _bufs: dict = {}
 
     @classmethod
-    def get(cls, device: torch.device, nbytes: int) -> torch.Tensor:
-        key = (device.index, stream_handle(device))
+    def get(cls, device: torch.device, nbytes: int, stream: Optional[int] = None) -> torch.Tensor:
+        key = (device.index, stream_handle(device) if stream is None else stream)
         buf = cls._bufs.get(key)
         if buf is None or buf.numel() < nbytes:
             buf = torch.zeros(max(nbytes, 1 << 20), dtype=torch.uint8, device=device)
             cls._bufs[key] = buf
         return buf
+
+
+@lru_cache(maxsize=1024)
+def _workspace_bytes(B: int, Hq: int, Hkv: int, n_pages: int, pps: int) -> int:
+    """tp_decode_workspace_bytes (its size does not depend on the tail)."""
+    return int(lib().tp_decode_workspace_bytes(B, Hq, Hkv, n_pages, 0, pps))
 
 
 def decode_attention(
@@ -325,11 +335,7 @@ def decode_attention(
         require_hip(tail_k, "tail_k")
         if tail_k.shape != tail_v.shape or tuple(tail_k.shape[:2]) != (B, Hkv) or tail_k.shape[3] != HEAD_DIM:
             raise ValueError(f"tail shape {tuple(tail_k.shape)} does not match [B={B}, H_kv={Hkv}, T, {HEAD_DIM}]")
-        tk, tail_stride = _tail_view(tail_k.to(torch.float16))
-        tv, tail_stride_v = _tail_view(tail_v.to(torch.float16))
-        if tail_stride_v != tail_stride:
-            tk, tv = _fresh(tk), _fresh(tv)
-            tail_stride = tail_len
+        tk, tv, tail_stride = _tail_pair(tail_k, tail_v)
     layout = pageset.layout if pageset is not None else _DEFAULT_LAYOUT
     pages = pageset.pages if pageset is not None else _NO_PAGES
     if qjl is not None:
@@ -349,22 +355,16 @@ def _launch_decode(q16, Hkv, layout, pages, n_pages, tk, tv, tail_len, tail_stri
     if out is None:
         out = torch.empty((B, Hq, HEAD_DIM), dtype=torch.float16, device=dev)
     L = lib()
-    pps = int(pps) or int(L.tp_default_pages_per_split(B, Hq, Hkv, n_pages))
-    need = int(L.tp_decode_workspace_bytes(B, Hq, Hkv, n_pages, tail_len, pps))
-    ws = _Workspace.get(dev, need)
-    with on_device(dev):
-        if qjl is None:
-            st = L.tp_decode_attention(
-                ptr(q16), B, Hq, Hkv, ctypes.byref(layout), ctypes.byref(pages), n_pages,
-                ptr(tk), ptr(tv), tail_len, tail_stride, int(seq_len), float(scale), pps,
-                ws.data_ptr(), ws.numel(), ptr(out), stream_handle(dev),
-            )
-        else:
-            st = L.tp_decode_attention_qjl(
-                ptr(q16), B, Hq, Hkv, ctypes.byref(layout), ctypes.byref(pages), n_pages, ctypes.byref(qjl.desc),
-                ptr(tk), ptr(tv), tail_len, tail_stride, int(seq_len), float(scale), pps,
-                ws.data_ptr(), ws.numel(), ptr(out), stream_handle(dev),
-            )
+    pps = int(pps)  # 0: the library's default
+    stream = stream_handle(dev)
+    ws = _Workspace.get(dev, _workspace_bytes(B, Hq, Hkv, n_pages, pps), stream)
+    head = (ptr(q16), B, Hq, Hkv, ctypes.byref(layout), ctypes.byref(pages), n_pages)
+    rest = (None if tk is None else tk.data_ptr(), None if tv is None else tv.data_ptr(), tail_len, tail_stride,
+            int(seq_len), float(scale), pps, ws.data_ptr(), ws.numel(), ptr(out), stream)
+    if qjl is None:
+        st = call_on(dev, L.tp_decode_attention, *head, *rest)
+    else:
+        st = call_on(dev, L.tp_decode_attention_qjl, *head, ctypes.byref(qjl.desc), *rest)
     check(st, "tp_decode_attention_qjl" if qjl is not None else "tp_decode_attention")
     return out
 
@@ -414,9 +414,8 @@ def decode_attention_dense_v(
     if out is None:
         out = torch.empty((B, Hq, HEAD_DIM), dtype=torch.float16, device=dev)
     L = lib()
-    pps = int(pages_per_split) or int(L.tp_default_pages_per_split(B, Hq, Hkv, n_pages))
-    need = int(L.tp_decode_workspace_bytes(B, Hq, Hkv, n_pages, 0, pps))
-    ws = _Workspace.get(dev, need)
+    pps = int(pages_per_split)
+    ws = _Workspace.get(dev, _workspace_bytes(B, Hq, Hkv, n_pages, pps))
     with on_device(dev):
         st = L.tp_decode_attention_dense_v(
             ptr(q16), B, Hq, Hkv, ctypes.byref(pageset.layout), ctypes.byref(pageset.pages), n_pages,
@@ -439,10 +438,7 @@ def decode_attention_store(q: torch.Tensor, layout, pages: TPPages, n_pages: int
     tk = tv = None
     tail_stride = 0
     if tail_len:
-        tk, tail_stride = _tail_view(tail_k.to(torch.float16))
-        tv, stride_v = _tail_view(tail_v.to(torch.float16))
-        if stride_v != tail_stride:
-            tk, tv, tail_stride = _fresh(tk), _fresh(tv), tail_len
+        tk, tv, tail_stride = _tail_pair(tail_k, tail_v)
     if pages is None:
         pages, n_pages = _NO_PAGES, 0
     return _launch_decode(q16, num_kv_heads, layout, pages, n_pages, tk, tv, tail_len, tail_stride, seq_len, scale,
@@ -462,14 +458,14 @@ def decode_step(q: torch.Tensor, layout, pages: Optional[TPPages], n_pages: int,
     Hkv = new_k.shape[1]
     dev = q16.device
     out = torch.empty((B, Hq, HEAD_DIM), dtype=torch.float16, device=dev)
-    L = lib()
-    ws = _Workspace.get(dev, L.tp_decode_workspace_bytes(B, Hq, Hkv, n_pages, 0, 0))
-    with on_device(dev):
-        st = L.tp_decode_step(
-            q16.data_ptr(), B, Hq, Hkv, ctypes.byref(layout), ctypes.byref(pages if pages is not None else _NO_PAGES),
-            n_pages, new_k.data_ptr(), new_v.data_ptr(), tail_k.data_ptr(), tail_v.data_ptr(), tail_len, PAGE, scale, 0,
-            ws.data_ptr(), ws.numel(), out.data_ptr(), check_mode, flag.data_ptr(), epoch, stream_handle(dev),
-        )
+    stream = stream_handle(dev)
+    ws = _Workspace.get(dev, _workspace_bytes(B, Hq, Hkv, n_pages, 0), stream)
+    st = call_on(
+        dev, lib().tp_decode_step,
+        q16.data_ptr(), B, Hq, Hkv, ctypes.byref(layout), ctypes.byref(pages if pages is not None else _NO_PAGES),
+        n_pages, new_k.data_ptr(), new_v.data_ptr(), tail_k.data_ptr(), tail_v.data_ptr(), tail_len, PAGE, scale, 0,
+        ws.data_ptr(), ws.numel(), out.data_ptr(), check_mode, flag.data_ptr(), epoch, stream,
+    )
     if st == _lib.TP_ERR_NONFINITE:
         raise ValueError("append() inputs must contain finite values")
     check(st, "tp_decode_step")
@@ -480,13 +476,14 @@ def _tail_view(t: torch.Tensor):
     """(tensor, token stride) such that rows are dense 128-element fp16 rows and
     (batch, head) planes are ``stride`` rows apart."""
     B, H, T, D = t.shape
-    ok = t.stride(3) == 1 and (T == 1 or t.stride(2) == D)
+    s0, s1, s2, s3 = t.stride()
+    ok = s3 == 1 and (T == 1 or s2 == D)
     if ok:
         if H > 1:
-            plane = t.stride(1)
-            ok = plane % D == 0 and (B == 1 or t.stride(0) == H * plane)
+            plane = s1
+            ok = plane % D == 0 and (B == 1 or s0 == H * plane)
         elif B > 1:
-            plane = t.stride(0)
+            plane = s0
             ok = plane % D == 0
         else:
             plane = T * D
@@ -496,3 +493,12 @@ def _tail_view(t: torch.Tensor):
                 return t, stride
     t = _fresh(t)
     return t, T
+
+
+def _tail_pair(tail_k: torch.Tensor, tail_v: torch.Tensor):
+    """fp16 K and V tails and the token stride they share (``_tail_view``)."""
+    tk, stride = _tail_view(tail_k if tail_k.dtype is torch.float16 else tail_k.to(torch.float16))
+    tv, stride_v = _tail_view(tail_v if tail_v.dtype is torch.float16 else tail_v.to(torch.float16))
+    if stride_v != stride:
+        tk, tv, stride = _fresh(tk), _fresh(tv), tk.shape[2]
+    return tk, tv, stride

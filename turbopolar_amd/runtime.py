@@ -85,7 +85,7 @@ class TurboPolarKVCacheRuntime:
         """Views of the valid dense tail (rewritten in place by the next append)."""
         if not self._tail_len:
             return None, None
-        return self._tail_k[:, :, : self._tail_len], self._tail_v[:, :, : self._tail_len]
+        return self._tail_k.narrow(2, 0, self._tail_len), self._tail_v.narrow(2, 0, self._tail_len)
 
     def _validate_shapes(self, k_new, v_new) -> None:
         # turbo_polar_cache.py:55-68, same order and messages.

@@ -13,6 +13,7 @@ reporting the counters the doubling sequence would produce.
 from __future__ import annotations
 
 from dataclasses import dataclass, field
+from math import prod
 from typing import Optional, Tuple
 
 import torch
@@ -57,7 +58,7 @@ class Growth:
     def __init__(self, fresh: int = 0):
         self.fresh = fresh
         self._sets: list = []  # (storage, {attribute: new buffer}, capacity, reallocations, bytes grown)
-        self._rows: list = []  # (old buffer or None, new buffer, pages kept)
+        self._rows: list = []  # (old buffer or None, new buffer, pages kept, page bytes, (batch, head) rows)
 
     def add(self, storage, shapes: dict, needed: int, initial_capacity: int, device) -> None:
         """Room for ``needed`` pages in ``storage``; ``shapes`` maps its buffer
@@ -69,43 +70,41 @@ class Growth:
         caps, new_cap = _doublings(cap, needed)
         if not caps and not first:
             return
+        make = torch.empty if device.type == "cuda" else torch.zeros
         made, per_slot = {}, 0
         for name, spec in shapes.items():
             if spec is None:
                 made[name] = None
                 continue
             (B, H), page, dtype = spec
-            old = getattr(storage, name)
-            make = torch.empty if device.type == "cuda" else torch.zeros
-            new = make((B, H, new_cap) + page, dtype=dtype, device=device)
-            per_slot += new.numel() * new.element_size() // new_cap
-            if new.numel():
-                self._rows.append((old, new, storage.block_count))
-            made[name] = new
+            page_bytes = prod(page) * dtype.itemsize
+            new = made[name] = make((B, H, new_cap) + page, dtype=dtype, device=device)
+            per_slot += B * H * page_bytes
+            if page_bytes:
+                self._rows.append((getattr(storage, name), new, storage.block_count, page_bytes, B * H))
         self._sets.append((storage, made, new_cap, len(caps), per_slot * sum(caps)))
 
     def fill(self) -> None:
         """Copies the kept pages and clears the spare ones."""
-        rows = []
-        for old, new, keep in self._rows:
-            if new.device.type != "cuda":
+        held, rows, heads, dev = [], [], 0, None
+        for old, new, keep, page, heads in self._rows:
+            dev = new.device
+            if dev.type != "cuda":
                 if keep:
                     new[:, :, :keep] = old[:, :, :keep]
                 continue
-            if keep and not old.is_contiguous():
-                old = old.contiguous()
             cap = new.shape[2]
-            page = new.numel() * new.element_size() // (new.shape[0] * new.shape[1] * cap)
             used = min(cap, keep + self.fresh)
             if keep or used < cap:
-                rows.append((old, _lib.TPGrow(old.data_ptr() if keep else None, new.data_ptr(),
-                                              old.shape[2] * page if keep else 0, cap * page, keep * page, used * page)))
+                if keep and not old.is_contiguous():
+                    old = old.contiguous()
+                held.append(old)
+                rows.append(_lib.TPGrow(old.data_ptr() if keep else None, new.data_ptr(),
+                                        old.shape[2] * page if keep else 0, cap * page, keep * page, used * page))
         if not rows:
             return
-        new = self._rows[0][1]
-        descs = (_lib.TPGrow * len(rows))(*(d for _, d in rows))
-        with _lib.on_device(new.device):
-            st = _lib.lib().tp_grow_rows(descs, len(rows), new.shape[0] * new.shape[1], _lib.stream_handle(new.device))
+        st = _lib.call_on(dev, _lib.lib().tp_grow_rows, (_lib.TPGrow * len(rows))(*rows), len(rows), heads,
+                          _lib.stream_handle(dev))
         _lib.check(st, "tp_grow_rows")
 
     def buffer(self, storage, name: str):
