@@ -151,6 +151,16 @@ def test_decode_attention_batched(device, B, layout_name, hq, hkv, S, tail, pps,
     assert max_abs(out[0], out[1]) > 1e-2
 
 
+@pytest.mark.parametrize("B,layout_name,hq,hkv,S", [(5, "default", 16, 8, 29), (3, "fast", 24, 24, 25), (17, "default", 8, 8, 9),
+                                                    (33, "default", 8, 8, 11), (43, "fast", 18, 6, 9), (65, "default", 6, 6, 5)])
+def test_default_split_of_units_that_do_not_divide_the_gpu(device, B, layout_name, hq, hkv, S):
+    """40, 72, 136, 264, 258 and 390 units: several splits, one, and two."""
+    print(f"[attn-units] B={B} layout={layout_name} hq={hq} hkv={hkv} S={S}", flush=True)
+    block, qv, host, tk, tv, q = build_case(device, LAYOUTS[layout_name], hq, hkv, S, 7, seed=B, B=B)
+    out = run_gpu(device, block, qv, tk, tv, q, S * PAGE + 7)
+    check(out, oracle_out(host, tk, tv, q, S * PAGE + 7), f"units {B * hkv}")
+
+
 @pytest.mark.parametrize("B,S,tail,pps,drop", [(1, 3, 37, 1, 0), (2, 2, 63, 0, 0), (2, 4, 1, 2, 0),
                                                 (1, 2, 37, 1, 5), (3, 0, 20, 0, 0)])
 def test_decode_attention_tail_rows_past_len(device, B, S, tail, pps, drop):
