@@ -1352,7 +1352,7 @@ struct DecodeSlot {
   int64_t bkv;
 };
 
-template <bool STEP>
+template <bool STEP = false>
 __device__ __forceinline__ DecodeSlot decode_slot(const AttnArgs& a) {
   DecodeSlot d;
   d.kv = (int)blockIdx.x;
