@@ -542,6 +542,32 @@ def test_page_decode_parity(device):
         assert np.all(np.abs(kd - kref) <= ulp + 1e-12), name
 
 
+@pytest.mark.parametrize("layout", ANY_LAYOUTS)
+def test_page_decode_any_layout(device, layout):
+    """Every packing of the code rows, K and V together, K alone, V alone and a
+    gather of repeated and reordered pages: V exactly, K within one fp16 ulp."""
+    print(f"[decode-any] {layout}", flush=True)
+    block, qv, host, tk, tv, q = build_case(device, layout, 4, 2, 5, 0, seed=layout[3], B=2)
+    ps = PageSet(block, qv)
+    kg, vg = kernels.decode_pages(ps)
+    k_alone, _ = kernels.decode_pages(ps, want_v=False)
+    _, v_alone = kernels.decode_pages(ps, want_k=False)
+    idx = torch.tensor([4, 0, 0, 3], dtype=torch.int32, device=device)
+    kx, vx = kernels.decode_pages_gather(ps.layout, ps.pages, 2, 2, 5, idx, want_v=True)
+    torch.cuda.synchronize()
+    blk = {k: host[k] for k in ("radii", "radii_scales", "angle_codes_l1", "angle_codes_deep", "metadata")}
+    rs = None if blk["radii_scales"] is None else blk["radii_scales"].reshape(blk["radii"].shape[:3] + (1, 1))
+    kref = oracle.decode_block(blk["radii"], rs, blk["angle_codes_l1"], blk["angle_codes_deep"], blk["metadata"])
+    vref = oracle.dequantize_block(host["v_codes"], host["v_scales"]).reshape(kref.shape)
+    assert np.array_equal(vg.cpu().numpy().view(np.uint16), vref.view(np.uint16))
+    kd = kg.cpu().numpy().astype(np.float64)
+    ulp = np.spacing(np.abs(kref).astype(np.float16)).astype(np.float64)
+    assert np.all(np.abs(kd - kref) <= ulp + 1e-12)
+    assert torch.equal(k_alone, kg) and torch.equal(v_alone, vg)
+    pick = lambda t: t.reshape(2, 2, 5, PAGE, 128)[:, :, idx.long()].reshape(2, 2, 4 * PAGE, 128)  # noqa: E731
+    assert torch.equal(kx, pick(kg)) and torch.equal(vx, pick(vg))
+
+
 def test_repeated_launches_share_workspace(device):
     """300 back-to-back launches alternating two caches on one workspace, with
     many splits: every output is bit-identical to that cache's first output, so

@@ -238,13 +238,6 @@ __device__ __forceinline__ float code_angle(uint32_t code, int bits) {
   return t - kF32Pi;
 }
 
-// Extract code `idx` of a packed angle-code row (encoder.py:101-130 packing).
-__device__ __forceinline__ uint32_t packed_code(const uint8_t* row, int idx, int bits) {
-  if (bits == 8) return row[idx];
-  if (bits == 4) return (row[idx >> 1] >> ((idx & 1) * 4)) & 15u;
-  return (row[idx >> 2] >> ((idx & 3) * 2)) & 3u;
-}
-
 // Packed row length in bytes of n codes of `bits` bits.
 __host__ __device__ inline int packed_row_bytes(int n, int bits) {
   if (bits == 8) return n;

@@ -6,13 +6,6 @@
 // f32(2*pi) - f32(pi); r = f32(radius) or exp(f32(code) * f32(scale));
 // k = f16(r * cos(angle)), f16(r * sin(angle)); v = f16(f32(code) * f32(scale)).
 //
-// One 256-thread workgroup per page; thread (t = tid/4, q = tid%4) writes key
-// pairs [16q, 16q+16) and value group q of token t (64 contiguous bytes each).
-// The page's code rows are staged in LDS, and the fp32 cos / sin of every code
-// angle (and, for int8 log radii, exp(code * scale) of every code) are built
-// once per workgroup into LDS tables, so a pair costs two lookups and two fp32
-// multiplies; the table entries are the same fp32 values the per-pair
-// expressions give, so the output is unchanged.
 #include "tp_common.h"
 
 namespace tp {
@@ -50,107 +43,24 @@ __device__ __forceinline__ int64_t source_page(const DecodeArgs& a, int page) {
   return a.page_begin + page;
 }
 
-template <bool GATHER>
-__global__ __launch_bounds__(256) void decode_pages_kernel(DecodeArgs a) {
-  __shared__ float2 s_cs_l1[256];
-  __shared__ float2 s_cs_deep[256];
-  __shared__ float s_exp[256];
-  __shared__ uint32_t s_l1[kPageTokens * 64 / 4];
-  __shared__ uint32_t s_deep[kPageTokens * 64 / 4];
-  const int page = blockIdx.x;
-  const int64_t bh = blockIdx.y;
-  const int tid = threadIdx.x;
-  const int t = tid >> 2;
-  const int qq = tid & 3;
-  const int64_t slot = bh * a.capacity + source_page<GATHER>(a, page);
-  const int64_t row = slot * kPageTokens + t;
-  const int64_t out_off = (bh * a.out_tokens + a.out_offset + (int64_t)page * kPageTokens + t) * kHeadDim + 32 * qq;
-
-  if (a.k_out) {
-    // Tables: (cos, sin) of each l1 / deep code angle (decoder.py:37-55) and
-    // exp(code * scale) of each int8 log-radius code (decoder.py:57-62).
-    if (tid < (1 << a.l1_bits) && a.split_half > 0) {
-      const float th = code_angle((uint32_t)tid, a.l1_bits);
-      s_cs_l1[tid] = make_float2(cosf(th), sinf(th));
-    }
-    if (tid < (1 << a.deep_bits)) {
-      const float th = code_angle((uint32_t)tid, a.deep_bits);
-      s_cs_deep[tid] = make_float2(cosf(th), sinf(th));
-    }
-    if (a.int8_radii) s_exp[tid] = expf((float)(tid - 128) * h2f(a.radii_scales[slot]));
-    // The page's code rows: 64 rows of l1_row / deep_row bytes each, contiguous.
-    const uint32_t* l1src = reinterpret_cast<const uint32_t*>(a.angle_l1 + slot * kPageTokens * a.l1_row);
-    for (int i = tid; i < 16 * a.l1_row; i += 256) s_l1[i] = l1src[i];
-    const uint32_t* deepsrc = reinterpret_cast<const uint32_t*>(a.angle_deep + slot * kPageTokens * a.deep_row);
-    for (int i = tid; i < 16 * a.deep_row; i += 256) s_deep[i] = deepsrc[i];
-    // Radii of the thread's 16 pairs: 32 bytes (fp16) or 16 bytes (int8 codes).
-    uint4 rv[2];
-    if (a.int8_radii) {
-      rv[0] = *reinterpret_cast<const uint4*>(static_cast<const int8_t*>(a.radii) + row * kPairs + 16 * qq);
-      rv[1] = make_uint4(0u, 0u, 0u, 0u);
-    } else {
-      const uint4* rp = reinterpret_cast<const uint4*>(static_cast<const uint16_t*>(a.radii) + row * kPairs + 16 * qq);
-      rv[0] = rp[0];
-      rv[1] = rp[1];
-    }
-    __syncthreads();
-    const uint8_t* l1row = reinterpret_cast<const uint8_t*>(s_l1) + t * a.l1_row;
-    const uint8_t* deeprow = reinterpret_cast<const uint8_t*>(s_deep) + t * a.deep_row;
-    const uint32_t rw[8] = {rv[0].x, rv[0].y, rv[0].z, rv[0].w, rv[1].x, rv[1].y, rv[1].z, rv[1].w};
-    uint32_t w[16];
-#pragma unroll
-    for (int j = 0; j < 16; ++j) {
-      const int p = 16 * qq + j;
-      float r;
-      if (a.int8_radii) {
-        r = s_exp[((rw[j >> 2] >> (8 * (j & 3))) + 128u) & 0xffu];
-      } else {
-        r = h2f((uint16_t)(rw[j >> 1] >> (16 * (j & 1))));
-      }
-      const float2 cs = p < a.split_half ? s_cs_l1[packed_code(l1row, p, a.l1_bits)]
-                                         : s_cs_deep[packed_code(deeprow, p - a.split_half, a.deep_bits)];
-      w[j] = (uint32_t)f2h(r * cs.x) | ((uint32_t)f2h(r * cs.y) << 16);
-    }
-    uint4* dst = reinterpret_cast<uint4*>(a.k_out + out_off);
-#pragma unroll
-    for (int i = 0; i < 4; ++i) dst[i] = make_uint4(w[4 * i], w[4 * i + 1], w[4 * i + 2], w[4 * i + 3]);
-  }
-
-  if (a.v_out) {
-    const float s = h2f(a.v_scales[row * kVGroups + qq]);
-    const uint4* src = reinterpret_cast<const uint4*>(a.v_codes + row * kHeadDim + 32 * qq);
-    const uint4 c0 = src[0];
-    const uint4 c1 = src[1];
-    const uint32_t cw[8] = {c0.x, c0.y, c0.z, c0.w, c1.x, c1.y, c1.z, c1.w};
-    uint32_t w[16];
-#pragma unroll
-    for (int i = 0; i < 16; ++i) {
-      const int e0 = 2 * i, e1 = 2 * i + 1;
-      const float v0 = (float)(int8_t)((cw[e0 >> 2] >> (8 * (e0 & 3))) & 0xffu) * s;
-      const float v1 = (float)(int8_t)((cw[e1 >> 2] >> (8 * (e1 & 3))) & 0xffu) * s;
-      w[i] = (uint32_t)f2h(v0) | ((uint32_t)f2h(v1) << 16);
-    }
-    uint4* dst = reinterpret_cast<uint4*>(a.v_out + out_off);
-#pragma unroll
-    for (int i = 0; i < 4; ++i) dst[i] = make_uint4(w[4 * i], w[4 * i + 1], w[4 * i + 2], w[4 * i + 3]);
-  }
-}
-
-// ---- specialised layouts ------------------------------------------------------
+// One 256-thread workgroup per page.  Thread T decodes the 8-dim chunk c = T % 16
+// (pairs 4c .. 4c+3, V group c / 4) of tokens T / 16 + 16 k, k = 0..3, so every
+// load and store instruction of a wave covers consecutive bytes (a wave's
+// 16-byte output stores fill 1 KiB runs).  All loads are issued first; the fp32
+// (cos, sin) of every code angle and, for int8 log radii, the page's exp(code *
+// scale) are built in LDS while they are in flight, and V is decoded and stored
+// before the barrier that guards the tables, so a pair costs two lookups and two
+// fp32 multiplies, of the same fp32 values as the per-pair expressions.  V is
+// dequantised as fp16 pairs, f16(code * scale) with one rounding of the exact
+// product, as the f32 expression rounds it.
 //
-// The default layout (fp16 radii, 4-bit l1 and deep codes, split 64) and the
-// fast layout (int8 log radii with an fp16 page scale, 8-bit deep codes,
-// split 0) get their own kernel, one page per workgroup.  Thread T decodes
-// the 8-dim chunk c = T % 16 (pairs 4c .. 4c+3, V group c / 4) of tokens
-// T / 16 + 16 k, k = 0..3, so every load and store instruction of a wave
-// covers consecutive bytes (a wave's 16-byte output stores fill 1 KiB runs).
-// All loads are issued first; the (cos, sin) table (16 or 256 entries) and,
-// for the fast layout, the page's exp table are built in LDS while they are in
-// flight, and V is decoded and stored before the barrier that guards the
-// tables.  V is dequantised as fp16 pairs, f16(code * scale) with one
-// rounding of the exact product, as the f32 expression rounds it.  Outputs
-// are the generic kernel's, bit for bit.
-enum DecodeKind { kDecDefault = 0, kDecFast = 1 };
+// The default layout (fp16 radii, 4-bit l1 and deep codes, split 64) and the fast
+// layout (int8 log radii with an fp16 page scale, 8-bit deep codes, split 0) load
+// their codes by the chunk.  Any other layout's code rows are loaded as dwords,
+// staged in LDS beside the tables and read there by the byte (a kernel of its own,
+// with 64 contiguous bytes a thread, took 60.8 us for 512 pages x 8 heads of 2-bit
+// deep angles, 7.7 us for 5; this one 33.3 and 3.5).
+enum DecodeKind { kDecDefault = 0, kDecFast = 1, kDecAnyF16 = 2, kDecAnyI8 = 3 };
 
 __device__ __forceinline__ uint32_t i8pair_to_h2(uint32_t w, int first) {
   // Bytes `first` and `first + 1` of w (int8) as an exact fp16 pair.
@@ -164,12 +74,16 @@ __device__ __forceinline__ uint32_t i8pair_to_h2(uint32_t w, int first) {
 // branch made the compiler wait for the K loads at its join, so the V loads
 // went out one memory round trip late.
 template <int KIND, bool WANT_K, bool WANT_V, bool GATHER = false>
-__global__ __launch_bounds__(256) void decode_pages_spec_kernel(DecodeArgs a) {
+__global__ __launch_bounds__(256) void decode_pages_kernel(DecodeArgs a) {
   constexpr bool kFast = KIND == kDecFast;
-  constexpr int kCodes = kFast ? 256 : 16;
+  constexpr bool kAny = KIND == kDecAnyF16 || KIND == kDecAnyI8;
+  constexpr bool kI8 = kFast || KIND == kDecAnyI8;
+  constexpr int kCodes = kAny ? 512 : kFast ? 256 : 16;  // any layout: level-1 codes, then deep codes at 256
   constexpr int kTok = 4;  // tokens per thread
   __shared__ float2 s_cs[kCodes];
-  __shared__ float s_exp[kFast ? 256 : 1];
+  __shared__ float s_exp[kI8 ? 256 : 1];
+  constexpr int kRowWords = 4;  // dwords of code rows per thread: at most 64 code bytes a token
+  __shared__ uint32_t s_rows[kAny && WANT_K ? 256 * kRowWords : 1];
   const int tid = threadIdx.x;
   const int c = tid & 15;    // 8-dim chunk
   const int t0 = tid >> 4;   // first token; the others are t0 + 16 k
@@ -182,23 +96,38 @@ __global__ __launch_bounds__(256) void decode_pages_spec_kernel(DecodeArgs a) {
   constexpr bool want_v = WANT_V;
 
   // All loads first.
-  uint32_t rw[kTok][kFast ? 1 : 2];  // radii of pairs 4c..4c+3
+  uint32_t rw[kTok][kI8 ? 1 : 2];    // radii of pairs 4c..4c+3
   uint32_t cw[kTok];                 // their angle codes (low 16 bits for 4-bit codes)
   uint16_t ls16 = 0;
   if constexpr (want_k) {
 #pragma unroll
     for (int k = 0; k < kTok; ++k) {
       const int64_t row = row0 + t0 + 16 * k;
-      if constexpr (kFast) {
+      if constexpr (kI8) {
         rw[k][0] = *reinterpret_cast<const uint32_t*>(static_cast<const int8_t*>(a.radii) + row * kPairs + 4 * c);
-        cw[k] = *reinterpret_cast<const uint32_t*>(a.angle_deep + row * kPairs + 4 * c);
       } else {
         const uint2 r = *reinterpret_cast<const uint2*>(static_cast<const uint16_t*>(a.radii) + row * kPairs + 4 * c);
         rw[k][0] = r.x, rw[k][1] = r.y;
-        cw[k] = *reinterpret_cast<const uint16_t*>((c < 8 ? a.angle_l1 : a.angle_deep) + row * 16 + 2 * (c & 7));
       }
+      if constexpr (KIND == kDecFast)
+        cw[k] = *reinterpret_cast<const uint32_t*>(a.angle_deep + row * kPairs + 4 * c);
+      else if constexpr (KIND == kDecDefault)
+        cw[k] = *reinterpret_cast<const uint16_t*>((c < 8 ? a.angle_l1 : a.angle_deep) + row * 16 + 2 * (c & 7));
     }
-    if constexpr (kFast) ls16 = a.radii_scales[slot];
+    if constexpr (kI8) ls16 = a.radii_scales[slot];
+  }
+  // Any layout: dword i of the page's code rows, the level-1 ones first; threads
+  // past the last dword reread it.
+  uint32_t rows[kRowWords];
+  if constexpr (kAny && want_k) {
+    const int l1_words = kPageTokens / 4 * a.l1_row, words = l1_words + kPageTokens / 4 * a.deep_row;
+    const uint32_t* l1 = reinterpret_cast<const uint32_t*>(a.angle_l1 + row0 * a.l1_row);
+    const uint32_t* deep = reinterpret_cast<const uint32_t*>(a.angle_deep + row0 * a.deep_row);
+#pragma unroll
+    for (int j = 0; j < kRowWords; ++j) {
+      const int i = min(tid + 256 * j, words - 1);
+      rows[j] = *(i < l1_words ? l1 + i : deep + (i - l1_words));
+    }
   }
   uint2 vc[kTok];
   uint16_t vs16[kTok];
@@ -212,7 +141,16 @@ __global__ __launch_bounds__(256) void decode_pages_spec_kernel(DecodeArgs a) {
   }
 
   // Tables (decoder.py:37-62) while the loads are in flight.
-  if (want_k && tid < kCodes) {
+  if constexpr (kAny && want_k) {
+    if (tid < (1 << a.l1_bits)) {
+      const float th = code_angle((uint32_t)tid, a.l1_bits);
+      s_cs[tid] = make_float2(cosf(th), sinf(th));
+    }
+    if (tid < (1 << a.deep_bits)) {
+      const float th = code_angle((uint32_t)tid, a.deep_bits);
+      s_cs[256 + tid] = make_float2(cosf(th), sinf(th));
+    }
+  } else if (want_k && tid < kCodes) {
     const float th = code_angle((uint32_t)tid, kFast ? 8 : 4);
     s_cs[tid] = make_float2(cosf(th), sinf(th));
   }
@@ -232,7 +170,26 @@ __global__ __launch_bounds__(256) void decode_pages_spec_kernel(DecodeArgs a) {
     }
   }
   if constexpr (!want_k) return;
-  if constexpr (kFast) s_exp[tid] = expf((float)(tid - 128) * h2f(ls16));
+  if constexpr (kI8) s_exp[tid] = expf((float)(tid - 128) * h2f(ls16));
+  // Any layout: where the codes of pairs 4c .. 4c+3 sit in a token's rows.
+  int at[4], sh[4], step[4], table[4];
+  uint32_t mask[4];
+  if constexpr (kAny && want_k) {
+#pragma unroll
+    for (int j = 0; j < kRowWords; ++j) s_rows[tid + 256 * j] = rows[j];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const int p = 4 * c + j;
+      const bool in_l1 = p < a.split_half;
+      const int bits = in_l1 ? a.l1_bits : a.deep_bits;
+      const int bit = (in_l1 ? p : p - a.split_half) * bits;
+      step[j] = in_l1 ? a.l1_row : a.deep_row;
+      at[j] = (in_l1 ? 0 : kPageTokens * a.l1_row) + t0 * step[j] + (bit >> 3);
+      sh[j] = bit & 7;
+      mask[j] = (1u << bits) - 1u;
+      table[j] = in_l1 ? 0 : 256;
+    }
+  }
   __syncthreads();
 
   // K (decoder.py:57-67).
@@ -243,13 +200,14 @@ __global__ __launch_bounds__(256) void decode_pages_spec_kernel(DecodeArgs a) {
     for (int j = 0; j < 4; ++j) {
       float r;
       uint32_t code;
-      if constexpr (kFast) {
+      if constexpr (kI8)
         r = s_exp[((rw[k][0] >> (8 * j)) + 128u) & 0xffu];
-        code = (cw[k] >> (8 * j)) & 0xffu;
-      } else {
+      else
         r = h2f((uint16_t)(rw[k][j >> 1] >> (16 * (j & 1))));
-        code = (cw[k] >> (4 * j)) & 0xfu;
-      }
+      if constexpr (kAny)
+        code = table[j] + ((reinterpret_cast<const uint8_t*>(s_rows)[at[j] + 16 * k * step[j]] >> sh[j]) & mask[j]);
+      else
+        code = kFast ? (cw[k] >> (8 * j)) & 0xffu : (cw[k] >> (4 * j)) & 0xfu;
       const float2 cs = s_cs[code];
       w[j] = (uint32_t)f2h(r * cs.x) | ((uint32_t)f2h(r * cs.y) << 16);
     }
@@ -264,11 +222,21 @@ using namespace tp;
 template <int KIND, bool GATHER>
 static void launch_spec(const DecodeArgs& a, dim3 grid, hipStream_t s) {
   if (a.k_out && a.v_out)
-    hipLaunchKernelGGL((decode_pages_spec_kernel<KIND, true, true, GATHER>), grid, dim3(256), 0, s, a);
+    hipLaunchKernelGGL((decode_pages_kernel<KIND, true, true, GATHER>), grid, dim3(256), 0, s, a);
   else if (a.k_out)
-    hipLaunchKernelGGL((decode_pages_spec_kernel<KIND, true, false, GATHER>), grid, dim3(256), 0, s, a);
-  else
-    hipLaunchKernelGGL((decode_pages_spec_kernel<KIND, false, true, GATHER>), grid, dim3(256), 0, s, a);
+    hipLaunchKernelGGL((decode_pages_kernel<KIND, true, false, GATHER>), grid, dim3(256), 0, s, a);
+  else  // values alone: the key layout does not matter
+    hipLaunchKernelGGL((decode_pages_kernel<kDecDefault, false, true, GATHER>), grid, dim3(256), 0, s, a);
+}
+
+template <bool GATHER>
+static void launch_kind(const DecodeArgs& a, int kind, dim3 grid, hipStream_t s) {
+  switch (kind) {
+    case kDecDefault: launch_spec<kDecDefault, GATHER>(a, grid, s); break;
+    case kDecFast: launch_spec<kDecFast, GATHER>(a, grid, s); break;
+    case kDecAnyI8: launch_spec<kDecAnyI8, GATHER>(a, grid, s); break;
+    default: launch_spec<kDecAnyF16, GATHER>(a, grid, s); break;
+  }
 }
 
 // Pages [page_begin, page_begin + n_pages) (page_index NULL), or the stored
@@ -331,28 +299,12 @@ static int32_t decode_pages_impl(const tp_page_layout* layout, const tp_pages* p
   hipStream_t s = static_cast<hipStream_t>(stream);
   const bool is_default = !layout->int8_radii && layout->l1_bits == 4 && layout->deep_bits == 4 && layout->split_dim == 64;
   const bool is_fast = layout->int8_radii && layout->deep_bits == 8 && layout->split_dim == 0;
-  const bool aligned = (!k_out || (is_default ? ((uintptr_t)pages->angle_l1 & 1u) == 0 && ((uintptr_t)pages->angle_deep & 1u) == 0
-                                              : ((uintptr_t)pages->angle_deep & 3u) == 0 &&
-                                                    ((uintptr_t)pages->radii & 3u) == 0)) &&
-                       (!v_out || ((uintptr_t)pages->v_codes & 7u) == 0);
+  const int kind = is_default || !k_out ? kDecDefault : is_fast ? kDecFast : layout->int8_radii ? kDecAnyI8 : kDecAnyF16;
   const dim3 grid((unsigned)n_pages, (unsigned)bh);
-  if ((is_default || is_fast) && aligned) {
-    if (page_index) {
-      if (is_default)
-        launch_spec<kDecDefault, true>(a, grid, s);
-      else
-        launch_spec<kDecFast, true>(a, grid, s);
-    } else {
-      if (is_default)
-        launch_spec<kDecDefault, false>(a, grid, s);
-      else
-        launch_spec<kDecFast, false>(a, grid, s);
-    }
-  } else if (page_index) {
-    hipLaunchKernelGGL(decode_pages_kernel<true>, grid, dim3(256), 0, s, a);
-  } else {
-    hipLaunchKernelGGL(decode_pages_kernel<false>, grid, dim3(256), 0, s, a);
-  }
+  if (page_index)
+    launch_kind<true>(a, kind, grid, s);
+  else
+    launch_kind<false>(a, kind, grid, s);
   return launch_status("tp_decode_pages");
 }
 
