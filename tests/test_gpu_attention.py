@@ -232,7 +232,8 @@ ANY_LAYOUTS = [(False, 4, 2, 0), (False, 8, 8, 64), (True, 8, 2, 128), (False, 4
 
 
 @pytest.mark.parametrize("layout", ANY_LAYOUTS)
-@pytest.mark.parametrize("hq,hkv,S,tail,pps,B,drop", [(8, 2, 3, 5, 0, 2, 0), (4, 2, 21, 0, 9, 1, 70), (24, 2, 5, 9, 2, 1, 0)])
+@pytest.mark.parametrize("hq,hkv,S,tail,pps,B,drop", [(8, 2, 3, 5, 0, 2, 0), (4, 2, 21, 0, 9, 1, 70), (24, 2, 5, 9, 2, 1, 0),
+                                                     (8, 2, 11, 3, 5, 1, 0)])
 def test_any_layout(device, layout, hq, hkv, S, tail, pps, B, drop):
     """Decode attention and fused QK over every packing of the code rows, on 4
     and 8 waves, with several pages a wave, a masked suffix and a tail.

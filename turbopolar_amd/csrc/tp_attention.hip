@@ -2325,8 +2325,15 @@ static void launch_decode_w(const AttnArgs& a, dim3 grid, hipStream_t s) {
 // combine), 13.12 -> 12.61 at 16k and 11.98 -> 11.41 at 12k (8 kv heads, 8-
 // and 6-page splits), 13.10 -> 12.20 for batch 2 at 8k; longer splits stay on
 // 8 waves (at 32k, 4-wave workgroups with 8-page splits took 20.68 us against
-// 18.40 for the default 16-page splits on 8 waves).
-static bool four_waves(const AttnArgs& a) { return a.g <= 8 && a.pages_per_split <= 8; }
+// 18.40 for the default 16-page splits on 8 waves).  The kernels of any other
+// layout unpack a page for about as long as they wait for it, so a second page
+// on the same wave costs its whole time: they stay on 8 waves from 5 pages a
+// split on (32/8 heads, deep codes of 2 bits, 4 against 8 waves: 14.95 -> 13.59
+// us at 9,000 tokens, 15.88 -> 14.17 at 16,400; at 4 pages a split 11.20 on 4
+// waves against 12.01).
+static bool four_waves(const AttnArgs& a, int kind) {
+  return a.g <= 8 && a.pages_per_split <= (any_kind(kind) ? 4 : 8);
+}
 
 // The decode kernel's kind for a layout kind: default-layout pages take the
 // half-row token order when every head block has at most 8 query heads (its
@@ -2339,7 +2346,7 @@ static int decode_kind(int kind, const AttnArgs& a) { return kind == kKindDefaul
 
 template <int KIND, int QJL>
 static void launch_decode(const AttnArgs& a, dim3 grid, hipStream_t s) {
-  if (four_waves(a))
+  if (four_waves(a, KIND))
     launch_decode_w<KIND, 4, QJL>(a, grid, s);
   else
     launch_decode_w<KIND, kDecodeWaves, QJL>(a, grid, s);
@@ -2378,7 +2385,7 @@ static void launch_decode_tail(const AttnArgs& a, dim3 grid, hipStream_t s) {
 // size rule as the quantised V pages.
 template <int QJL>
 static void launch_decode_dense_v(const AttnArgs& a, int kind, dim3 grid, hipStream_t s) {
-  const bool w4 = four_waves(a);
+  const bool w4 = four_waves(a, kind);
   switch (decode_kind(kind, a)) {
     case kKindDefaultHR:
       if (w4)
@@ -2818,7 +2825,7 @@ extern "C" unsigned long long tp_selftest_decode_bounds(const tp_bounds_case* c,
     AttnArgs a{};
     a.g = g;
     a.pages_per_split = pps;
-    const int waves = four_waves(a) ? 4 : kDecodeWaves;
+    const int waves = four_waves(a, kind) ? 4 : kDecodeWaves;
     const Tiers tiers = S > 1 ? tiers_of(units, S) : Tiers{0, 0};
     const int slots = 1 + tiers.groups;
     const int32_t cstride = counter_stride_of(units * slots);
