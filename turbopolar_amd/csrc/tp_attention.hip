@@ -701,7 +701,7 @@ __device__ __forceinline__ void fold_halves(const float4v& acc, float4v& s, int 
 // A lane needs the codes of pairs 16 l4 .. +15 of four tokens.  Gathered byte by
 // byte from memory (64 loads a lane and page, none of them ahead of its use) the
 // codes took the decode step of a 2-bit deep layout at 16,400 tokens x 8 heads
-// to 54 us (16.5 now).  Instead a page's rows travel with the other page loads as whole
+// to 54 us (13.8 now).  Instead a page's rows travel with the other page loads as whole
 // chunks, go through the wave's own LDS (its merge area, free until the pages
 // are done), and come back as a bit stream per token: 16 codes of 2, 4 or 8 bits
 // from the bit where the lane's run starts, five dwords funnelled to that bit.
@@ -717,15 +717,13 @@ __device__ __forceinline__ void code_stream(const uint32_t* words, int bit, uint
   for (int i = 0; i < 4; ++i) s[i] = __builtin_amdgcn_alignbit(w[i + 1], w[i], sh);
 }
 
-// Codes 4 kk .. 4 kk + 3 of a stream as bytes.
+// Codes 4 kk .. 4 kk + 3 of a stream, from bit 0 of the word: code i is its bits
+// i * bits .. +bits-1, one v_bfe each (spreading them over bytes first took twice
+// the instructions: 32/8 heads, 2-bit deep codes, 14.17 -> 13.77 us at 16,400
+// tokens and 21.6 -> 20.7 at 32k; int8 radii with the split at pair 23, 15.1 -> 14.4).
 __device__ __forceinline__ uint32_t stream_codes(const uint32_t (&s)[4], int kk, int bits) {
-  uint32_t x4 = (s[kk >> 1] >> (16 * (kk & 1))) & 0xffffu;
-  x4 = (x4 | (x4 << 8)) & 0x00ff00ffu;
-  x4 = (x4 | (x4 << 4)) & 0x0f0f0f0fu;
-  uint32_t x2 = (s[0] >> (8 * kk)) & 0xffu;
-  x2 = (x2 | (x2 << 12)) & 0x000f000fu;
-  x2 = (x2 | (x2 << 6)) & 0x03030303u;
-  return bits == 8 ? s[kk] : bits == 4 ? x4 : x2;
+  const uint32_t w = bits == 8 ? s[kk] : bits == 4 ? s[kk >> 1] : s[0];
+  return w >> ((4 * kk * bits) & 31);
 }
 
 // QK over one compressed page: s[mt][i] = score(token score_token(mt, i, l4,
@@ -817,7 +815,7 @@ __device__ __forceinline__ void qk_regs(const AttnArgs& a, const Lut& lut, const
     const int row = 8 * (in_l1 ? a.l1_row : a.deep_row);
     const int deep0 = 8 * kPageTokens * a.l1_row;  // first deep bit of the page
     const int start = in_l1 ? p0 * bits : deep0 + (p0 - a.split_half) * bits;
-    const int table = in_l1 ? 0 : kLutDeep;
+    const uint32_t table = in_l1 ? 0 : kLutDeep;
     const bool holds_split = (a.split_half & 15) != 0;  // some lane's run does
     const int n_l1 = min(max(a.split_half - p0, 0), 16);
     float ls2 = 0.0f;
@@ -831,14 +829,17 @@ __device__ __forceinline__ void qk_regs(const AttnArgs& a, const Lut& lut, const
       float4v acc = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
       for (int kk = 0; kk < 4; ++kk) {
-        uint32_t codes = stream_codes(st, kk, bits);
-        int tab[4] = {table, table, table, table};
-        if (holds_split) {
-          const int n = min(max(n_l1 - 4 * kk, 0), 4);  // of these four pairs, the level-1 ones
-          const uint32_t mask = n == 4 ? 0xffffffffu : (1u << (8 * n)) - 1u;
-          codes = (codes & mask) | (stream_codes(sd, kk, a.deep_bits) & ~mask);
+        const uint32_t w4 = stream_codes(st, kk, bits);
+        uint32_t entry[4];
 #pragma unroll
-          for (int i = 0; i < 4; ++i) tab[i] = i < n ? 0 : kLutDeep;
+        for (int i = 0; i < 4; ++i) entry[i] = table + __builtin_amdgcn_ubfe(w4, i * bits, bits);
+        if (holds_split) {  // past the run's level-1 pairs, the deep row's
+          const uint32_t d4 = stream_codes(sd, kk, a.deep_bits);
+#pragma unroll
+          for (int i = 0; i < 4; ++i) {
+            const uint32_t deep = kLutDeep + __builtin_amdgcn_ubfe(d4, i * a.deep_bits, a.deep_bits);
+            entry[i] = 4 * kk + i < n_l1 ? entry[i] : deep;
+          }
         }
         uint32_t e[4];
 #pragma unroll
@@ -854,7 +855,7 @@ __device__ __forceinline__ void qk_regs(const AttnArgs& a, const Lut& lut, const
             const uint32_t w = (kk & 1) ? ((i & 2) ? q.w : q.z) : ((i & 2) ? q.y : q.x);
             r = (i & 1) ? hi_hi(w) : lo_lo(w);
           }
-          const uint32_t cs = lut.code[tab[i] + (int)((codes >> (8 * i)) & 0xffu)];
+          const uint32_t cs = lut.code[entry[i]];
           e[i] = pack_h2(r * __builtin_bit_cast(half2v, cs));
         }
         acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(as_half8(e[0], e[1], e[2], e[3]), qb[kk], acc, 0, 0, 0);
