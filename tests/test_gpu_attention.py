@@ -161,6 +161,29 @@ def test_default_split_of_units_that_do_not_divide_the_gpu(device, B, layout_nam
     check(out, oracle_out(host, tk, tv, q, S * PAGE + 7), f"units {B * hkv}")
 
 
+@pytest.mark.parametrize("units_batch,accepted", [(33, True), (31, False)])
+def test_default_split_without_a_workspace(device, units_batch, accepted):
+    """Above 256 units the default needs no workspace (its two splits become
+    one); at 248 units with a split of 4 pages forced it does."""
+    from turbopolar_amd import _lib
+
+    print(f"[attn-nows] B={units_batch}", flush=True)
+    S = 9
+    block, qv, host, tk, tv, q = build_case(device, LAYOUTS["default"], 8, 8, S, 0, seed=units_batch, B=units_batch)
+    ps = PageSet(block, qv)
+    qt = torch.from_numpy(q).to(device)
+    out = torch.empty((units_batch, 8, 128), dtype=torch.float16, device=device)
+    stream = torch.cuda.current_stream(device).cuda_stream
+    st = _lib.lib().tp_decode_attention(qt.data_ptr(), units_batch, 8, 8, ctypes.byref(ps.layout), ctypes.byref(ps.pages),
+                                        S, None, None, 0, 0, S * PAGE, SCALE16, 0 if accepted else 4, None, 0,
+                                        out.data_ptr(), stream)
+    if not accepted:
+        assert st == _lib.TP_ERR_WORKSPACE
+        return
+    assert st == _lib.TP_OK, _lib.lib().tp_last_error()
+    check(out.float().cpu().numpy(), oracle_out(host, tk, tv, q, S * PAGE), "one split")
+
+
 @pytest.mark.parametrize("B,S,tail,pps,drop", [(1, 3, 37, 1, 0), (2, 2, 63, 0, 0), (2, 4, 1, 2, 0),
                                                 (1, 2, 37, 1, 5), (3, 0, 20, 0, 0)])
 def test_decode_attention_tail_rows_past_len(device, B, S, tail, pps, drop):

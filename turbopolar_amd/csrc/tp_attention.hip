@@ -2470,7 +2470,15 @@ static int32_t decode_attention_impl(const void* q, int64_t batch, int32_t hq, i
     return TP_ERR_INVALID;
   }
   if (actual_seq_len > total) actual_seq_len = total;
-  if (pages_per_split <= 0) pages_per_split = tp_default_pages_per_split(batch, hq, hkv, n_pages);
+  if (pages_per_split <= 0) {
+    pages_per_split = tp_default_pages_per_split(batch, hq, hkv, n_pages);
+    // Above 256 units one split, which takes no workspace, fills the GPU too: a
+    // call without room for the default's two keeps to it.
+    if ((int64_t)batch * hkv * a.head_blocks > kTargetWorkgroups && n_splits_of(n_pages, pages_per_split) > 1 &&
+        (!workspace || ((uintptr_t)workspace & 255u) ||
+         workspace_bytes < tp_decode_workspace_bytes(batch, hq, hkv, n_pages, tail_len, pages_per_split)))
+      pages_per_split = n_pages;
+  }
   const int32_t n_splits = n_splits_of(n_pages, pages_per_split);
   // The grid is (hkv, batch * head_blocks, n_splits); y and z are at most 65535.
   const int64_t n_rows = (int64_t)batch * a.head_blocks;
