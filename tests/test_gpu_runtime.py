@@ -490,3 +490,21 @@ def test_decode_step_equals_append_then_attend(device, layout_name, hq, hkv, sta
         assert fast.runtime.get_io_telemetry() == ref.get_io_telemetry()
         assert ref.partial_k is None and fast.runtime.partial_k is None or torch.equal(fast.runtime.partial_k, ref.partial_k)
         assert ref.partial_v is None and fast.runtime.partial_v is None or torch.equal(fast.runtime.partial_v, ref.partial_v)
+
+
+def test_decode_step_of_another_batch_appends_every_row(device):
+    """A query of one batch over a cache of two takes the append and the attention
+    apart: every batch's rows reach the tail, and batch 0 is attended."""
+    cfg = TurboPolarConfig(num_q_heads=8, num_kv_heads=2)
+    g = torch.Generator(device=device).manual_seed(5)
+    k, v = (torch.randn((2, 2, 11, 128), generator=g, device=device).half() for _ in range(2))
+    q = torch.randn((1, 8, 1, 128), generator=g, device=device).half()
+    fast, ref = TurboPolarFastCache(cfg), TurboPolarKVCacheRuntime(cfg)
+    for rt in (fast.runtime, ref):
+        rt.append(k[:, :, :10].contiguous(), v[:, :, :10].contiguous())
+    out = fast.decode_attention(q, k[:, :, 10:], v[:, :, 10:], cfg.attention_scale)
+    ref.append(k[:, :, 10:].contiguous(), v[:, :, 10:].contiguous())
+    assert torch.equal(fast.runtime.partial_k, ref.partial_k) and torch.equal(fast.runtime.partial_v, ref.partial_v)
+    want = kernels.decode_attention_store(q[:, :, 0], ref.polar_encoder.layout, None, 0, 2, *ref._tail_views(), 11,
+                                          fp16_scale(cfg.attention_scale))
+    assert torch.equal(out, want)

@@ -280,6 +280,7 @@ class TurboPolarKVCacheRuntime:
             self._initialized and self._tail_k is not None and self._flag is not None and self._tail_len < PAGE - 1
             and self._input_dtype is torch.float16 and k_new.dtype is torch.float16 and v_new.dtype is torch.float16
             and tuple(k_new.shape) == shape and tuple(v_new.shape) == shape
+            and q.dim() == 3 and q.shape[0] == self._batch_size
             and k_new.device == self._tail_k.device == v_new.device == q.device and q.is_cuda
         ):
             return None
