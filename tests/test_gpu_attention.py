@@ -613,3 +613,40 @@ def test_repeated_launches_share_workspace(device):
         bad += (out != refs[it % 2]).sum() if it % 3 == 0 else (torch.abs(out.float() - refs[it % 2].float()) > 1e-3).sum()
     torch.cuda.synchronize()
     assert int(bad.item()) == 0
+
+
+@pytest.mark.parametrize("layout_name", ["default", "fast"])
+def test_scores_follow_the_block_as_it_is(device, layout_name):
+    """The bridge's scores of one block object, called again after its buffers were
+    exchanged in place, replaced by other forms (a larger store's views, a
+    transposed copy) and after the block was copied: each time those of a PageSet
+    built anew, and nothing is left on the block."""
+    import copy
+
+    from turbopolar_amd import HipKernelBridge, TurboPolarConfig
+
+    cfg = TurboPolarConfig(num_q_heads=8, num_kv_heads=2)
+    bridge = HipKernelBridge()
+    block, *_, q = build_case(device, LAYOUTS[layout_name], 8, 2, 3, 0)
+    q = torch.from_numpy(q).to(device)
+    other = build_case(device, LAYOUTS[layout_name], 8, 2, 3, 0, seed=9)[0]
+
+    def same():
+        got = bridge.execute_fused_qk(q, block, cfg)
+        want = kernels.fused_qk(q, PageSet(block, None, 128), fp16_scale(cfg.attention_scale))
+        assert torch.equal(got, want)
+        assert not [n for n in block.__dict__ if n.startswith("_")]
+        return got
+
+    first = same()
+    assert torch.equal(same(), first)
+    block.radii.data = other.radii.clone()
+    assert not torch.equal(same(), first)
+    block.angle_codes_deep = other.angle_codes_deep
+    same()
+    block.radii = torch.cat((block.radii, block.radii), dim=2)[:, :, :3]  # views of a store of six pages
+    same()
+    block.radii = block.radii.transpose(3, 4).contiguous().transpose(3, 4)
+    same()
+    twin = copy.deepcopy(block)
+    assert torch.equal(bridge.execute_fused_qk(q, twin, cfg), same())

@@ -26,7 +26,7 @@ import torch
 
 from . import _lib
 from .kernels import PageSet, decode_attention, decode_attention_dense_v, fp16_scale, fused_qk
-from .payload import PolarKeyBlock, QuantizedVBlock
+from .payload import PolarKeyBlock, QuantizedVBlock, layout_from_metadata
 from .qjl import QJLPages
 
 
@@ -43,16 +43,29 @@ def _pages_of(block: PolarKeyBlock, quant_v: Optional[QuantizedVBlock], head_dim
 
 
 def _key_pages_of(block: PolarKeyBlock, head_dim: int) -> PageSet:
-    """PageSet of a key block alone, kept on the block object while its buffers
-    are those it was built from and are used in place."""
+    """PageSet of a key block alone.  What its checks find depends only on the
+    buffers' forms (shape, strides, type, device) and the layout, so that is kept
+    by form and the buffers themselves are taken anew on each call: nothing is
+    attached to the block, and a buffer that was exchanged, resized or freed in
+    between is seen."""
     bufs = (block.radii, block.angle_codes_l1, block.angle_codes_deep, block.radii_scales)
-    hit = block.__dict__.get("_tp_key_pages")
-    if hit is not None and hit[1] == head_dim and hit[2] is block.metadata and all(a is b for a, b in zip(hit[0], bufs)):
-        return hit[3]
+    form = (head_dim, layout_from_metadata(block.metadata, head_dim)) + tuple(
+        None if t is None else (t.shape, t.stride(), t.dtype, t.device) for t in bufs)
+    plan = _key_plans.get(form)
+    if plan is not None:
+        return PageSet.of_plan(plan, bufs)
     pages = PageSet(block, None, head_dim)
-    if pages.in_place:
-        block.__dict__["_tp_key_pages"] = (bufs, head_dim, block.metadata, pages)
+    plan = pages.plan(bufs)
+    if plan is not None:
+        if len(_key_plans) >= _KEY_PLANS_MAX:
+            _key_plans.clear()
+        _key_plans[form] = plan
     return pages
+
+
+# A form holds no tensor; 256 of them are a context of 16k tokens scored page by page.
+_KEY_PLANS_MAX = 256
+_key_plans: dict = {}
 
 
 class HipKernelBridge:

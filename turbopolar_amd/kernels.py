@@ -156,6 +156,30 @@ class PageSet:
             int(self.capacity),
         )
 
+    def plan(self, bufs) -> Optional[tuple]:
+        """What ``of_plan`` takes to describe other key buffers of the same forms as
+        ``bufs`` (radii, level-1 codes, deep codes, scales), or None if one of
+        these was copied."""
+        used = [self.tensors.get(n) for n in ("radii", "angle_l1", "angle_deep", "radii_scales")]
+        if not self.in_place or any(u is not None and u.data_ptr() != t.data_ptr() for u, t in zip(used, bufs)):
+            return None
+        return self.layout, self.l1_row, self.deep_row, self.B, self.H, self.S, self.capacity, used[3] is not None
+
+    @classmethod
+    def of_plan(cls, plan: tuple, bufs) -> "PageSet":
+        """The PageSet of key buffers used in place, by a ``plan`` of their forms."""
+        self = cls.__new__(cls)
+        self.layout, self.l1_row, self.deep_row, self.B, self.H, self.S, self.capacity, scaled = plan
+        self.in_place = True
+        radii, l1, deep, scales = bufs
+        self.tensors = {"radii": radii, "angle_l1": l1, "angle_deep": deep}
+        if scaled:
+            self.tensors["radii_scales"] = scales
+        self.keep = list(bufs)
+        self.pages = TPPages(radii.data_ptr(), scales.data_ptr() if scaled else None, l1.data_ptr(), deep.data_ptr(),
+                             None, None, self.capacity)
+        return self
+
 
 # --------------------------------------------------------------------------
 # kernel calls
