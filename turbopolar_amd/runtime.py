@@ -272,6 +272,7 @@ class TurboPolarKVCacheRuntime:
         tokens that leave the dense tail below a page: the launch checks the token,
         copies it to the tail and attends it from ``k_new`` / ``v_new``, and the
         state moves on once its verdict is in (``defer_check`` as for ``append``).
+        The launch reads ``k_new`` and ``v_new`` to its end, as it does ``q``.
         ``pages``: the store's descriptor (ignored without pages).  None, with
         nothing done, if the call is not of that kind; the caller then appends and
         attends (a step at 300 tokens: 30.2 us in two launches, 18.3 in one)."""
