@@ -448,6 +448,32 @@ def test_append_of_whole_pages(device, dtype, layout_name, before, T):
         assert torch.equal(rt.partial_k, ref.partial_k) and torch.equal(rt.partial_v, ref.partial_v)
 
 
+@pytest.mark.parametrize("refused_T,T", [(3, 5), (3, 130), (70, 5), (70, 130)])
+@pytest.mark.parametrize("B,dtype", [(4, torch.float16), (1, torch.float32), (3, torch.float32)])
+def test_first_append_after_a_refused_one(device, refused_T, T, B, dtype):
+    """A refused first append (below a page, or of whole pages) leaves no buffer
+    behind that a larger batch or a wider type would then be written into."""
+    print(f"[refused-first] T={refused_T} then {T} B={B} {dtype}", flush=True)
+    cfg = _cfg("default", hq=4, hkv=2)
+    rt, ref = TurboPolarKVCacheRuntime(cfg), TurboPolarKVCacheRuntime(cfg)
+    bad = torch.zeros((1, 2, refused_T, 128), dtype=torch.float16, device=device)
+    bad[0, 1, refused_T - 1, 5] = float("nan")
+    with pytest.raises(ValueError, match="finite"):
+        rt.append(bad, bad)
+    assert rt.partial_k is None and rt.get_io_telemetry() == {}
+    g = torch.Generator(device=device).manual_seed(T)
+    k, v = (torch.randn((B, 2, T, 128), generator=g, device=device).to(dtype) for _ in range(2))
+    for c in (rt, ref):
+        c.append(k, v)
+    assert rt._tail_k.shape == (B, 2, PAGE, 128) and rt._tail_k.dtype == dtype
+    assert rt.get_io_telemetry() == ref.get_io_telemetry()
+    assert torch.equal(rt.partial_k, k[:, :, T // PAGE * PAGE:]) and torch.equal(rt.partial_v, v[:, :, T // PAGE * PAGE:])
+    n = rt.k_storage.block_count
+    if n:
+        assert torch.equal(rt.k_storage.radii[:, :, :n], ref.k_storage.radii[:, :, :n])
+        assert torch.equal(rt.v_storage.codes[:, :, :n], ref.v_storage.codes[:, :, :n])
+
+
 STEP_LAYOUTS = {"default": (False, 4, 4, 64), "fast": (True, 4, 8, 0), "deep2": (False, 4, 2, 64),
                 "odd_split": (True, 4, 2, 46)}
 

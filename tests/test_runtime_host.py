@@ -127,3 +127,14 @@ def test_storage_append_and_views_on_cpu():
     u = st.to_unified_block((1, 2, 5 * 64, 128))
     assert u.radii.shape == (1, 2, 5, 64, 64)
     assert [float(u.radii[0, 0, s, 0, 0]) for s in range(5)] == [0, 1, 2, 3, 4]
+
+
+def test_tail_of_a_refused_first_append_is_not_kept():
+    """A cache that has accepted nothing takes any batch and type: the dense tail's
+    buffers follow the first accepted append, not a refused one before it."""
+    rt = _rt()
+    rt._tail_k = rt._tail_v = torch.zeros((1, 4, 64, 128), dtype=torch.float16)  # as the refused append sized it
+    k, v = _x(B=3, T=5, dtype=torch.float32), _x(B=3, T=5, dtype=torch.float32)
+    rt.append(k, v)
+    assert rt._tail_k.shape == (3, 4, 64, 128) and rt._tail_k.dtype == torch.float32
+    assert torch.equal(rt.partial_k, k) and torch.equal(rt.partial_v, v)

@@ -221,6 +221,9 @@ class TurboPolarKVCacheRuntime:
         if self._pending and not (defer_check and k_new.ndim == 4 and k_new.shape[2] == 1 and self._tail_len > 0):
             self.resolve_deferred_check()
         self._validate_shapes(k_new, v_new)
+        if not self._initialized:
+            # What a refused first append left: it may have had another batch, type or device.
+            self._tail_k = self._tail_v = None
         if not (k_new.is_cuda and v_new.is_cuda) or self._invariant_error(k_new) is not None:
             self._validate_append_inputs(k_new, v_new)
             self._append_host_path(k_new, v_new)
