@@ -5,6 +5,7 @@ import ctypes
 import re
 
 import pytest
+import torch
 
 from turbopolar_amd import _lib
 from turbopolar_amd.payload import packed_row_bytes
@@ -251,3 +252,23 @@ def test_default_split_fills_the_gpu_once():
             limit = 256 if units <= 256 else 2 * units if units <= 384 else units
             assert units * splits <= limit, (units, n, pps)
     assert L.tp_default_pages_per_split(2, 40, 2, 300) == -(-300 // 32)  # 8 units: two head blocks each
+
+
+@pytest.mark.parametrize("change", [dict(k_angle_bits_deep=2), dict(k_angle_bits_level1=8), dict(split_dim=46),
+                                    dict(use_int8_radii=True), dict(k_angle_bits_deep=8, split_dim=0, use_int8_radii=True)])
+def test_encoder_layout_follows_its_attributes(change):
+    """An encoder's launches take the layout that its page buffers are sized for,
+    also after its public attributes were changed, and changed back."""
+    from turbopolar_amd import TurboPolarConfig
+    from turbopolar_amd.codecs import PolarQuantEncoder
+
+    enc = PolarQuantEncoder(TurboPolarConfig())
+    before = {name: getattr(enc, name) for name in change}
+    for attrs in (before, change, before):
+        for name, value in attrs.items():
+            setattr(enc, name, value)
+        lay = enc.layout
+        assert _lib.row_bytes(lay) == enc.row_bytes()
+        assert (bool(lay.int8_radii), lay.l1_bits, lay.deep_bits, lay.split_dim) == (
+            enc.use_int8_radii, enc.k_angle_bits_level1, enc.k_angle_bits_deep, enc.split_dim)
+        assert enc.page_shapes(1, 2)["radii"][2] == (torch.int8 if lay.int8_radii else torch.float16)

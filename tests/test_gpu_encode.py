@@ -207,6 +207,21 @@ def test_encode_into_capacity_slot(device):
     check_against_oracle(k, v, LAYOUTS["default"], device, capacity=8, page_begin=3)
 
 
+def test_encode_block_follows_the_encoders_attributes(device):
+    """One encoder whose public attributes change between blocks encodes each as a
+    new encoder of those widths does."""
+    k = torch.from_numpy(gen_kv(9, 1, 2, PAGE, "normal", np.float16)[0]).to(device)
+    enc = _encoder(LAYOUTS["default"])
+    for name in ("default", "deep2", "fast", "odd_split", "l1_8bit", "default"):
+        print(f"[encode-attributes] {name}", flush=True)
+        enc.use_int8_radii, enc.k_angle_bits_level1, enc.k_angle_bits_deep, enc.split_dim = LAYOUTS[name]
+        got, want = enc.encode_block(k), _encoder(LAYOUTS[name]).encode_block(k)
+        assert got.metadata == want.metadata
+        for f in ("radii", "angle_codes_l1", "angle_codes_deep", "radii_scales"):
+            a, b = getattr(got, f), getattr(want, f)
+            assert (a is None and b is None) or (a.dtype == b.dtype and torch.equal(a, b)), (name, f)
+
+
 def test_f16_tables_exhaustive(device):
     """sqrt, log and the angle->code rule over all 65536 fp16 bit patterns."""
     sq = torch.empty(65536, dtype=torch.int16, device=device)

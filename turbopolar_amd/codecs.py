@@ -30,8 +30,7 @@ class PolarQuantEncoder:
         self.l1_scale = float(self.l1_levels - 1)
         self.deep_scale = float(self.deep_levels - 1)
         self.use_int8_radii = bool(getattr(config, "use_int8_radii", False))
-        self._layout = _lib.make_layout(self.use_int8_radii, self.k_angle_bits_level1, self.k_angle_bits_deep,
-                                        self.split_dim)
+        self._layout = (None, None)  # (the attributes it was built from, tp_page_layout)
 
     @property
     def metadata(self):
@@ -41,7 +40,12 @@ class PolarQuantEncoder:
 
     @property
     def layout(self):
-        return self._layout
+        """tp_page_layout of the attributes as they are now, which ``row_bytes`` and the
+        page buffers follow too; the struct is kept for as long as they stay."""
+        form = (self.use_int8_radii, self.k_angle_bits_level1, self.k_angle_bits_deep, self.split_dim)
+        if self._layout[0] != form:
+            self._layout = (form, _lib.make_layout(*form))
+        return self._layout[1]
 
     def row_bytes(self):
         split_half = self.split_dim // 2
