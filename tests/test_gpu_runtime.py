@@ -518,6 +518,24 @@ def test_decode_step_equals_append_then_attend(device, layout_name, hq, hkv, sta
         assert ref.partial_v is None and fast.runtime.partial_v is None or torch.equal(fast.runtime.partial_v, ref.partial_v)
 
 
+@pytest.mark.parametrize("start", [10, 63])
+def test_decode_scale_changed_in_place(device, start):
+    """A step takes the scale's value at the call, of a tensor changed in place too
+    (one launch and, where the token completes a page, append and attention)."""
+    cfg = _cfg("default", hq=8, hkv=2)
+    g = torch.Generator(device=device).manual_seed(start)
+    k = torch.randn((1, 2, start + 2, 128), generator=g, device=device).half()
+    q = torch.randn((1, 8, 1, 128), generator=g, device=device).half()
+    a, b = TurboPolarFastCache(cfg), TurboPolarFastCache(cfg)
+    scale = torch.tensor(0.05)
+    for c in (a, b):
+        c.runtime.append(k[:, :, :start].contiguous(), k[:, :, :start].contiguous())
+    for t, value in ((start, 0.05), (start + 1, 0.25)):
+        scale.fill_(value)
+        tok = k[:, :, t:t + 1]
+        assert torch.equal(a.decode_attention(q, tok, tok, scale), b.decode_attention(q, tok, tok, value)), t
+
+
 def test_decode_step_of_another_batch_appends_every_row(device):
     """A query of one batch over a cache of two takes the append and the attention
     apart: every batch's rows reach the tail, and batch 0 is attended."""

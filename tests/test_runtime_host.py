@@ -8,6 +8,7 @@ import pytest
 import torch
 
 from turbopolar_amd import PolarKBlockStorage, TurboPolarConfig, TurboPolarFastCache, TurboPolarKVCacheRuntime
+from turbopolar_amd.kernels import fp16_scale
 from turbopolar_amd.storage import _doublings
 
 
@@ -127,6 +128,22 @@ def test_storage_append_and_views_on_cpu():
     u = st.to_unified_block((1, 2, 5 * 64, 128))
     assert u.radii.shape == (1, 2, 5, 64, 64)
     assert [float(u.radii[0, 0, s, 0, 0]) for s in range(5)] == [0, 1, 2, 3, 4]
+
+
+def test_fp16_scale_of_any_number():
+    """The scale is taken from what the caller hands over now: NumPy arrays and
+    tensors are accepted, one changed in place gives its new value, and a zero
+    keeps its sign."""
+    for make in (float, np.float32, np.float64, np.array, torch.tensor):
+        assert fp16_scale(make(0.088388)) == float(np.float16(0.088388)), make
+    for x in (torch.tensor(0.5), np.array(0.5)):
+        assert fp16_scale(x) == 0.5
+        x *= 4
+        assert fp16_scale(x) == 2.0
+    assert fp16_scale(1) == fp16_scale(True) == 1.0
+    assert [str(fp16_scale(z)) for z in (0.0, -0.0)] == ["0.0", "-0.0"]
+    with pytest.raises(TypeError):
+        fp16_scale(np.array([0.5, 0.6]))
 
 
 def test_tail_of_a_refused_first_append_is_not_kept():

@@ -47,7 +47,6 @@ class TurboPolarFastCache:
         self.v_dequantizer = GroupedVQuantizer(group_size=32)
         self.qjl_encoder = None
         self._store = None  # (radii buffer, V codes buffer, their tp_pages)
-        self._scale = (None, None)  # (scale given, the fp16 scale the kernel takes)
 
     @property
     def offset(self) -> int:
@@ -129,10 +128,9 @@ class TurboPolarFastCache:
         self._validate_decode_shape(q, k_new, v_new, self.config)
         rt = self.runtime
         k_new, v_new = k_new.to(torch.float16), v_new.to(torch.float16)
-        if self._scale[0] != scale:
-            self._scale = (scale, fp16_scale(scale))
+        scale = fp16_scale(scale)
         layout = rt.polar_encoder.layout
-        out = rt.append_and_attend(q[:, :, 0], k_new, v_new, self._scale[1],
+        out = rt.append_and_attend(q[:, :, 0], k_new, v_new, scale,
                                    self._store_pages() if rt.k_storage.block_count else None, layout, defer_check)
         if out is not None:
             return out
@@ -141,7 +139,7 @@ class TurboPolarFastCache:
         tail_k, tail_v = rt._tail_views()
         pages = self._store_pages() if n_pages else None
         return decode_attention_store(q[:, :, 0], layout, pages, n_pages, rt._num_kv_heads, tail_k, tail_v,
-                                      rt.actual_seq_len, self._scale[1])
+                                      rt.actual_seq_len, scale)
 
     # ------------------------------------------------------------------ mlx_lm cache protocol
     def size(self) -> int:

@@ -23,10 +23,18 @@ PAIRS = 64
 V_GROUPS = 4
 
 
-@lru_cache(maxsize=64)
-def fp16_scale(scale: float) -> float:
+def fp16_scale(scale) -> float:
     """The attention scale as the reference kernels receive it: a 0-d fp16
-    array (rfsn_v11/kernels/turbo_polar/metal.py:518,692,774)."""
+    array (rfsn_v11/kernels/turbo_polar/metal.py:518,692,774).  ``scale`` is
+    anything that NumPy converts; only plain non-zero floats, which nobody can
+    change, are looked up (0.2 us against 0.7; 0.0 and -0.0 are one key)."""
+    if type(scale) is float and scale:
+        return _fp16_of_float(scale)
+    return float(np.float16(scale))
+
+
+@lru_cache(maxsize=64)
+def _fp16_of_float(scale: float) -> float:
     return float(np.float16(scale))
 
 
