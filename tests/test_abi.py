@@ -241,16 +241,19 @@ def test_missing_library_fails_loudly(monkeypatch, tmp_path):
 
 
 def test_default_split_fills_the_gpu_once():
-    """The default split leaves at most 256 workgroups for up to 256 units (and
-    two splits a unit up to 384), covers every page, and keeps 4 pages a split."""
+    """The library's default split leaves at most 256 workgroups for up to 256 units
+    and one split a unit above, which takes no workspace; it covers every page,
+    keeps 4 pages a split, and never takes more splits than the rounded rule
+    ceil(n_pages x units / 256) that it replaced."""
     L = _lib.lib()
     for units in list(range(1, 300)) + [384, 385, 512, 4096]:
         for n in (1, 3, 4, 16, 62, 100, 512, 2049, 70000):
             pps = L.tp_default_pages_per_split(units, 4, 1, n)
             splits = -(-n // pps)
             assert pps >= 4 and splits <= 256
-            limit = 256 if units <= 256 else 2 * units if units <= 384 else units
-            assert units * splits <= limit, (units, n, pps)
+            assert units * splits <= max(256, units), (units, n, pps)
+            assert splits <= -(-n // max(4, -(-n * units // 256), -(-n // 256)))
+            assert L.tp_decode_workspace_bytes(units, 4, 1, n, 0, 0) == L.tp_decode_workspace_bytes(units, 4, 1, n, 0, pps)
     assert L.tp_default_pages_per_split(2, 40, 2, 300) == -(-300 // 32)  # 8 units: two head blocks each
 
 

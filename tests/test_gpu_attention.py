@@ -154,7 +154,7 @@ def test_decode_attention_batched(device, B, layout_name, hq, hkv, S, tail, pps,
 @pytest.mark.parametrize("B,layout_name,hq,hkv,S", [(5, "default", 16, 8, 29), (3, "fast", 24, 24, 25), (17, "default", 8, 8, 9),
                                                     (33, "default", 8, 8, 11), (43, "fast", 18, 6, 9), (65, "default", 6, 6, 5)])
 def test_default_split_of_units_that_do_not_divide_the_gpu(device, B, layout_name, hq, hkv, S):
-    """40, 72, 136, 264, 258 and 390 units: several splits, one, and two."""
+    """40, 72, 136, 264, 258 and 390 units: several splits and, from 136 on, one."""
     print(f"[attn-units] B={B} layout={layout_name} hq={hq} hkv={hkv} S={S}", flush=True)
     block, qv, host, tk, tv, q = build_case(device, LAYOUTS[layout_name], hq, hkv, S, 7, seed=B, B=B)
     out = run_gpu(device, block, qv, tk, tv, q, S * PAGE + 7)
@@ -163,8 +163,8 @@ def test_default_split_of_units_that_do_not_divide_the_gpu(device, B, layout_nam
 
 @pytest.mark.parametrize("units_batch,accepted", [(33, True), (31, False)])
 def test_default_split_without_a_workspace(device, units_batch, accepted):
-    """Above 256 units the default needs no workspace (its two splits become
-    one); at 248 units with a split of 4 pages forced it does."""
+    """Above 256 units the library's default is one split, which needs no workspace;
+    at 248 units with a split of 4 pages forced it does."""
     from turbopolar_amd import _lib
 
     print(f"[attn-nows] B={units_batch}", flush=True)

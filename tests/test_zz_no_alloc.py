@@ -65,6 +65,36 @@ def test_noalloc_matches_workspace_entry_point(device):
     assert torch.equal(out_again, first[8])
 
 
+def test_noalloc_default_above_256_units_leaves_the_scratch_alone(device):
+    """At 264 units the default split takes none of the scratch that every call on
+    the GPU shares, so calls on two streams do not meet: each of a run of pairs
+    gives the bits of the one-split launch."""
+    L = _lib.lib()
+    lay, S, B = LAYOUTS["default"], 9, 33
+    assert L.tp_default_pages_per_split(B, 8, 8, S) >= S
+    streams = [torch.cuda.Stream(device) for _ in range(2)]
+    cases = []
+    for seed in (93, 94):
+        print(f"[noalloc-streams] seed={seed}", flush=True)
+        block, qv, host, _, _, q = build_case(device, lay, 8, 8, S, 0, seed=seed, B=B)
+        ps, qt = PageSet(block, qv), torch.from_numpy(np.ascontiguousarray(q)).to(device)
+        outs = [torch.full((B, 8, 128), float("nan"), dtype=torch.float16, device=device) for _ in range(5)]
+        cases.append((ps, qt, outs))
+        common = (qt.data_ptr(), B, 8, 8, ctypes.byref(ps.layout), ctypes.byref(ps.pages), S, None, None, 0, 0,
+                  S * PAGE, SCALE16)
+        assert L.tp_decode_attention(*common, S, None, 0, outs[0].data_ptr(),
+                                     torch.cuda.current_stream(device).cuda_stream) == 0
+    torch.cuda.synchronize()
+    for i in range(1, 5):
+        for st, (ps, qt, outs) in zip(streams, cases):
+            assert L.tp_decode_attention_noalloc(qt.data_ptr(), B, 8, 8, ctypes.byref(ps.layout), ctypes.byref(ps.pages),
+                                                 S, None, None, 0, 0, S * PAGE, SCALE16, 0, outs[i].data_ptr(),
+                                                 st.cuda_stream) == 0
+    torch.cuda.synchronize()
+    for ps, qt, outs in cases:
+        assert all(torch.equal(o, outs[0]) for o in outs[1:])
+
+
 def test_noalloc_rejects_calls_beyond_its_scratch(device):
     L = _lib.lib()
     lay = _lib.make_layout(False, 4, 4, 64)

@@ -2156,23 +2156,20 @@ using namespace tp;
 extern "C" {
 
 // Pages per workgroup such that the workgroups fill the 256 CUs once: as many
-// splits per unit (batch row x kv head x head block) as 256 / units whole ones.
-// Rounding the pages per split instead (n_pages x units / 256 rounded up) left
-// 257 to 300 workgroups wherever the units do not divide 256, and the few past
-// the 256th cost a second round of the GPU.  Measured, 32 query / 8 kv heads, us
-// before -> now: batch 3 x 200 pages 26.2 -> 19.4, 5 x 62 18.2 -> 13.3, 6 x 100
-// 24.9 -> 19.5, 7 x 200 40.1 -> 35.9, 12 x 62 27.3 -> 23.6, 17 x 62 43.4 ->
-// 34.4; 24 kv heads x 200 25.9 -> 19.2.  Above 256 units one split per unit,
-// except where two splits take three rounds of half the pages and one takes two
-// of all (257..384 units): 33 x 62 72.9 -> 68.2, 40 x 62 75.5 -> 70.7.
+// splits per unit (batch row x kv head x head block) as 256 / units whole ones,
+// one above 256 units: such a launch takes no workspace, so calls on several
+// streams may share one or have none.  Rounding the pages per split instead
+// (n_pages x units / 256 rounded up) left 257 to 300 workgroups wherever the
+// units do not divide 256, and the few past the 256th cost a second round of the
+// GPU.  Measured, 32 query / 8 kv heads, us before -> now: batch 3 x 200 pages
+// 26.2 -> 19.4, 5 x 62 18.2 -> 13.3, 6 x 100 24.9 -> 19.5, 7 x 200 40.1 -> 35.9,
+// 12 x 62 27.3 -> 23.6, 17 x 62 43.4 -> 34.4; 24 kv heads x 200 25.9 -> 19.2.
+// (At 257..384 units two splits would be 6 % faster: 33 x 62 72.9 -> 68.2, 40 x 62
+// 75.5 -> 70.7.)
 int32_t tp_default_pages_per_split(int64_t batch, int32_t hq, int32_t hkv, int32_t n_pages) {
   if (batch < 1 || hq < 1 || hkv < 1 || n_pages < 1) return 4;
   const int64_t units = batch * hkv * (int64_t)head_blocks_of(hq, hkv);
-  int64_t splits = 1;
-  if (units <= kTargetWorkgroups)
-    splits = kTargetWorkgroups / units;
-  else if (units <= kTargetWorkgroups + kTargetWorkgroups / 2)
-    splits = 2;
+  const int64_t splits = units <= kTargetWorkgroups ? kTargetWorkgroups / units : 1;
   int64_t pps = (n_pages + splits - 1) / splits;
   if (pps < 4) pps = 4;
   const int64_t min_pps = (n_pages + 255) / 256;  // at most 256 splits per head
@@ -2470,15 +2467,7 @@ static int32_t decode_attention_impl(const void* q, int64_t batch, int32_t hq, i
     return TP_ERR_INVALID;
   }
   if (actual_seq_len > total) actual_seq_len = total;
-  if (pages_per_split <= 0) {
-    pages_per_split = tp_default_pages_per_split(batch, hq, hkv, n_pages);
-    // Above 256 units one split, which takes no workspace, fills the GPU too: a
-    // call without room for the default's two keeps to it.
-    if ((int64_t)batch * hkv * a.head_blocks > kTargetWorkgroups && n_splits_of(n_pages, pages_per_split) > 1 &&
-        (!workspace || ((uintptr_t)workspace & 255u) ||
-         workspace_bytes < tp_decode_workspace_bytes(batch, hq, hkv, n_pages, tail_len, pages_per_split)))
-      pages_per_split = n_pages;
-  }
+  if (pages_per_split <= 0) pages_per_split = tp_default_pages_per_split(batch, hq, hkv, n_pages);
   const int32_t n_splits = n_splits_of(n_pages, pages_per_split);
   // The grid is (hkv, batch * head_blocks, n_splits); y and z are at most 65535.
   const int64_t n_rows = (int64_t)batch * a.head_blocks;
