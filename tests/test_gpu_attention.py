@@ -18,7 +18,7 @@ import oracle
 from common import ATOL, LAYOUTS, PAGE, RTOL_L2, cosine, gen_kv, gen_q, max_abs, rel_l2
 from turbopolar_amd import kernels
 from turbopolar_amd.kernels import PageSet, fp16_scale
-from turbopolar_amd.payload import PolarKeyBlock, QuantizedVBlock
+from turbopolar_amd.payload import PolarKeyBlock, QuantizedVBlock, layout_metadata
 from test_gpu_encode import encode_gpu
 
 pytestmark = pytest.mark.gpu
@@ -590,6 +590,42 @@ def test_page_decode_any_layout(device, layout):
     assert torch.equal(k_alone, kg) and torch.equal(v_alone, vg)
     pick = lambda t: t.reshape(2, 2, 5, PAGE, 128)[:, :, idx.long()].reshape(2, 2, 4 * PAGE, 128)  # noqa: E731
     assert torch.equal(kx, pick(kg)) and torch.equal(vx, pick(vg))
+
+
+def test_int8_radii_of_any_layout_are_the_rounded_exponential(device):
+    """The radius of an int8 code in any layout but the benchmark's is fp16(exp(code *
+    scale)) of a float32 exponential, read back exactly as scores of one-hot queries
+    over keys of angle -pi.  The scales are those for which an exponential of code *
+    fp32(scale * log2 e), one rounding more and off by up to 1e-6, takes a
+    neighbouring fp16 value somewhere.  Radii whose exact value is within 1.5 float32
+    ulps of a midpoint (what a float32 exponential leaves open) or below fp16's
+    normal range are not compared."""
+    codes = np.arange(-128, 128)
+    scales = np.arange(np.float16(0.002).view(np.uint16), np.float16(0.0866).view(np.uint16), dtype=np.uint16).view(np.float16)
+    exact = np.exp(codes[None, :] * scales.astype(np.float64)[:, None])
+    r16 = exact.astype(np.float16)
+    up, down = (np.nextafter(r16, np.float16(d)).astype(np.float64) for d in (np.inf, 0))
+    to_midpoint = np.minimum(*(np.abs(exact - (r16.astype(np.float64) + n) / 2) for n in (up, down))) / exact
+    skip = (to_midpoint <= 1.5 * 2.0 ** -23) | (exact < 2.0 ** -14)
+    rounded = scales.astype(np.float32) * np.float32(np.log2(np.e))
+    coarse = np.exp2((codes.astype(np.float32) * rounded[:, None]).astype(np.float64)).astype(np.float16)
+    pick = np.flatnonzero(((coarse != r16) & ~skip).any(axis=1))
+    S = len(pick)
+    assert S >= 10
+    rows = np.broadcast_to(codes.astype(np.int8).reshape(1, 1, 1, 4, 64), (1, 1, S, 16, 4, 64)).reshape(1, 1, S, 64, 64)
+    t = lambda a: torch.from_numpy(np.ascontiguousarray(a)).to(device)  # noqa: E731
+    zeros = torch.zeros((1, 1, S, 64, 16), dtype=torch.uint8, device=device)
+    block = PolarKeyBlock(radii=t(rows), angle_codes_l1=zeros, angle_codes_deep=zeros, shape=(1, 1, S * 64, 128),
+                          block_size=64, head_dim=128, radii_scales=t(scales[pick].reshape(1, 1, S, 1, 1)),
+                          metadata=layout_metadata(4, 4, 64, True, 128))
+    q = torch.zeros((1, 64, 128), dtype=torch.float16, device=device)
+    q[0, torch.arange(64), 2 * torch.arange(64)] = -1.0  # head p: the first component of pair p
+    print(f"[int8-radii] {S} scales x 256 codes", flush=True)
+    got = kernels.fused_qk(q, PageSet(block, None), 1.0).cpu().numpy()  # [1, pair, 64 S]
+    at = (64 * (np.arange(64) % 4))[:, None] + np.arange(64)  # code index of (token, pair)
+    want, skip = r16[pick][:, at], skip[pick][:, at]
+    got = got[0].reshape(64, S, 64).transpose(1, 2, 0)
+    assert np.array_equal(got[~skip].view(np.uint16), want[~skip].view(np.uint16)), int((got != want)[~skip].sum())
 
 
 def test_repeated_launches_share_workspace(device):

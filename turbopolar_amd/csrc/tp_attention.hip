@@ -708,6 +708,7 @@ __device__ __forceinline__ void fold_halves(const float4v& acc, float4v& s, int 
 // A run that holds the split (split_dim not a multiple of 32) takes both rows'
 // streams and picks per pair.
 constexpr int kAnyCodeBytes = 16 * (64 * kAnyChunks + 2);  // the chunks, and what a stream reads past them
+constexpr int kAnyWaveBytes = kAnyCodeBytes + 256 * 2;      // and, for int8 log radii, the page's radii by code
 
 __device__ __forceinline__ void code_stream(const uint32_t* words, int bit, uint32_t (&s)[4]) {
   const uint32_t* d = words + (bit >> 5);
@@ -807,6 +808,20 @@ __device__ __forceinline__ void qk_regs(const AttnArgs& a, const Lut& lut, const
     wave_lds_sync();  // the previous page's streams are read
 #pragma unroll
     for (int j = 0; j < kAnyChunks; ++j) chunks[64 * j + 16 * l4 + l16] = k.c[j];
+    // int8 log radii: the page's 256 fp16 radii exp(code * scale) by the code's byte,
+    // four exponentials a lane instead of 64.  32/8 heads, us: 16,400 tokens 11.9 (the
+    // library's exp per pair 14.8), scores of 16,384 with the split at pair 23 7.7
+    // (10.8).  The hardware's exp2 of code * (scale * log2 e) per pair, 12.2 and 8.2,
+    // errs by up to 1.1e-6: 1.4e-4 of the radii took the neighbouring fp16 value.
+    f16* radius = reinterpret_cast<f16*>(static_cast<char*>(wave_lds) + kAnyCodeBytes);
+    if constexpr (KIND == kKindAnyI8) {
+      const float ls = h2f((uint16_t)k.ls_bits);
+      const int c0 = 4 * (16 * l4 + l16);
+      half2v x[2];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) x[i >> 1][i & 1] = (f16)expf((float)(int8_t)(c0 + i) * ls);
+      *reinterpret_cast<uint2*>(radius + c0) = make_uint2(pack_h2(x[0]), pack_h2(x[1]));
+    }
     wave_lds_sync();
     // The lane's stream: the row that its run starts in.
     const int p0 = 16 * l4;
@@ -818,8 +833,6 @@ __device__ __forceinline__ void qk_regs(const AttnArgs& a, const Lut& lut, const
     const uint32_t table = in_l1 ? 0 : kLutDeep;
     const bool holds_split = (a.split_half & 15) != 0;  // some lane's run does
     const int n_l1 = min(max(a.split_half - p0, 0), 16);
-    float ls2 = 0.0f;
-    if constexpr (KIND == kKindAnyI8) ls2 = h2f((uint16_t)k.ls_bits) * 1.44269504088896341f;
 #pragma unroll
     for (int mt = 0; mt < 4; ++mt) {
       const int t = 16 * mt + l16;
@@ -848,7 +861,7 @@ __device__ __forceinline__ void qk_regs(const AttnArgs& a, const Lut& lut, const
           if constexpr (KIND == kKindAnyI8) {
             const uint4 q = k.r[mt];
             const uint32_t w = kk == 0 ? q.x : kk == 1 ? q.y : kk == 2 ? q.z : q.w;
-            const f16 x = (f16)__builtin_amdgcn_exp2f((float)(int8_t)((w >> (8 * i)) & 0xffu) * ls2);
+            const f16 x = radius[(w >> (8 * i)) & 0xffu];
             r = half2v{x, x};
           } else {
             const uint4 q = k.r[mt][kk >> 1];
@@ -1842,7 +1855,7 @@ __global__ __launch_bounds__(WAVES * 64) void decode_attention_kernel(AttnArgs a
   // V: the page store's codes, or the dense V planes' rows (DV).
   typename std::conditional<DV, DenseVRegs, VRegs>::type vr;
   void* wave_lds = &sh.acc[wave][0];  // this wave's merge area, free until finish_unit
-  static_assert(sizeof(sh.acc[0]) >= kAnyCodeBytes, "a page's code rows fit the merge area");
+  static_assert(sizeof(sh.acc[0]) >= kAnyWaveBytes, "a page's code rows fit the merge area");
   if constexpr (KIND != kKindNone) {
     // A launch with pages has one in every split (p_begin < n_pages).  A wave
     // without a page of its own issues the same loads with every lane on the
@@ -1978,7 +1991,7 @@ __global__ __launch_bounds__(kQkWaves * 64) void fused_qk_kernel(AttnArgs a) {
   __shared__ float qjl_sin[QJL != kQjlOff ? kQjlMaxBits + 1 : 1];
   __shared__ uint32_t qjl_qw[QJL == kQjlAny ? 16 * kQjlMaxWords : 1];
   __shared__ uint4 stage[kQkWaves][16 * kQkRow / 8];
-  __shared__ uint4 code_rows[any_kind(KIND) ? kQkWaves : 1][any_kind(KIND) ? kAnyCodeBytes / 16 : 1];
+  __shared__ uint4 code_rows[any_kind(KIND) ? kQkWaves : 1][KIND == kKindAnyI8 ? kAnyWaveBytes / 16 : any_kind(KIND) ? kAnyCodeBytes / 16 : 1];
   const int tid = threadIdx.x;
   const int lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);  // wave-uniform: scalar branches
