@@ -518,6 +518,44 @@ def test_decode_step_equals_append_then_attend(device, layout_name, hq, hkv, sta
         assert ref.partial_v is None and fast.runtime.partial_v is None or torch.equal(fast.runtime.partial_v, ref.partial_v)
 
 
+@pytest.mark.parametrize("hq,hkv,start", [(8, 2, 5), (32, 8, 64 * 70 + 9), (4, 1, 64 * 600 + 3), (40, 2, 64 * 33 + 1)])
+def test_step_has_read_keys_and_values_when_it_returns(device, hq, hkv, start):
+    """With the immediate verdict a step's K and V are the caller's again when the
+    call is back: every unit that attends them has reported it, and a stream that
+    waits for nothing may overwrite them (a token that the append route takes,
+    too).  A cache without room for the reports takes that route."""
+    print(f"[step-inputs] hq={hq} hkv={hkv} start={start}", flush=True)
+    cfg = _cfg("default", hq=hq, hkv=hkv)
+    g = torch.Generator(device=device).manual_seed(start)
+    k, v = (torch.randn((1, hkv, start + 12, 128), generator=g, device=device).half() for _ in range(2))
+    q = torch.randn((12, 1, hq, 1, 128), generator=g, device=device).half()
+    rt, ref, small = (TurboPolarFastCache(cfg) for _ in range(3))
+    for c in (rt, ref, small):
+        c.runtime.append(k[:, :, :start].contiguous(), v[:, :, :start].contiguous())
+    units = hkv * -(-(hq // hkv) // 16)
+    assert rt.runtime._flag.numel() == 16 * (1 + units)
+    small.runtime._flag = torch.zeros(1, dtype=torch.int32, pin_memory=True)
+    other = torch.cuda.Stream(device)
+    kn, vn = torch.empty((1, hkv, 1, 128), dtype=torch.float16, device=device), torch.empty((1, hkv, 1, 128), dtype=torch.float16, device=device)
+    for i in range(12):
+        tok = slice(start + i, start + i + 1)
+        kn.copy_(k[:, :, tok])
+        vn.copy_(v[:, :, tok])
+        torch.cuda.synchronize()
+        out = rt.decode_attention(q[i], kn, vn, 0.088)
+        with torch.cuda.stream(other):
+            kn.fill_(float("nan"))
+            vn.fill_(float("nan"))
+        if rt.runtime._tail_len:  # a one-launch step, not the token that completed a page
+            assert (rt.runtime._flag.numpy()[::16] == rt.runtime._epoch).all()
+        want = ref.decode_attention(q[i], k[:, :, tok], v[:, :, tok], 0.088)
+        assert torch.equal(out, want), i
+        assert torch.equal(small.decode_attention(q[i], k[:, :, tok], v[:, :, tok], 0.088), want), i
+        torch.cuda.synchronize()
+    tail = (start + 12) // 64 * 64
+    assert torch.equal(rt.runtime.partial_k, k[:, :, tail:]) and torch.equal(rt.runtime.partial_v, v[:, :, tail:])
+
+
 @pytest.mark.parametrize("start", [10, 63])
 def test_decode_scale_changed_in_place(device, start):
     """A step takes the scale's value at the call, of a tensor changed in place too

@@ -56,15 +56,20 @@ int32_t launch_status(const char* what) {
   return TP_OK;
 }
 
-int32_t wait_verdict(const uint32_t* flag, uint32_t epoch, hipStream_t s, bool reports, const char* what) {
+int32_t wait_verdict(const uint32_t* flag, uint32_t epoch, hipStream_t s, bool reports, const char* what,
+                     int64_t n_done) {
   const volatile uint32_t* vf = flag;
   uint32_t verdict = 0;
-  bool done = false;
-  for (int spin = 0; reports && spin < (1 << 22) && !done; ++spin) {
-    verdict = *vf;
-    done = verdict == epoch || verdict == epoch + 1u;
+  int64_t seen = -1;  // what has come: the verdict, then the reports
+  for (int spin = 0; reports && spin < (1 << 22) && seen < n_done; ++spin) {
+    if (seen < 0) {
+      verdict = *vf;
+      if (verdict == epoch || verdict == epoch + 1u) seen = 0;
+    } else {
+      while (seen < n_done && vf[kReportStride * (seen + 1)] == epoch) ++seen;
+    }
   }
-  if (!done) {
+  if (seen < n_done) {
     if (hipStreamSynchronize(s) != hipSuccess) {
       set_error("%s: synchronising the stream failed", what);
       return TP_ERR_HIP;

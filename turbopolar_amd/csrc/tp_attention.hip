@@ -162,7 +162,7 @@ struct AttnArgs {
   const uint16_t* new_k;
   const uint16_t* new_v;
   int32_t new_rows;  // batch * hkv
-  int32_t check;     // as tp_append_stage: 2 reports the verdict, 3 only a non-finite value
+  int32_t check;     // as tp_append_stage: 2 reports the verdict (and take_new_row), 3 only a non-finite value
   uint32_t* flag;
   uint32_t epoch;
 };
@@ -971,9 +971,11 @@ struct TailRegs {
 };
 
 // STEP: the last row is not in the tail yet (stage_new_rows copies it there in
-// this launch); it comes from new_k / new_v, and the tail's range ends before it.
+// this launch); it comes from new_row (take_new_row) or, with nobody waiting, from
+// new_k and new_v, and the tail's range ends before it.
 template <bool HR, bool STEP>
-__device__ __forceinline__ void load_tail(const AttnArgs& a, int64_t bkv, int l16, int l4, TailRegs& r) {
+__device__ __forceinline__ void load_tail(const AttnArgs& a, int64_t bkv, int l16, int l4, const u32x4* new_row,
+                                          TailRegs& r) {
   const int64_t plane = bkv * a.tail_stride * kHeadDim;
   const int bytes = (a.tail_len - (STEP ? 1 : 0)) * kHeadDim * (int)sizeof(uint16_t);
   const __amdgpu_buffer_rsrc_t rk = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(a.tail_k + plane),
@@ -995,13 +997,19 @@ __device__ __forceinline__ void load_tail(const AttnArgs& a, int64_t bkv, int l1
     }
   }
   if constexpr (STEP) {
-    const uint16_t* nk = a.new_k + bkv * kHeadDim;
     const int row = a.tail_len - 1;
-    u32x4 w[HR ? 2 : 4];
+    const int c0 = HR ? 8 * (l16 & 1) + 2 * l4 : 4 * l4;
+    u32x4 w[HR ? 2 : 4], wv;
+    if (a.check == 2) {
 #pragma unroll
-    for (int kk = 0; kk < (HR ? 2 : 4); ++kk)
-      w[kk] = *reinterpret_cast<const u32x4*>(nk + (HR ? 64 * (l16 & 1) + 16 * l4 : 32 * l4) + 8 * kk);
-    const u32x4 wv = *reinterpret_cast<const u32x4*>(a.new_v + bkv * kHeadDim + 8 * l16);
+      for (int kk = 0; kk < (HR ? 2 : 4); ++kk) w[kk] = new_row[c0 + kk];
+      wv = new_row[16 + l16];
+    } else {
+      const u32x4* nk = reinterpret_cast<const u32x4*>(a.new_k + bkv * kHeadDim);
+#pragma unroll
+      for (int kk = 0; kk < (HR ? 2 : 4); ++kk) w[kk] = nk[c0 + kk];
+      wv = reinterpret_cast<const u32x4*>(a.new_v + bkv * kHeadDim)[l16];
+    }
     __builtin_amdgcn_sched_barrier(0);  // every load out before the first selection waits
 #pragma unroll
     for (int j = 0; j < 16; ++j) {
@@ -1018,7 +1026,9 @@ __device__ __forceinline__ void load_tail(const AttnArgs& a, int64_t bkv, int l1
 // rows to the tail, report), so the host has its verdict while the other
 // workgroups attend.  A launch of its own in front held the step up twice: the
 // attention launch waited for the verdict on the host, the next step's staging
-// for the attention on the GPU.
+// for the attention on the GPU.  The other readers of the rows, the workgroups that
+// attend the tail, report for themselves (take_new_row), so that the host returns once
+// nothing reads new_k and new_v any more.
 __device__ __forceinline__ void stage_new_rows(const AttnArgs& a) {
   if (blockIdx.x != 0 || blockIdx.y != 0) return;
   constexpr int kChunks = kHeadDim * 2 / 16;
@@ -1041,6 +1051,21 @@ __device__ __forceinline__ void stage_new_rows(const AttnArgs& a) {
   } else if (bad) {
     __hip_atomic_store(a.flag, a.epoch + 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
   }
+}
+
+// A step whose caller waits (check 2): the wave that will attend the tail takes its
+// unit's new rows (batch row, kv head, head block) into LDS, K's 16 chunks and then
+// V's, and reports that in the unit's own line after the flag's.  It does so before its
+// first page's loads: behind them the report came 4 us later while a 32k cache
+// streamed.  The wave has the fewest pages of its workgroup, so the others still wait
+// for theirs.
+__device__ __forceinline__ void take_new_row(const AttnArgs& a, int64_t bkv, int64_t unit, int lane, u32x4* new_row) {
+  const uint16_t* rows = (lane & 16) ? a.new_v : a.new_k;
+  const u32x4 w = *reinterpret_cast<const u32x4*>(rows + bkv * kHeadDim + 8 * (lane & 15));
+  if (lane < 32) new_row[lane] = w;
+  asm volatile("" ::"v"(w) : "memory");  // every lane's load is back before the report
+  if (lane == 0) __hip_atomic_store(a.flag + kReportStride * (1 + unit), a.epoch, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+  wave_lds_sync();
 }
 
 // QK over the dense tail (rows past tail_len are zero), in the token order
@@ -1370,7 +1395,9 @@ template <bool STEP = false>
 __device__ __forceinline__ DecodeSlot decode_slot(const AttnArgs& a) {
   DecodeSlot d;
   d.kv = (int)blockIdx.x;
-  d.split = (int)blockIdx.z - (STEP ? 1 : 0);  // a step's first z layer is stage_new_rows'
+  // A step's first z layer is stage_new_rows', and its splits run backwards: the last
+  // one, which attends the tail, starts first and has read the new rows early.
+  d.split = STEP ? a.n_splits - (int)blockIdx.z : (int)blockIdx.z;
   d.b = (int)fast_div(blockIdx.y, a.div_head_blocks);
   d.hb = (int)blockIdx.y - d.b * a.head_blocks;
   d.bkv = (int64_t)d.b * a.hkv + d.kv;
@@ -1825,6 +1852,7 @@ __global__ __launch_bounds__(WAVES * 64) void decode_attention_kernel(AttnArgs a
   // left to itself the compiler loaded the page pointers only after waiting
   // for the grid fields, a second round trip to fresh argument memory before
   // the first page request.
+  if constexpr (STEP) asm volatile("" ::"s"(a.n_splits), "s"(a.new_k), "s"(a.new_v));
   asm volatile("" ::"s"(a.q), "s"(a.radii), "s"(a.angle_l1), "s"(a.angle_deep), "s"(a.v_codes), "s"(a.v_scales),
                "s"(a.capacity), "s"(a.pages_per_split), "s"(a.live_end), "s"(a.head_blocks), "s"(a.hkv), "s"(a.g),
                "s"(a.hq), "s"(a.div_head_blocks.m), "s"(a.div_head_blocks.sh));
@@ -1844,6 +1872,12 @@ __global__ __launch_bounds__(WAVES * 64) void decode_attention_kernel(AttnArgs a
   // Compressed pages of this split that hold at least one unmasked token.
   const int p_begin = split * a.pages_per_split;
   const int p_end = min(p_begin + a.pages_per_split, a.live_end);
+
+  __shared__ u32x4 new_row[STEP ? 32 : 1];
+  if constexpr (STEP) {
+    if (a.check == 2 && split == a.n_splits - 1 && wave == max(p_end - p_begin, 0) % WAVES)
+      take_new_row(a, bkv, bkv * a.head_blocks + hb, lane, new_row);
+  }
 
   // Q and the first page's loads go out before the table build and the
   // barrier, and nothing before the barrier uses them.
@@ -1957,7 +1991,7 @@ __global__ __launch_bounds__(WAVES * 64) void decode_attention_kernel(AttnArgs a
       const int valid = (int)min((int64_t)a.tail_len, a.seq_len - tok0);
       if (valid > 0) {
         TailRegs tr;
-        load_tail<HR, STEP>(a, bkv, l16, l4, tr);
+        load_tail<HR, STEP>(a, bkv, l16, l4, new_row, tr);
         __builtin_amdgcn_sched_barrier(0);  // all 32 loads out before the first MFMA waits
         float4v s[4];
         qk_tail<HR>(tr, qb, s);
@@ -2607,7 +2641,8 @@ int32_t tp_decode_step(const void* q, int64_t batch, int32_t hq, int32_t hkv, co
                                            tail_len + 1, tail_stride, total, scale, pages_per_split, workspace,
                                            workspace_bytes, out, stream, false, nullptr, 0, &step);
   if (st != TP_OK || check == 3) return st;
-  return wait_verdict(flag, epoch, static_cast<hipStream_t>(stream), true, "tp_decode_step");
+  return wait_verdict(flag, epoch, static_cast<hipStream_t>(stream), true, "tp_decode_step",
+                      batch * hkv * head_blocks_of(hq, hkv));
 }
 
 int32_t tp_decode_attention_qjl(const void* q, int64_t batch, int32_t hq, int32_t hkv,
@@ -2935,12 +2970,16 @@ extern "C" unsigned long long tp_selftest_decode_bounds(const tp_bounds_case* c,
               std::min<int64_t>(c->tail_len, seq - (int64_t)n_pages * kPageTokens) > 0) {
             log.check("tail (buffer range)", bkv * c->tail_stride * kHeadDim * 2,
                       (int64_t)(c->tail_len - (c->step ? 1 : 0)) * kHeadDim * 2, sz_tail, L, wave, lane);
-            if (c->step) {  // load_tail's rows of the step's own token
-              const int l4 = lane >> 4;
-              for (int kk = 0; kk < (hr ? 2 : 4); ++kk)
-                log.check("new k", (bkv * kHeadDim + (hr ? 64 * (l16 & 1) + 16 * l4 : 32 * l4) + 8 * kk) * 2, 16,
-                          BH * kHeadDim * 2, L, wave, lane);
-              log.check("new v", (bkv * kHeadDim + 8 * l16) * 2, 16, BH * kHeadDim * 2, L, wave, lane);
+            if (c->step) {  // the new rows by take_new_row and by load_tail, the first one's LDS and report
+              const int l4 = lane >> 4, c0 = hr ? 8 * (l16 & 1) + 2 * l4 : 4 * l4;
+              const int64_t sz_new = BH * kHeadDim * 2;
+              log.check("new rows", (bkv * kHeadDim + 8 * (lane & 15)) * 2, 16, sz_new, L, wave, lane);
+              log.check("step flag", kReportStride * (1 + unit) * 4, 4, kReportStride * (1 + BH * head_blocks) * 4, L, wave, lane);
+              for (int kk = 0; kk < (hr ? 2 : 4); ++kk) {
+                log.check("new k", bkv * kHeadDim * 2 + (c0 + kk) * 16, 16, sz_new, L, wave, lane);
+                log.check("new k in LDS", (c0 + kk) * 16, 16, 256, L, wave, lane);
+              }
+              log.check("new v", bkv * kHeadDim * 2 + l16 * 16, 16, sz_new, L, wave, lane);
             }
           }
         }

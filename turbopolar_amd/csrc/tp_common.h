@@ -273,6 +273,10 @@ int32_t launch_status(const char* what);
 // The verdict of a check-2 launch on `s`: TP_OK, or TP_ERR_NONFINITE when the
 // pinned word `flag` holds epoch + 1.  A launch that also reports a finite input
 // (`reports`: it writes epoch then) is polled for, bounded, before the stream is
-// synchronised.
-int32_t wait_verdict(const uint32_t* flag, uint32_t epoch, hipStream_t s, bool reports, const char* what);
+// synchronised, and so are the n_done reports after it, one word each that the
+// launch sets to epoch, each on a 64-byte line of its own: side by side, the writes
+// of 8 XCDs and the host's polling cost a step 0.3 us more.
+constexpr int kReportStride = 16;
+int32_t wait_verdict(const uint32_t* flag, uint32_t epoch, hipStream_t s, bool reports, const char* what,
+                     int64_t n_done = 0);
 }  // namespace tp

@@ -120,7 +120,10 @@ class TurboPolarFastCache:
         """One decode step (turbopolar_fast_attention.py:106-188): append the
         token's K/V ``[1, H_kv, 1, 128]`` and attend ``q`` ``[1, H_q, 1, 128]``
         over every cached token with ``scale`` (taken as fp16, as the
-        reference's kernels receive it).  Returns fp16 ``[1, H_q, 128]``.
+        reference's kernels receive it).  Returns fp16 ``[1, H_q, 128]``.  The
+        caller may overwrite or free ``k_new`` and ``v_new`` on any stream once the
+        call is back (``q`` once its launch is through, and K and V too with
+        ``defer_check``).
 
         ``defer_check``: the append's non-finite verdict is read later by
         ``runtime.resolve_deferred_check()`` instead of now (no stream drain

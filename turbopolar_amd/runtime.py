@@ -27,7 +27,7 @@ import torch
 from . import _lib
 from .codecs import GroupedVQuantizer, PolarQuantDecoder, PolarQuantEncoder
 from .config import TurboPolarConfig
-from .kernels import PAGE, decode_pages_gather, decode_step, encode_pages
+from .kernels import PAGE, decode_pages_gather, decode_step, encode_pages, step_flag_words
 from .payload import PolarKeyBlock, QuantizedVBlock
 from .storage import Growth, PolarKBlockStorage, QuantVBlockStorage, pages_of
 
@@ -58,7 +58,7 @@ class TurboPolarKVCacheRuntime:
         self._tail_k: Optional[torch.Tensor] = None
         self._tail_v: Optional[torch.Tensor] = None
         self._tail_len = 0
-        self._flag: Optional[torch.Tensor] = None  # tp_append_stage verdict (pinned host memory)
+        self._flag: Optional[torch.Tensor] = None  # the launches' verdicts (pinned host memory)
         self._fused_views = None  # (block_count, storage buffers, (PolarKeyBlock, QuantizedVBlock))
         self._scratch = None  # one-page store for the padded tail when the storage is full
         self._epoch = 0
@@ -238,9 +238,10 @@ class TurboPolarKVCacheRuntime:
             self._tail_k = torch.empty((B, H, PAGE, D), dtype=k_new.dtype, device=k_new.device)
             self._tail_v = torch.empty((B, H, PAGE, D), dtype=k_new.dtype, device=k_new.device)
         if self._flag is None:
-            # Written by the staging kernel and read after one synchronisation,
-            # with no device-to-host copy.
-            self._flag = torch.zeros(1, dtype=torch.int32, pin_memory=True)
+            # Written by the append launches and read here, with no device-to-host
+            # copy; the words past the first are a one-launch step's.
+            words = step_flag_words(B, max(self.config.num_q_heads, H), H)
+            self._flag = torch.zeros(words, dtype=torch.int32, pin_memory=True)
         if self._tail_len:
             n_head, head_dst = min(PAGE - self._tail_len, T), self._tail_len
         elif T < PAGE:
@@ -275,16 +276,18 @@ class TurboPolarKVCacheRuntime:
         tokens that leave the dense tail below a page: the launch checks the token,
         copies it to the tail and attends it from ``k_new`` / ``v_new``, and the
         state moves on once its verdict is in (``defer_check`` as for ``append``).
-        The launch reads ``k_new`` and ``v_new`` to its end, as it does ``q``.
+        ``k_new`` and ``v_new`` are no longer read when the call returns, as after
+        ``append``; deferred they are read until the launch is through.
         ``pages``: the store's descriptor (ignored without pages).  None, with
         nothing done, if the call is not of that kind; the caller then appends and
         attends (a step at 300 tokens: 30.2 us in two launches, 18.3 in one)."""
-        shape = (self._batch_size, self._num_kv_heads, 1, self._head_dim)
+        shape, heads = (self._batch_size, self._num_kv_heads, 1, self._head_dim), q.shape
         if not (
             self._initialized and self._tail_k is not None and self._flag is not None and self._tail_len < PAGE - 1
             and self._input_dtype is torch.float16 and k_new.dtype is torch.float16 and v_new.dtype is torch.float16
-            and tuple(k_new.shape) == shape and tuple(v_new.shape) == shape
-            and q.dim() == 3 and q.shape[0] == self._batch_size
+            and k_new.shape == shape and v_new.shape == shape
+            and len(heads) == 3 and heads[0] == self._batch_size
+            and self._flag.numel() >= step_flag_words(heads[0], heads[1], self._num_kv_heads)
             and k_new.device == self._tail_k.device == v_new.device == q.device and q.is_cuda
         ):
             return None
