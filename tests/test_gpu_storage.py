@@ -57,6 +57,14 @@ def test_store_grows_like_one_reservation(device, int8, l1, deep, split):
     assert one.get_io_telemetry() == many.get_io_telemetry()
 
 
+def test_reservation_grows_a_store_in_its_own_form(device):
+    """The host test's stores on the GPU: two launches of the buffers' own rows."""
+    from test_runtime_host import grow_in_own_form
+
+    print("[grow-own-form]", flush=True)
+    grow_in_own_form("cuda")
+
+
 def test_grow_rows_rejects_bad_bounds():
     def call(n=1, rows=1, **kw):
         d = dict(src=4096, dst=8192, src_row=16, dst_row=32, keep=16, clear_from=16)

@@ -130,6 +130,48 @@ def test_storage_append_and_views_on_cpu():
     assert [float(u.radii[0, 0, s, 0, 0]) for s in range(5)] == [0, 1, 2, 3, 4]
 
 
+def test_reservation_grows_a_store_in_its_own_form():
+    """reserve() on a store that holds appended pages keeps their shape, type and
+    device, also where they are not the encoder's (32-token blocks, int8 radii), and
+    counts the growth by them."""
+    grow_in_own_form("cpu")
+
+
+def grow_in_own_form(device):
+    from turbopolar_amd.payload import PolarKeyBlock, QuantizedVBlock
+    from turbopolar_amd.codecs import PolarQuantEncoder
+    from turbopolar_amd.storage import QuantVBlockStorage
+
+    g = torch.Generator().manual_seed(7)
+    rand = lambda shape, dt: torch.randint(-100, 100, shape, generator=g).to(dt).to(device)  # noqa: E731
+    st, vs = PolarKBlockStorage(), QuantVBlockStorage()
+    blocks = [PolarKeyBlock(radii=rand((2, 3, 32, 64), torch.int8), angle_codes_l1=rand((2, 3, 32, 8), torch.uint8),
+                            angle_codes_deep=rand((2, 3, 32, 12), torch.uint8), shape=(2, 3, 32, 128), block_size=32,
+                            head_dim=128, radii_scales=rand((2, 3, 1, 1), torch.float16), metadata={"l1_bits": 4})
+              for _ in range(3)]
+    vblocks = [QuantizedVBlock(codes=rand((2, 3, 1, 64, 128), torch.int8), scales=rand((2, 3, 1, 64, 4), torch.float16),
+                               group_size=32) for _ in range(3)]
+    for b, v in zip(blocks, vblocks):
+        st.append(b)
+        vs.append(v)
+    other = PolarQuantEncoder(TurboPolarConfig(num_q_heads=4, num_kv_heads=1))
+    st.reserve(9, other, 1, 1, "cpu")
+    vs.reserve(9, 1, 1, "cpu")
+    assert (st.capacity, st.reallocation_count, vs.capacity) == (16, 2, 16)
+    assert st.bytes_copied_during_growth == (4 + 8) * 2 * 3 * (32 * (64 + 8 + 12) + 2)
+    for name in ("radii", "angle_codes_l1", "angle_codes_deep"):
+        t = getattr(st, name)
+        assert t.shape == (2, 3, 16) + getattr(blocks[0], name).shape[2:] and t.device.type == torch.device(device).type
+        assert t.dtype == getattr(blocks[0], name).dtype
+        for i, b in enumerate(blocks):
+            assert torch.equal(t[:, :, i], getattr(b, name)), (name, i)
+        assert not t[:, :, 3:].any()
+    for i, (b, v) in enumerate(zip(blocks, vblocks)):
+        assert torch.equal(st.radii_scales[:, :, i], b.radii_scales)
+        assert torch.equal(vs.codes[:, :, i], v.codes) and torch.equal(vs.scales[:, :, i], v.scales)
+    assert not vs.codes[:, :, 3:].any() and not vs.scales[:, :, 3:].any()
+
+
 def test_fp16_scale_of_any_number():
     """The scale is taken from what the caller hands over now: NumPy arrays and
     tensors are accepted, one changed in place gives its new value, and a zero

@@ -63,33 +63,39 @@ class Growth:
     def add(self, storage, shapes: dict, needed: int, initial_capacity: int, device) -> None:
         """Room for ``needed`` pages in ``storage``; ``shapes`` maps its buffer
         attributes to ((B, H), page shape, dtype), or None for a buffer that the
-        layout does not have.  The counters move as the reference's sequence of
+        layout does not have: the forms of a first reservation.  A buffer that is
+        there grows in its own form, on its own device (its pages may be ``append``'s,
+        of another length).  The counters move as the reference's sequence of
         doublings from the initial capacity moves them (storage.py:34-73)."""
-        first = storage.capacity == 0
+        first = all(getattr(storage, name) is None for name in shapes)
         cap = initial_capacity if first else storage.capacity
         caps, new_cap = _doublings(cap, needed)
         if not caps and not first:
             return
-        make = torch.empty if device.type == "cuda" else torch.zeros
         made, per_slot = {}, 0
         for name, spec in shapes.items():
+            old = getattr(storage, name)
+            if not first:
+                spec = None if old is None else (tuple(old.shape[:2]), tuple(old.shape[3:]), old.dtype)
             if spec is None:
                 made[name] = None
                 continue
+            if not first:
+                device = old.device
+            make = torch.empty if device.type == "cuda" else torch.zeros
             (B, H), page, dtype = spec
             page_bytes = prod(page) * dtype.itemsize
             new = made[name] = make((B, H, new_cap) + page, dtype=dtype, device=device)
             per_slot += B * H * page_bytes
             if page_bytes:
-                self._rows.append((getattr(storage, name), new, storage.block_count, page_bytes, B * H))
+                self._rows.append((old, new, storage.block_count, page_bytes, B * H))
         self._sets.append((storage, made, new_cap, len(caps), per_slot * sum(caps)))
 
     def fill(self) -> None:
         """Copies the kept pages and clears the spare ones."""
-        held, rows, heads, dev = [], [], 0, None
+        held, launches = [], {}  # (device, (batch, head) rows): buffers; one launch for a cache's two storages
         for old, new, keep, page, heads in self._rows:
-            dev = new.device
-            if dev.type != "cuda":
+            if new.device.type != "cuda":
                 if keep:
                     new[:, :, :keep] = old[:, :, :keep]
                 continue
@@ -99,13 +105,13 @@ class Growth:
                 if keep and not old.is_contiguous():
                     old = old.contiguous()
                 held.append(old)
-                rows.append(_lib.TPGrow(old.data_ptr() if keep else None, new.data_ptr(),
-                                        old.shape[2] * page if keep else 0, cap * page, keep * page, used * page))
-        if not rows:
-            return
-        st = _lib.call_on(dev, _lib.lib().tp_grow_rows, (_lib.TPGrow * len(rows))(*rows), len(rows), heads,
-                          _lib.stream_handle(dev))
-        _lib.check(st, "tp_grow_rows")
+                launches.setdefault((new.device, heads), []).append(
+                    _lib.TPGrow(old.data_ptr() if keep else None, new.data_ptr(),
+                                old.shape[2] * page if keep else 0, cap * page, keep * page, used * page))
+        for (dev, heads), rows in launches.items():
+            st = _lib.call_on(dev, _lib.lib().tp_grow_rows, (_lib.TPGrow * len(rows))(*rows), len(rows), heads,
+                              _lib.stream_handle(dev))
+            _lib.check(st, "tp_grow_rows")
 
     def buffer(self, storage, name: str):
         """``storage``'s buffer as it will be after ``commit``."""
