@@ -41,6 +41,19 @@ def _regrow(t: Optional[torch.Tensor], new_cap: int) -> Optional[torch.Tensor]:
     return out
 
 
+# The storages' buffers; their forms are the encoder's at the first reservation, then their own.
+_KEY_BUFFERS = dict.fromkeys(("radii", "angle_codes_l1", "angle_codes_deep", "radii_scales"))
+_VALUE_BUFFERS = dict.fromkeys(("codes", "scales"))
+
+
+def _form(t: Optional[torch.Tensor]):
+    """((B, H), page shape, dtype) of a page buffer, as an encoder's ``page_shapes`` gives them."""
+    if t is None:
+        return None
+    shape = tuple(t.shape)
+    return shape[:2], shape[3:], t.dtype
+
+
 class Growth:
     """Larger buffers of one or two storages, not yet theirs: ``commit`` hands
     them over, so a caller whose append is rejected afterwards leaves the
@@ -64,38 +77,37 @@ class Growth:
         """Room for ``needed`` pages in ``storage``; ``shapes`` maps its buffer
         attributes to ((B, H), page shape, dtype), or None for a buffer that the
         layout does not have: the forms of a first reservation.  A buffer that is
-        there grows in its own form, on its own device (its pages may be ``append``'s,
-        of another length).  The counters move as the reference's sequence of
-        doublings from the initial capacity moves them (storage.py:34-73)."""
-        first = all(getattr(storage, name) is None for name in shapes)
+        there grows in its own form, on its own device, whatever ``shapes`` says
+        (its pages may be ``append``'s, of another length).  The counters move as
+        the reference's sequence of doublings from the initial capacity moves them
+        (storage.py:34-73)."""
+        held = getattr(storage, next(iter(shapes)))
+        first = held is None
         cap = initial_capacity if first else storage.capacity
         caps, new_cap = _doublings(cap, needed)
         if not caps and not first:
             return
+        if not first:
+            device, shapes = held.device, {name: _form(getattr(storage, name)) for name in shapes}
+        make = torch.empty if device.type == "cuda" else torch.zeros
         made, per_slot = {}, 0
         for name, spec in shapes.items():
-            old = getattr(storage, name)
-            if not first:
-                spec = None if old is None else (tuple(old.shape[:2]), tuple(old.shape[3:]), old.dtype)
             if spec is None:
                 made[name] = None
                 continue
-            if not first:
-                device = old.device
-            make = torch.empty if device.type == "cuda" else torch.zeros
             (B, H), page, dtype = spec
             page_bytes = prod(page) * dtype.itemsize
             new = made[name] = make((B, H, new_cap) + page, dtype=dtype, device=device)
             per_slot += B * H * page_bytes
             if page_bytes:
-                self._rows.append((old, new, storage.block_count, page_bytes, B * H))
+                self._rows.append((getattr(storage, name), new, storage.block_count, page_bytes, B * H))
         self._sets.append((storage, made, new_cap, len(caps), per_slot * sum(caps)))
 
     def fill(self) -> None:
         """Copies the kept pages and clears the spare ones."""
-        held, launches = [], {}  # (device, (batch, head) rows): buffers; one launch for a cache's two storages
-        for old, new, keep, page, heads in self._rows:
-            if new.device.type != "cuda":
+        held, launches, dev, heads = [], [], None, 0  # one launch for a cache's two storages
+        for old, new, keep, page, rows in self._rows:
+            if not new.is_cuda:
                 if keep:
                     new[:, :, :keep] = old[:, :, :keep]
                 continue
@@ -105,20 +117,22 @@ class Growth:
                 if keep and not old.is_contiguous():
                     old = old.contiguous()
                 held.append(old)
-                launches.setdefault((new.device, heads), []).append(
-                    _lib.TPGrow(old.data_ptr() if keep else None, new.data_ptr(),
-                                old.shape[2] * page if keep else 0, cap * page, keep * page, used * page))
-        for (dev, heads), rows in launches.items():
-            st = _lib.call_on(dev, _lib.lib().tp_grow_rows, (_lib.TPGrow * len(rows))(*rows), len(rows), heads,
+                if rows != heads or new.device != dev:
+                    dev, heads, bufs = new.device, rows, []
+                    launches.append((dev, heads, bufs))
+                bufs.append(_lib.TPGrow(old.data_ptr() if keep else None, new.data_ptr(),
+                                        old.shape[2] * page if keep else 0, cap * page, keep * page, used * page))
+        for dev, heads, bufs in launches:
+            st = _lib.call_on(dev, _lib.lib().tp_grow_rows, (_lib.TPGrow * len(bufs))(*bufs), len(bufs), heads,
                               _lib.stream_handle(dev))
             _lib.check(st, "tp_grow_rows")
 
-    def buffer(self, storage, name: str):
-        """``storage``'s buffer as it will be after ``commit``."""
+    def buffers(self, storage) -> dict:
+        """``storage``'s buffers by name as they will be after ``commit``."""
         for s, made, _, _, _ in self._sets:
             if s is storage:
-                return made[name]
-        return getattr(storage, name)
+                return made
+        return vars(storage)
 
     def commit(self) -> None:
         for storage, made, cap, reallocs, grown in self._sets:
@@ -146,7 +160,8 @@ class PolarKBlockStorage:
 
     def plan(self, growth: Growth, needed: int, encoder, B: int, H: int, device, initial_capacity: int = 4) -> None:
         """Adds what ``needed`` pages take to ``growth`` (storage.py:34-73 growth rule)."""
-        growth.add(self, encoder.page_shapes(B, H), needed, initial_capacity, device)
+        growth.add(self, encoder.page_shapes(B, H) if self.radii is None else _KEY_BUFFERS, needed, initial_capacity,
+                   device)
 
     def reserve(self, needed: int, encoder, B: int, H: int, device, initial_capacity: int = 4) -> None:
         """Make room for ``needed`` pages."""
@@ -216,8 +231,8 @@ class QuantVBlockStorage:
 
     def plan(self, growth: Growth, needed: int, B: int, H: int, device, initial_capacity: int = 4) -> None:
         # Stored 6-D [B, H, cap, 1, 64, 128] like storage.py:121-131.
-        growth.add(self, {"codes": ((B, H), (1, 64, 128), torch.int8), "scales": ((B, H), (1, 64, 4), torch.float16)},
-                   needed, initial_capacity, device)
+        growth.add(self, {"codes": ((B, H), (1, 64, 128), torch.int8), "scales": ((B, H), (1, 64, 4), torch.float16)}
+                   if self.codes is None else _VALUE_BUFFERS, needed, initial_capacity, device)
 
     def reserve(self, needed: int, B: int, H: int, device, initial_capacity: int = 4) -> None:
         growth = Growth()
@@ -258,15 +273,16 @@ def pages_of(k_storage: PolarKBlockStorage, v_storage: QuantVBlockStorage, growt
     """``tp_pages`` over the whole capacity of a pair of storages (as they will
     be after ``growth`` is committed, if given)."""
     if growth is None:
-        get, capacity = getattr, k_storage.capacity
+        k, v, capacity = vars(k_storage), vars(v_storage), k_storage.capacity
     else:
-        get, capacity = growth.buffer, growth.buffer(k_storage, "radii").shape[2]
+        k, v = growth.buffers(k_storage), growth.buffers(v_storage)
+        capacity = k["radii"].shape[2]
     return _lib.TPPages(
-        _lib.ptr(get(k_storage, "radii")),
-        _lib.ptr(get(k_storage, "radii_scales")),
-        _lib.ptr(get(k_storage, "angle_codes_l1")),
-        _lib.ptr(get(k_storage, "angle_codes_deep")),
-        _lib.ptr(get(v_storage, "codes")),
-        _lib.ptr(get(v_storage, "scales")),
+        _lib.ptr(k["radii"]),
+        _lib.ptr(k["radii_scales"]),
+        _lib.ptr(k["angle_codes_l1"]),
+        _lib.ptr(k["angle_codes_deep"]),
+        _lib.ptr(v["codes"]),
+        _lib.ptr(v["scales"]),
         int(capacity),
     )
