@@ -60,16 +60,15 @@ int32_t wait_verdict(const uint32_t* flag, uint32_t epoch, hipStream_t s, bool r
                      int64_t n_done) {
   const volatile uint32_t* vf = flag;
   uint32_t verdict = 0;
-  int64_t seen = -1;  // what has come: the verdict, then the reports
-  for (int spin = 0; reports && spin < (1 << 22) && seen < n_done; ++spin) {
-    if (seen < 0) {
-      verdict = *vf;
-      if (verdict == epoch || verdict == epoch + 1u) seen = 0;
-    } else {
-      while (seen < n_done && vf[kReportStride * (seen + 1)] == epoch) ++seen;
-    }
+  bool done = false;
+  const int64_t spins = (1 << 22) / (1 + n_done);
+  for (int64_t spin = 0; reports && spin < spins && !done; ++spin) {
+    verdict = *vf;
+    uint32_t missing = 0;  // every line is read each time, so that their cache misses overlap
+    for (int64_t i = 1; i <= n_done; ++i) missing |= vf[kReportStride * i] ^ epoch;
+    done = (verdict == epoch || verdict == epoch + 1u) && missing == 0;
   }
-  if (seen < n_done) {
+  if (!done) {
     if (hipStreamSynchronize(s) != hipSuccess) {
       set_error("%s: synchronising the stream failed", what);
       return TP_ERR_HIP;
