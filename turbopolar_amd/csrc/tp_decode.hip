@@ -19,8 +19,6 @@ struct DecodeArgs {
   const uint16_t* v_scales;
   int64_t capacity;
   int64_t page_begin;
-  int32_t n_pages;
-  int32_t int8_radii;
   int32_t l1_bits;
   int32_t deep_bits;
   int32_t split_half;
@@ -283,8 +281,6 @@ static int32_t decode_pages_impl(const tp_page_layout* layout, const tp_pages* p
   a.v_scales = static_cast<const uint16_t*>(pages->v_scales);
   a.capacity = pages->capacity;
   a.page_begin = page_begin;
-  a.n_pages = n_pages;
-  a.int8_radii = layout->int8_radii;
   a.l1_bits = layout->l1_bits;
   a.deep_bits = layout->deep_bits;
   a.split_half = layout->split_dim / 2;

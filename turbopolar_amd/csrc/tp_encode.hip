@@ -77,8 +77,9 @@ __device__ __forceinline__ bool any_nonfinite(uint4 w) {
   return bad;
 }
 
-// The tokens of row blockIdx.y outside the launch's whole pages, by one
-// 256-thread workgroup: at most 126 rows, one 16-byte chunk of k and of v at a time.
+// The tokens of row blockIdx.y outside the launch's whole pages, by one workgroup of
+// the launch (256 or 1024 threads): at most 126 rows, a 16-byte chunk of k and of v
+// at a time.
 template <bool kF32>
 __device__ __forceinline__ void edge_tokens(const EncodeArgs& a) {
   constexpr int kChunks = kHeadDim * (kF32 ? 4 : 2) / 16;  // per token row

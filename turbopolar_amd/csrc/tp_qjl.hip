@@ -61,9 +61,10 @@ __global__ __launch_bounds__(256) void qjl_sketch_kernel(const void* e, int64_t 
 // scalar kernel's FMAs): a wave takes 16 rows x 16 projections, with its 32 W
 // values per lane in registers for every row tile it walks, so nothing goes
 // through LDS.  The k order is free as long as both operands follow it: lane
-// group l4 holds k = 32 l4 .. +31, 128 contiguous bytes of its row.  The accumulator of lane (l16, l4) holds rows 4 l4 + i, projection
-// l16, so one ballot per i yields 16 sketch bits of four rows.
-// Measured at 65,536 rows and 64 bits: 22.8 us (the scalar kernel below: 123).
+// group l4 holds k = 32 l4 .. +31, 128 contiguous bytes of its row.  The accumulator
+// of lane (l16, l4) holds rows 4 l4 + i, projection l16, so one ballot per i yields
+// 16 sketch bits of four rows.  Measured at 65,536 rows and 64 bits: 22.8 us (the
+// scalar kernel above: 123).
 constexpr int kSketchDim = 128;
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
@@ -331,8 +332,9 @@ int32_t tp_qjl_sketch(const void* e, int32_t in_dtype, int64_t rows, int32_t dim
   if (dim == kSketchDim && !((uintptr_t)e & 15u) && !((uintptr_t)packed & 1u)) {
     const unsigned cols = (unsigned)((proj_dim + 63) / 64);
     if (in_dtype) {
-      // At most three workgroups a CU, which then walk several row tiles on one load of W (measured
-      // at 65,536 rows: 256 / 512 / 768 / 1024 / 2048 workgroups 27.7 / 22.2 / 22.8 / 24.5 / 29.5 us).
+      // At most 768 workgroups, three a CU, per 64 projections, which then walk several row tiles on
+      // one load of W (65,536 rows, 64 bits: 256 / 512 / 768 / 1024 / 2048 workgroups 27.7 / 22.2 /
+      // 22.8 / 24.5 / 29.5 us).
       const unsigned x = (unsigned)std::min<int64_t>((rows + 15) / 16, 768);
       hipLaunchKernelGGL(qjl_sketch_f32_kernel, dim3(x, cols), dim3(256), 0, s, static_cast<const float*>(e), rows, w,
                          proj_dim, packed, norms);
@@ -341,6 +343,9 @@ int32_t tp_qjl_sketch(const void* e, int32_t in_dtype, int64_t rows, int32_t dim
       // Whole rows / column tiles, us: 32 rows 5.6 / 4.2, 8,192 6.5 / 4.7, 16,384 6.6 / 6.5, 32,768 6.7 / 9.2.
       const int by_column = rows <= 8192;
       const int per = (by_column ? 1 : 4) * kSketchRows;  // rows of a workgroup at a time
+      // At most 768 workgroups per 64 projections here too, above 98,304 rows (64 bits, 256 / 512 /
+      // 768 / 1024 / 2048 workgroups, us: 131,072 rows 16.2 / 12.7 / 12.6 / 14.0 / 14.0, 262,144 rows
+      // 28.5 / 21.7 / 20.3 / 22.4 / 24.9, 1,048,576 rows 101 / 77 / 69 / 73 / 74).
       const unsigned x = (unsigned)std::min<int64_t>((rows + per - 1) / per, 768);
       hipLaunchKernelGGL(qjl_sketch_f16_kernel, dim3(x, cols), dim3(256), 0, s, static_cast<const uint16_t*>(e), rows, w,
                          proj_dim, packed, norms, by_column);

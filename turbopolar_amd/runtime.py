@@ -10,10 +10,12 @@ rfsn_v11/generation/turbo_polar_cache.py:18-395.  Differences of mechanism
   them, like the reference's immutable arrays); ``get_fused_attention_inputs``
   returns views of it, valid until the next append, so a decode step copies
   nothing;
-* an append of whole pages is one ``tp_append_pages`` launch, which checks,
-  encodes and copies to the tail in one read of the input and writes straight
-  into the storage slots (no per-page Python loop, no intermediate block
-  copies);
+* an append of whole pages to an empty tail is one ``tp_append_pages`` launch,
+  which checks, encodes and copies to the tail in one read of the input and
+  writes straight into the storage slots (no per-page Python loop, no
+  intermediate block copies); a tail that holds tokens is completed by that
+  launch, then encoded by a second one, and a third copies the tokens that
+  start the next tail;
 * a bulk append reserves capacity once (the doubling telemetry is unchanged).
 """
 
@@ -312,7 +314,8 @@ class TurboPolarKVCacheRuntime:
         encodes the whole pages and copies the tokens bound for the tail, with
         one synchronisation.  Pages are encoded into slots past the stored ones
         (of larger buffers, if the store has to grow), which only become part of
-        the cache once the verdict is in."""
+        the cache once the verdict is in.  Of a tail that held tokens, the completed
+        page is encoded and the next tail's tokens copied by two launches after it."""
         B, H, T, _ = k_new.shape
         ks = self.k_storage
         rest, flush = (T - n_head) % PAGE, 1 if self._tail_len else 0
