@@ -168,14 +168,15 @@ int32_t tp_decode_attention(const void* q, int64_t batch, int32_t hq, int32_t hk
  * its rows at row tail_len.  Attends every stored token and the new one.  check 2:
  * the call returns once the launch has reported whether every value of new_k and
  * new_v is finite, TP_ERR_NONFINITE if not (`out` and the tail's row tail_len
- * then hold no result; the tokens before it are as they were), and that it has read
- * both for the last time, so the caller may overwrite or free them on any stream;
- * q is read until the launch is through.  flag holds 16 * (1 + batch * hkv *
- * ceil(hq / hkv / 16)) words then: the first is the verdict, and the launch sets
- * words 16, 32, ... to epoch.  check 3 (deferred) returns after the launch, which reads new_k and new_v
- * until it is through and writes epoch + 1 to the first word of flag on a
- * non-finite value.  flag and epoch otherwise as for tp_append_stage with check 2
- * and 3, everything else as for tp_decode_attention (at most 65534 splits).
+ * then hold no result; the tokens before it are as they were); check 3 (deferred)
+ * returns after the launch, which writes epoch + 1 to flag on a non-finite value.
+ * Either way the launch reads new_k and new_v, like q, until it is through.
+ * check 4: as check 2, and the call returns only once the launch has read new_k and
+ * new_v for the last time, so that the caller may overwrite or free them on any
+ * stream; flag then holds 16 * (1 + batch * hkv * ceil(hq / hkv / 16)) words, the
+ * first of which is the verdict, and the launch sets words 16, 32, ... to epoch.
+ * flag and epoch otherwise as for tp_append_stage with check 2 and 3, everything
+ * else as for tp_decode_attention (at most 65534 splits).
  */
 int32_t tp_decode_step(const void* q, int64_t batch, int32_t hq, int32_t hkv,
                        const tp_page_layout* layout, const tp_pages* pages, int32_t n_pages,

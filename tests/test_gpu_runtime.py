@@ -556,6 +556,25 @@ def test_step_has_read_keys_and_values_when_it_returns(device, hq, hkv, start):
     assert torch.equal(rt.runtime.partial_k, k[:, :, tail:]) and torch.equal(rt.runtime.partial_v, v[:, :, tail:])
 
 
+@pytest.mark.parametrize("check,words", [(2, 1), (3, 1), (4, 16 * 9)])
+def test_step_writes_the_flag_words_of_its_check(device, check, words):
+    """A step with check 2 or 3 needs one word of flag and writes no other; with
+    check 4 it reports each unit on a line of its own."""
+    print(f"[step-flag] check={check}", flush=True)
+    g = torch.Generator(device=device).manual_seed(1)
+    rand = lambda *s: torch.randn(s, generator=g, device=device).half()  # noqa: E731
+    q, k, v, tk, tv = rand(1, 32, 128), rand(1, 8, 1, 128), rand(1, 8, 1, 128), rand(1, 8, 64, 128), rand(1, 8, 64, 128)
+    assert kernels.step_flag_words(1, 32, 8) == 16 * 9
+    flag = torch.full((16 * 9,), 7, dtype=torch.int32, pin_memory=True)
+    out = kernels.decode_step(q, kernels._DEFAULT_LAYOUT, None, 0, k, v, tk, tv, 20, 0.088, check, flag, 10)
+    torch.cuda.synchronize()
+    lines, rest = flag.numpy()[::16], flag.numpy().reshape(9, 16)[:, 1:]
+    assert lines[0] == (7 if check == 3 else 10) and (lines[1:] == (10 if words > 1 else 7)).all() and (rest == 7).all()
+    want = kernels.decode_attention_store(q, kernels._DEFAULT_LAYOUT, None, 0, 8, tk.narrow(2, 0, 21),
+                                          tv.narrow(2, 0, 21), 21, 0.088)
+    assert torch.equal(out, want) and torch.equal(tk[:, :, 20:21], k) and torch.equal(tv[:, :, 20:21], v)
+
+
 @pytest.mark.parametrize("start", [10, 63])
 def test_decode_scale_changed_in_place(device, start):
     """A step takes the scale's value at the call, of a tensor changed in place too

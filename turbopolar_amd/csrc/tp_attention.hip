@@ -162,7 +162,7 @@ struct AttnArgs {
   const uint16_t* new_k;
   const uint16_t* new_v;
   int32_t new_rows;  // batch * hkv
-  int32_t check;     // as tp_append_stage: 2 reports the verdict (and take_new_row), 3 only a non-finite value
+  int32_t check;     // 2 reports the verdict, 3 only a non-finite value, 4 the verdict and the reads (take_new_row)
   uint32_t* flag;
   uint32_t epoch;
 };
@@ -970,9 +970,11 @@ struct TailRegs {
   u32x4 v[16];
 };
 
+constexpr int kCheckReads = 4;
+
 // STEP: the last row is not in the tail yet (stage_new_rows copies it there in
-// this launch); it comes from new_row (take_new_row) or, with nobody waiting, from
-// new_k and new_v, and the tail's range ends before it.
+// this launch); it comes from new_row (take_new_row) or, with nobody waiting for the
+// reads, from new_k and new_v, and the tail's range ends before it.
 template <bool HR, bool STEP>
 __device__ __forceinline__ void load_tail(const AttnArgs& a, int64_t bkv, int l16, int l4, const u32x4* new_row,
                                           TailRegs& r) {
@@ -1000,7 +1002,7 @@ __device__ __forceinline__ void load_tail(const AttnArgs& a, int64_t bkv, int l1
     const int row = a.tail_len - 1;
     const int c0 = HR ? 8 * (l16 & 1) + 2 * l4 : 4 * l4;
     u32x4 w[HR ? 2 : 4], wv;
-    if (a.check == 2) {
+    if (a.check == kCheckReads) {
 #pragma unroll
       for (int kk = 0; kk < (HR ? 2 : 4); ++kk) w[kk] = new_row[c0 + kk];
       wv = new_row[16 + l16];
@@ -1027,8 +1029,8 @@ __device__ __forceinline__ void load_tail(const AttnArgs& a, int64_t bkv, int l1
 // workgroups attend.  A launch of its own in front held the step up twice: the
 // attention launch waited for the verdict on the host, the next step's staging
 // for the attention on the GPU.  The other readers of the rows, the workgroups that
-// attend the tail, report for themselves (take_new_row), so that the host returns once
-// nothing reads new_k and new_v any more.
+// attend the tail, report for themselves where the host waits until nothing reads
+// new_k and new_v any more (take_new_row).
 __device__ __forceinline__ void stage_new_rows(const AttnArgs& a) {
   if (blockIdx.x != 0 || blockIdx.y != 0) return;
   constexpr int kChunks = kHeadDim * 2 / 16;
@@ -1044,7 +1046,7 @@ __device__ __forceinline__ void stage_new_rows(const AttnArgs& a) {
     reinterpret_cast<uint4*>(const_cast<uint16_t*>(a.tail_k))[dst] = k;
     reinterpret_cast<uint4*>(const_cast<uint16_t*>(a.tail_v))[dst] = v;
   }
-  if (a.check == 2) {
+  if (a.check != 3) {
     const bool any_bad = __syncthreads_or(bad);
     if (threadIdx.x == 0)
       __hip_atomic_store(a.flag, any_bad ? a.epoch + 1u : a.epoch, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
@@ -1053,7 +1055,7 @@ __device__ __forceinline__ void stage_new_rows(const AttnArgs& a) {
   }
 }
 
-// A step whose caller waits (check 2): the wave that will attend the tail takes its
+// A step whose caller waits for its reads (check 4): the wave that will attend the tail takes its
 // unit's new rows (batch row, kv head, head block) into LDS, K's 16 chunks and then
 // V's, and reports that in the unit's own line after the flag's.  It does so before its
 // first page's loads: behind them the report came 4 us later while a 32k cache
@@ -1875,7 +1877,7 @@ __global__ __launch_bounds__(WAVES * 64) void decode_attention_kernel(AttnArgs a
 
   __shared__ u32x4 new_row[STEP ? 32 : 1];
   if constexpr (STEP) {
-    if (a.check == 2 && split == a.n_splits - 1 && wave == max(p_end - p_begin, 0) % WAVES)
+    if (a.check == kCheckReads && split == a.n_splits - 1 && wave == max(p_end - p_begin, 0) % WAVES)
       take_new_row(a, bkv, bkv * a.head_blocks + hb, lane, new_row);
   }
 
@@ -2626,8 +2628,8 @@ int32_t tp_decode_step(const void* q, int64_t batch, int32_t hq, int32_t hkv, co
               "k=%p v=%p and %d tail tokens", new_k, new_v, tail_len);
     return TP_ERR_INVALID;
   }
-  if ((check != 2 && check != 3) || !flag || (epoch & 1u)) {
-    set_error("check must be 2 or 3 (deferred) with a pinned host flag and an even epoch");
+  if (check < 2 || check > kCheckReads || !flag || (epoch & 1u)) {
+    set_error("check must be 2, 3 (deferred) or 4 (2 and the reads) with a pinned host flag and an even epoch");
     return TP_ERR_INVALID;
   }
   AttnArgs step{};
@@ -2642,7 +2644,7 @@ int32_t tp_decode_step(const void* q, int64_t batch, int32_t hq, int32_t hkv, co
                                            workspace_bytes, out, stream, false, nullptr, 0, &step);
   if (st != TP_OK || check == 3) return st;
   return wait_verdict(flag, epoch, static_cast<hipStream_t>(stream), true, "tp_decode_step",
-                      batch * hkv * head_blocks_of(hq, hkv));
+                      check == kCheckReads ? batch * hkv * head_blocks_of(hq, hkv) : 0);
 }
 
 int32_t tp_decode_attention_qjl(const void* q, int64_t batch, int32_t hq, int32_t hkv,

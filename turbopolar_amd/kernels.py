@@ -479,7 +479,7 @@ def decode_attention_store(q: torch.Tensor, layout, pages: TPPages, n_pages: int
 
 @lru_cache(maxsize=1024)
 def step_flag_words(B: int, Hq: int, Hkv: int) -> int:
-    """Words of tp_decode_step's flag with check 2: a 64-byte line for the verdict and
+    """Words of tp_decode_step's flag with check 4: a 64-byte line for the verdict and
     one per unit (batch row, kv head, head block of 16)."""
     return 16 * (1 + B * Hkv * -(-(Hq // Hkv) // 16))
 
@@ -491,8 +491,8 @@ def decode_step(q: torch.Tensor, layout, pages: Optional[TPPages], n_pages: int,
     (contiguous fp16) joins the ``tail_len`` tokens of the tail buffers
     ``[B, H_kv, 64, 128]`` and ``q`` ``[B, H_q, 128]`` attends all of it in one
     launch.  Raises the append's ValueError when the launch reports a non-finite
-    value (``check_mode`` 2; the caller's ``flag`` holds ``step_flag_words`` words
-    then, and ``new_k`` and ``new_v`` are no longer read when this returns)."""
+    value (``check_mode`` 2 and 4; with 4 ``new_k`` and ``new_v`` are no longer read
+    when this returns, and ``flag`` holds ``step_flag_words`` words)."""
     q16 = _q16(q)
     B, Hq, _ = q16.shape
     Hkv = new_k.shape[1]

@@ -301,7 +301,7 @@ class TurboPolarKVCacheRuntime:
         # Even epochs, as for the staging kernel.
         self._epoch = ((self._epoch + 2) & 0xFFFFFFFE) or 2
         out = decode_step(q, layout, pages, self.k_storage.block_count, k_new, v_new, self._tail_k, self._tail_v,
-                          self._tail_len, scale, 3 if defer_check else 2, self._flag, self._epoch)
+                          self._tail_len, scale, 3 if defer_check else 4, self._flag, self._epoch)
         if defer_check:
             self._pending.append((self._epoch, self._state()))
         self.actual_seq_len += 1
