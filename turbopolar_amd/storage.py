@@ -46,14 +46,6 @@ _KEY_BUFFERS = dict.fromkeys(("radii", "angle_codes_l1", "angle_codes_deep", "ra
 _VALUE_BUFFERS = dict.fromkeys(("codes", "scales"))
 
 
-def _form(t: Optional[torch.Tensor]):
-    """((B, H), page shape, dtype) of a page buffer, as an encoder's ``page_shapes`` gives them."""
-    if t is None:
-        return None
-    shape = tuple(t.shape)
-    return shape[:2], shape[3:], t.dtype
-
-
 class Growth:
     """Larger buffers of one or two storages, not yet theirs: ``commit`` hands
     them over, so a caller whose append is rejected afterwards leaves the
@@ -71,7 +63,8 @@ class Growth:
     def __init__(self, fresh: int = 0):
         self.fresh = fresh
         self._sets: list = []  # (storage, {attribute: new buffer}, capacity, reallocations, bytes grown)
-        self._rows: list = []  # (old buffer or None, new buffer, pages kept, page bytes, (batch, head) rows)
+        # (old buffer or None, its capacity, new buffer, its capacity, pages kept, page bytes, (batch, head) rows)
+        self._rows: list = []
 
     def add(self, storage, shapes: dict, needed: int, initial_capacity: int, device) -> None:
         """Room for ``needed`` pages in ``storage``; ``shapes`` maps its buffer
@@ -88,30 +81,35 @@ class Growth:
         if not caps and not first:
             return
         if not first:
-            device, shapes = held.device, {name: _form(getattr(storage, name)) for name in shapes}
+            device = held.device
         make = torch.empty if device.type == "cuda" else torch.zeros
         made, per_slot = {}, 0
         for name, spec in shapes.items():
-            if spec is None:
+            old, old_cap = None if first else getattr(storage, name), 0
+            if old is not None:
+                shape, dtype = list(old.shape), old.dtype
+                old_cap, shape[2] = shape[2], new_cap
+            elif first and spec is not None:
+                (B, H), page, dtype = spec
+                shape = [B, H, new_cap, *page]
+            else:
                 made[name] = None
                 continue
-            (B, H), page, dtype = spec
-            page_bytes = prod(page) * dtype.itemsize
-            new = made[name] = make((B, H, new_cap) + page, dtype=dtype, device=device)
-            per_slot += B * H * page_bytes
+            page_bytes, rows = prod(shape[3:]) * dtype.itemsize, shape[0] * shape[1]
+            new = made[name] = make(shape, dtype=dtype, device=device)
+            per_slot += rows * page_bytes
             if page_bytes:
-                self._rows.append((getattr(storage, name), new, storage.block_count, page_bytes, B * H))
+                self._rows.append((old, old_cap, new, new_cap, storage.block_count, page_bytes, rows))
         self._sets.append((storage, made, new_cap, len(caps), per_slot * sum(caps)))
 
     def fill(self) -> None:
         """Copies the kept pages and clears the spare ones."""
         held, launches, dev, heads = [], [], None, 0  # one launch for a cache's two storages
-        for old, new, keep, page, rows in self._rows:
+        for old, old_cap, new, cap, keep, page, rows in self._rows:
             if not new.is_cuda:
                 if keep:
                     new[:, :, :keep] = old[:, :, :keep]
                 continue
-            cap = new.shape[2]
             used = min(cap, keep + self.fresh)
             if keep or used < cap:
                 if keep and not old.is_contiguous():
@@ -121,7 +119,7 @@ class Growth:
                     dev, heads, bufs = new.device, rows, []
                     launches.append((dev, heads, bufs))
                 bufs.append(_lib.TPGrow(old.data_ptr() if keep else None, new.data_ptr(),
-                                        old.shape[2] * page if keep else 0, cap * page, keep * page, used * page))
+                                        old_cap * page if keep else 0, cap * page, keep * page, used * page))
         for dev, heads, bufs in launches:
             st = _lib.call_on(dev, _lib.lib().tp_grow_rows, (_lib.TPGrow * len(bufs))(*bufs), len(bufs), heads,
                               _lib.stream_handle(dev))
